@@ -42,6 +42,42 @@ int from_device_v(void *src, bool fp64, std::vector<double> &dst)
   return 0;
 }
 
+// Cells per lane of a march along an extent of n cells, for `across` cells in
+// the plane it crosses.  A lane solves L + 1 faces for its L cells, one after
+// the other, and loads its window first (about half a face's time).  Long
+// marches waste the fewest solves; on a small box they leave most of the chip
+// idle.
+//
+// FP64: one wavefront's Riemann solve already fills a SIMD's issue slots about
+// as well as two, so a launch takes ceil(blocks / CUs) (L + 1.5).  The shortest
+// such time over L <= 16 is taken, L = 16 unless another is 5% shorter (a box
+// that streams from HBM gains nothing from the model).  y and z march, us at
+// L = 16 -> at the rule's L: 64^3 54 + 57 -> 23 + 25 (L = 4), RMHD HLLD
+// 50x44x38 276 + 285 -> 59 + 59 (L = 2), 16^3 52 + 53 -> 11 + 12 (L = 1);
+// 128^3 100 + 106 against 108 + 113 at 8 and 117 + 127 at 4.
+//
+// FP32: four wavefronts per SIMD hide the load latency, so L is the largest of
+// 8, 4, 2, 1 that leaves 8192 wavefronts (512 for the last halving).  z march
+// and x+y kernel, us at 16 -> rule: 64^3 48 + 64 -> 16 + 20 (L = 2), 128^3
+// 81 + 110 -> 82 + 90 (L = 4), 192^3 280 + 270 -> 250 + 263 (L = 8).
+int march_length(bool fp64, long long across, int n)
+{
+  if (!fp64) {
+    int l = 8;
+    while (l > 1 && across*((n + l - 1)/l)/64 < (l > 2 ? 8192 : 512)) l /= 2;
+    return l;
+  }
+  constexpr int kCUs = 256, kBlock = 256;
+  int best = 16;
+  double tbest = 0.0;
+  for (int l = 16; l >= 1; l--) {
+    const long long blocks = (across*((n + l - 1)/l) + kBlock - 1)/kBlock;
+    const double t = (double)((blocks + kCUs - 1)/kCUs)*(l + 1.5);
+    if (l == 16 || t < 0.95*tbest) { best = l; tbest = t; }
+  }
+  return best;
+}
+
 class Mhd3dEngine : public Engine {
 public:
   gpl_config cfg;
@@ -61,7 +97,9 @@ public:
   void *F = nullptr, *CM = nullptr, *FD = nullptr, *E = nullptr;
   void *dU = nullptr, *Cdt = nullptr;   // R: the within-stage sums (FP64 in the drop-in)
   bool fused = true;          // fused sweep kernels (nx <= 512) or the split path
-  int march = 16;             // cells per thread in the y/z marching sweeps
+  // cells per lane of the y march (rows per block of the x+y kernel) and of
+  // the z march (march_length)
+  int march[2] = {16, 16};
   // x and y sweeps in one row-marching kernel: the mixed form, where it saves
   // HBM traffic (its three LDS rows must fit in 64 KB); the FP64 sweeps are
   // VALU-bound and run faster as two kernels
@@ -135,9 +173,6 @@ public:
     // the fused x sweep holds one periodic x-row per block
     fused = g.nx <= 512 && getenv("GPL_SPLIT_KERNELS") == nullptr;
     if (padded && !fused) return GPL_EUNSUPPORTED;
-    // GPL_MARCH = 8/16/32: cells per thread in the y/z marching sweeps
-    if (const char *m = getenv("GPL_MARCH")) march = atoi(m);
-    if (march != 8 && march != 16 && march != 32) march = 16;
     emf_march = -32;
     if (const char *m = getenv("GPL_EMF_MARCH")) emf_march = atoi(m);
     {
@@ -147,7 +182,13 @@ public:
     fused_xy = !fp64;
     if (const char *m = getenv("GPL_FUSED_XY")) fused_xy = atoi(m) != 0;
     fused_xy = fused_xy && fused && !rmhd && 20*(size_t)g.nx*rs <= 65536;
-    nparts = fused ? mhd3d_march_blocks(g, march) : mhd3d_blocks(g);
+    march[0] = march_length(fp64, (long long)g.nx*g.nz, g.ny);
+    march[1] = march_length(fp64, (long long)g.nx*g.ny, g.nz);
+    // GPL_MARCH = 1, 2, 4 .. 64 fixes both
+    if (const char *m = getenv("GPL_MARCH")) {
+      const int l = atoi(m);
+      if (l >= 1 && l <= 64 && (l & (l - 1)) == 0) march[0] = march[1] = l;
+    }
     // the slab pipeline: GPL_PIPE_SLABS slabs (0 or 1: off); every slab but
     // the last starts and ends at a multiple of the y/z march and of the EMF
     // tiles' march length
@@ -157,10 +198,12 @@ public:
       // a slab's EMF launch covers only its planes: tiles marching 8 planes
       // keep four times as many workgroups in flight as the default 32
       if (want >= 3 && !getenv("GPL_EMF_MARCH")) emf_march = -8;
+      // a slab starts at a multiple of every march length
+      if (want >= 3 && !getenv("GPL_MARCH")) march[0] = march[1] = 16;
       const int lt = emf_march < 0 ? -emf_march : 0;
       if (want >= 3 && fp64 && fused && !fused_xy && lt > 0 &&
           c.ct_emf_average == GPL_UCT_HLL && want <= kMaxSlab) {
-        const int unit = march > lt ? march : lt;
+        const int unit = march[1] > lt ? march[1] : lt;
         int p = (g.nz + want - 1)/want;
         p = (p + unit - 1)/unit*unit;
         if (p > 0 && (g.nz + p - 1)/p >= 3) {
@@ -171,6 +214,7 @@ public:
       }
       if (!pipelined && want >= 3 && !getenv("GPL_EMF_MARCH")) emf_march = -32;
     }
+    nparts = fused ? mhd3d_march_blocks(g, march[1]) : mhd3d_blocks(g);
     if (pipelined) {
       // C_dt partial slots: each slab's z march writes its own range
       slab_part0.resize(nslab);
@@ -178,7 +222,7 @@ public:
       for (int s = 0; s < nslab; s++) {
         slab_part0[s] = total;
         const int nk = (s + 1)*slab_planes < g.nz ? slab_planes : g.nz - s*slab_planes;
-        const long long nt = (long long)g.nx*g.ny*((nk + march - 1)/march);
+        const long long nt = (long long)g.nx*g.ny*((nk + march[1] - 1)/march[1]);
         total += (int)((nt + 255)/256);
       }
       nparts = total;
@@ -357,6 +401,7 @@ public:
     b.F = (R *)F; b.CM = (R *)CM; b.FD = (R *)FD; b.E = (R *)E;
     b.dU = (R *)dU; b.Cdt = (R *)Cdt;
     b.cdt_part = cdt_part; b.err = env.err;
+    b.march[0] = march[0]; b.march[1] = march[1];
     b.emf_march = emf_march;
     b.phys = rmhd ? 1 : 0;
     b.net = net_on ? net : nullptr;
@@ -376,7 +421,7 @@ public:
       // solver 4: HLLD with the UCT_HLLD edge EMF (CT_Store_UCTHlld)
       const int solver = cfg.ct_emf_average == GPL_UCT_HLLD ? 4 : cfg.solver;
       mhd3d_launch<R>(k, b, g, env.ctl, w, first_stage, want_dt, cfg.limiter, solver,
-                      march, cfg.gamma, cfg.small_rho, cfg.small_prs, env.stream);
+                      cfg.gamma, cfg.small_rho, cfg.small_prs, env.stream);
       if (t) t->end(k);
     }
   }
@@ -406,7 +451,7 @@ public:
     };
     auto launch = [&](int k, const Mhd3dBufs<R> &bb, int s, hipStream_t st) {
       mhd3d_launch<R>(k, bb, slab_box(s), env.ctl, w, first_stage, want_dt, cfg.limiter, solver,
-                      march, cfg.gamma, cfg.small_rho, cfg.small_prs, st);
+                      cfg.gamma, cfg.small_rho, cfg.small_prs, st);
     };
     (void)hipEventRecord(ev_fork, sa);
     (void)hipStreamWaitEvent(s2, ev_fork, 0);

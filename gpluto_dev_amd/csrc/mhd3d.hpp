@@ -49,6 +49,7 @@ struct Mhd3dBufs {
   R *Cdt;          // [n]    C_dt accumulator within a stage (fused path)
   double *cdt_part;
   uint32_t *err;
+  int march[2];    // cells per lane of the y march (and rows per block of the x+y kernel), of the z march
   int emf_march;   // EMF kernel: 0 one edge per thread, n > 0 register z-march of n, -n LDS tiles marching n
   int phys;        // 0: ideal MHD, 1: relativistic MHD (FP64, fused kernels)
   const NetPack *net; // RMHD: learned con2prim guess (nullptr: the reference's A27 guess)
@@ -57,7 +58,7 @@ struct Mhd3dBufs {
 
 template <typename R>
 void mhd3d_launch(int which, const Mhd3dBufs<R> &b, const Box3 &g, const StepCtl *ctl, RKW w,
-                  int first_stage, int want_dt, int limiter, int solver, int march, double gamma,
+                  int first_stage, int want_dt, int limiter, int solver, double gamma,
                   double small_rho, double small_prs, hipStream_t s);
 
 // Ghost-zone fill of a padded box (non-periodic sides), side by side;

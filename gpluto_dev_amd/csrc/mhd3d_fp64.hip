@@ -4,6 +4,6 @@
 
 namespace gpl {
 template void mhd3d_launch<double>(int, const Mhd3dBufs<double> &, const Box3 &, const StepCtl *,
-                                   RKW, int, int, int, int, int, double, double, double,
+                                   RKW, int, int, int, int, double, double, double,
                                    hipStream_t);
 }

@@ -381,9 +381,9 @@ void k_sweepx_fused(Box3 g, const R *__restrict__ V, const double *__restrict__ 
 // instead of written, read and written again, and V is read once.  The
 // three LDS rows are disjoint, so a row needs three barriers.
 // ---------------------------------------------------------------------------
-template <typename R, int LIM, int SOLVER, int L, int PH>
+template <typename R, int LIM, int SOLVER, int PH>
 __global__ __launch_bounds__(512)
-void k_sweep_xy(Box3 g, const R *__restrict__ V, const double *__restrict__ Vs,
+void k_sweep_xy(Box3 g, int L, const R *__restrict__ V, const double *__restrict__ Vs,
                 R *__restrict__ FD, R *__restrict__ dU, R *__restrict__ Cdt,
                 const StepCtl *__restrict__ ctl, R gamma, int want_cdt,
                 uint32_t *__restrict__ err)
@@ -548,9 +548,9 @@ void k_sweep_xy(Box3 g, const R *__restrict__ V, const double *__restrict__ Vs,
 // (rk_step.cpp:366-374,509-518,670-708) and the per-block max of C_dt
 // (getMax, update_stage.cpp:446-458).
 // ---------------------------------------------------------------------------
-template <typename R, int D, int LIM, int SOLVER, int L, int PH>
+template <typename R, int D, int LIM, int SOLVER, int PH>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 && D == 1 ? 4 : (PH == 1 && SOLVER == 1 ? 2 : 1))))
-void k_sweep_march(Box3 g, const R *__restrict__ V, const double *__restrict__ Vs,
+void k_sweep_march(Box3 g, int L, const R *__restrict__ V, const double *__restrict__ Vs,
                    R *__restrict__ FD, R *__restrict__ dU, R *__restrict__ Cdt,
                    const double *Uin, double *U, const double *U0,
                    const StepCtl *__restrict__ ctl, RKW w, int first_stage, int want_cdt,
@@ -1185,7 +1185,7 @@ void k_finish(Box3 g, const R *__restrict__ E, const double *__restrict__ Vin,
 // Host-side launch helpers: one entry per kernel family, so that the host
 // orchestration can bracket each launch with timing events.
 // ---------------------------------------------------------------------------
-template <typename R, int LIM, int SOLVER, int L, int PH>
+template <typename R, int LIM, int SOLVER, int PH>
 static void launch_t(int which, const Mhd3dBufs<R> &b, const Box3 &g, const StepCtl *ctl, RKW w,
                      int first_stage, int want_dt, double gamma, double small_rho,
                      double small_prs, hipStream_t s)
@@ -1222,23 +1222,23 @@ static void launch_t(int which, const Mhd3dBufs<R> &b, const Box3 &g, const Step
     // wavefront has (the engine never selects it for RMHD)
     if constexpr (PH == 0) {
       const size_t shm = 20*(size_t)g.nx*sizeof(R);
-      const int nb = g.nz*((g.ny + L - 1)/L);
-      hipLaunchKernelGGL((k_sweep_xy<R, LIM, SOLVER, L, PH>), dim3(nb), dim3(g.nx), shm, s,
-                         g, b.V, b.Vin, b.FD, b.dU, b.Cdt, ctl, (R)gamma, want_dt, b.err);
+      const int L = b.march[0], nb = g.nz*((g.ny + L - 1)/L);
+      hipLaunchKernelGGL((k_sweep_xy<R, LIM, SOLVER, PH>), dim3(nb), dim3(g.nx), shm, s,
+                         g, L, b.V, b.Vin, b.FD, b.dU, b.Cdt, ctl, (R)gamma, want_dt, b.err);
     }
     break;
   }
   case K_SWEEPY_F: {
-    const int nt = g.nx*nk*((g.ny + L - 1)/L);
-    hipLaunchKernelGGL((k_sweep_march<R, 1, LIM, SOLVER, L, PH>), dim3((nt + T - 1)/T), dim3(T), 0, s,
-                       g, b.V, b.Vin, b.FD, b.dU, b.Cdt, b.Uin, b.U, b.U0, ctl, w, first_stage, want_dt,
+    const int L = b.march[0], nt = g.nx*nk*((g.ny + L - 1)/L);
+    hipLaunchKernelGGL((k_sweep_march<R, 1, LIM, SOLVER, PH>), dim3((nt + T - 1)/T), dim3(T), 0, s,
+                       g, L, b.V, b.Vin, b.FD, b.dU, b.Cdt, b.Uin, b.U, b.U0, ctl, w, first_stage, want_dt,
                        b.cdt_part, (R)gamma, b.err);
     break;
   }
   case K_SWEEPZ_F: {
-    const int nt = g.nx*g.ny*((nk + L - 1)/L);
-    hipLaunchKernelGGL((k_sweep_march<R, 2, LIM, SOLVER, L, PH>), dim3((nt + T - 1)/T), dim3(T), 0, s,
-                       g, b.V, b.Vin, b.FD, b.dU, b.Cdt, b.Uin, b.U, b.U0, ctl, w, first_stage, want_dt,
+    const int L = b.march[1], nt = g.nx*g.ny*((nk + L - 1)/L);
+    hipLaunchKernelGGL((k_sweep_march<R, 2, LIM, SOLVER, PH>), dim3((nt + T - 1)/T), dim3(T), 0, s,
+                       g, L, b.V, b.Vin, b.FD, b.dU, b.Cdt, b.Uin, b.U, b.U0, ctl, w, first_stage, want_dt,
                        b.cdt_part, (R)gamma, b.err);
     break;
   }
@@ -1291,49 +1291,39 @@ static void launch_t(int which, const Mhd3dBufs<R> &b, const Box3 &g, const Step
   }
 }
 
-template <typename R, int LIM, int SOLVER, int PH>
-static void launch_l(int which, const Mhd3dBufs<R> &b, const Box3 &g, const StepCtl *ctl, RKW w,
-                     int first_stage, int want_dt, int march, double gamma, double small_rho,
-                     double small_prs, hipStream_t s)
-{
-  if (march == 32) launch_t<R, LIM, SOLVER, 32, PH>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
-  else if (march == 8) launch_t<R, LIM, SOLVER, 8, PH>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
-  else launch_t<R, LIM, SOLVER, 16, PH>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
-}
-
 template <typename R>
 void mhd3d_launch(int which, const Mhd3dBufs<R> &b, const Box3 &g, const StepCtl *ctl, RKW w,
-                  int first_stage, int want_dt, int limiter, int solver, int march, double gamma,
+                  int first_stage, int want_dt, int limiter, int solver, double gamma,
                   double small_rho, double small_prs, hipStream_t s)
 {
   if constexpr (std::is_same<R, double>::value) {
     if (b.phys == 1) {            // RMHD: HLL, HLLC or HLLD, FP64 only
       if (solver == 3) {
-        if (limiter == MC_LIM) launch_l<R, MC_LIM, 3, 1>(which, b, g, ctl, w, first_stage, want_dt, march, gamma, small_rho, small_prs, s);
-        else                   launch_l<R, VANLEER_LIM, 3, 1>(which, b, g, ctl, w, first_stage, want_dt, march, gamma, small_rho, small_prs, s);
+        if (limiter == MC_LIM) launch_t<R, MC_LIM, 3, 1>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
+        else                   launch_t<R, VANLEER_LIM, 3, 1>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
       } else if (solver == 2) {
-        if (limiter == MC_LIM) launch_l<R, MC_LIM, 2, 1>(which, b, g, ctl, w, first_stage, want_dt, march, gamma, small_rho, small_prs, s);
-        else                   launch_l<R, VANLEER_LIM, 2, 1>(which, b, g, ctl, w, first_stage, want_dt, march, gamma, small_rho, small_prs, s);
+        if (limiter == MC_LIM) launch_t<R, MC_LIM, 2, 1>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
+        else                   launch_t<R, VANLEER_LIM, 2, 1>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
       } else {
-        if (limiter == MC_LIM) launch_l<R, MC_LIM, 1, 1>(which, b, g, ctl, w, first_stage, want_dt, march, gamma, small_rho, small_prs, s);
-        else                   launch_l<R, VANLEER_LIM, 1, 1>(which, b, g, ctl, w, first_stage, want_dt, march, gamma, small_rho, small_prs, s);
+        if (limiter == MC_LIM) launch_t<R, MC_LIM, 1, 1>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
+        else                   launch_t<R, VANLEER_LIM, 1, 1>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
       }
       return;
     }
   }
   if (solver == 4) {               // HLLD with the UCT_HLLD EMF
-    if (limiter == MC_LIM) launch_l<R, MC_LIM, 4, 0>(which, b, g, ctl, w, first_stage, want_dt, march, gamma, small_rho, small_prs, s);
-    else                   launch_l<R, VANLEER_LIM, 4, 0>(which, b, g, ctl, w, first_stage, want_dt, march, gamma, small_rho, small_prs, s);
+    if (limiter == MC_LIM) launch_t<R, MC_LIM, 4, 0>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
+    else                   launch_t<R, VANLEER_LIM, 4, 0>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
     return;
   }
   if (limiter == MC_LIM) {
-    if (solver == 3)      launch_l<R, MC_LIM, 3, 0>(which, b, g, ctl, w, first_stage, want_dt, march, gamma, small_rho, small_prs, s);
-    else if (solver == 2) launch_l<R, MC_LIM, 2, 0>(which, b, g, ctl, w, first_stage, want_dt, march, gamma, small_rho, small_prs, s);
-    else                  launch_l<R, MC_LIM, 1, 0>(which, b, g, ctl, w, first_stage, want_dt, march, gamma, small_rho, small_prs, s);
+    if (solver == 3)      launch_t<R, MC_LIM, 3, 0>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
+    else if (solver == 2) launch_t<R, MC_LIM, 2, 0>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
+    else                  launch_t<R, MC_LIM, 1, 0>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
   } else {
-    if (solver == 3)      launch_l<R, VANLEER_LIM, 3, 0>(which, b, g, ctl, w, first_stage, want_dt, march, gamma, small_rho, small_prs, s);
-    else if (solver == 2) launch_l<R, VANLEER_LIM, 2, 0>(which, b, g, ctl, w, first_stage, want_dt, march, gamma, small_rho, small_prs, s);
-    else                  launch_l<R, VANLEER_LIM, 1, 0>(which, b, g, ctl, w, first_stage, want_dt, march, gamma, small_rho, small_prs, s);
+    if (solver == 3)      launch_t<R, VANLEER_LIM, 3, 0>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
+    else if (solver == 2) launch_t<R, VANLEER_LIM, 2, 0>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
+    else                  launch_t<R, VANLEER_LIM, 1, 0>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
   }
 }
 

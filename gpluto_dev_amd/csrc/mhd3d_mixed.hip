@@ -5,6 +5,6 @@
 
 namespace gpl {
 template void mhd3d_launch<float>(int, const Mhd3dBufs<float> &, const Box3 &, const StepCtl *,
-                                  RKW, int, int, int, int, int, double, double, double,
+                                  RKW, int, int, int, int, double, double, double,
                                   hipStream_t);
 }

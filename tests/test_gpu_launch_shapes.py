@@ -1,0 +1,49 @@
+"""GPU: every launch shape that the size rules can pick gives the same bits as
+the oracle (FP64) or as one fixed shape (mixed precision), at sizes where a
+shape leaves remainders."""
+import numpy as np
+import pytest
+
+from gpluto_dev_amd import ic
+from gpluto_dev_amd.stage import Definitions, RuntimeSetup, StageUpdate
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(n, steps, first_dt, precision="fp64", ts="RK2", lim="MC_LIM", sides=()):
+    vc, vs = ic.mhd_turbulence(n, 17)
+    print(f"case n={n} {precision} {ts} {lim} {sides}", flush=True)
+    g = StageUpdate(Definitions(time_stepping=ts, limiter=lim), RuntimeSetup(n=n, sides=tuple(sides)),
+                    precision=precision)
+    g.upload(vc, vs)
+    res = g.run(steps, first_dt)
+    vc, vs, uc = g.download()
+    g.close()
+    return res, vc, vs, uc
+
+
+@pytest.mark.parametrize("march", ["", "1", "2", "4", "8", "32", "64"])
+def test_march_lengths_match_oracle(march, monkeypatch):
+    """y and z marches of every length, remainders included, in FP64."""
+    import oracle
+    if march:
+        monkeypatch.setenv("GPL_MARCH", march)
+    n = (19, 23, 37)
+    (err, t, dt), vc, vs, _ = _run(n, 4, 1e-3)
+    o = oracle.Oracle(phys="mhd", n=n, gamma=5 / 3)
+    o.set_state(*ic.mhd_turbulence(n, 17))
+    assert (err, t, dt) == o.run(4, 1e-3)
+    ovc, ovs, _ = o.get_state()
+    assert np.array_equal(vc, ovc) and np.array_equal(vs, ovs)
+
+
+@pytest.mark.parametrize("n", [(19, 23, 37), (64, 17, 33)])
+def test_march_lengths_mixed(n, monkeypatch):
+    """The mixed form's x+y kernel and z march: the same bits at every length."""
+    monkeypatch.setenv("GPL_MARCH", "16")
+    ref = _run(n, 4, 1e-3, precision="mixed")
+    for march in ("", "1", "2", "4", "8"):
+        monkeypatch.setenv("GPL_MARCH", march)
+        got = _run(n, 4, 1e-3, precision="mixed")
+        assert got[0] == ref[0]
+        assert all(np.array_equal(a, b) for a, b in zip(got[1:], ref[1:])), march
