@@ -78,6 +78,25 @@ int march_length(bool fp64, long long across, int n)
   return best;
 }
 
+// EMF kernel of a box (Mhd3dBufs::emf_march): 0 one edge per thread, -n LDS
+// tiles of 64 x 4 edges marching n planes.  A tile reads every HBM byte about
+// once, but its planes follow one another, so it needs enough tiles to fill the
+// chip; the per-edge kernel has no serial part and re-reads its stencils through
+// the caches, which hold a small box.
+// us a launch, edge / tiles of 4 / 8 / 32 planes:
+//   FP64 MC  64^3 13 / 16 / 25 / 82    96^3 43 / 46 / 51 / 90    128^3 108 / 86 / 91 / 104
+//            192^3 331 / 256 / 258 / 292                         256^3 -- / -- / 621 / 597
+//   FP64 VL  96^3 52 / 57 / 69 / 116   128^3 123 / 101 / 98 / 134   192^3 370 / 316 / 306 / 323
+//   FP32 MC  96^3 25 / 29 / 33 / 80    128^3 63 / 55 / 53 / 102     192^3 196 / 158 / 158 / 167
+// so the edge kernel up to a million cells, tiles of 8 planes above, and tiles
+// of 32 (fewest bytes) once they alone are 2048, eight per CU.
+int emf_choice(const Box3 &g)
+{
+  if (g.ncell <= 1000000) return 0;
+  const long long across = (long long)((g.nx + 63)/64)*((g.ny + 3)/4);
+  return across*((g.nz + 31)/32) >= 2048 ? -32 : -8;
+}
+
 class Mhd3dEngine : public Engine {
 public:
   gpl_config cfg;
@@ -105,7 +124,7 @@ public:
   // VALU-bound and run faster as two kernels
   bool fused_xy = false;
   // EMF kernel: n > 0 register z-march of n edges per thread, -n LDS-staged
-  // 64 x 4 tiles marching n planes (the default, 32), 0 one edge per thread
+  // 64 x 4 tiles marching n planes, 0 one edge per thread (emf_choice)
   int emf_march = -32;
   double *cdt_part = nullptr;
   int nparts = 0;
@@ -173,11 +192,12 @@ public:
     // the fused x sweep holds one periodic x-row per block
     fused = g.nx <= 512 && getenv("GPL_SPLIT_KERNELS") == nullptr;
     if (padded && !fused) return GPL_EUNSUPPORTED;
-    emf_march = -32;
-    if (const char *m = getenv("GPL_EMF_MARCH")) emf_march = atoi(m);
-    {
+    const int emf_auto = emf_choice(g);
+    emf_march = emf_auto;
+    if (const char *m = getenv("GPL_EMF_MARCH")) {
+      emf_march = atoi(m);
       const int l = emf_march < 0 ? -emf_march : emf_march;
-      if (emf_march != 0 && l != 4 && l != 8 && l != 16 && l != 32) emf_march = -32;
+      if (emf_march != 0 && l != 4 && l != 8 && l != 16 && l != 32) emf_march = emf_auto;
     }
     fused_xy = !fp64;
     if (const char *m = getenv("GPL_FUSED_XY")) fused_xy = atoi(m) != 0;
@@ -212,7 +232,7 @@ public:
           nslab = (g.nz + p - 1)/p;
         }
       }
-      if (!pipelined && want >= 3 && !getenv("GPL_EMF_MARCH")) emf_march = -32;
+      if (!pipelined && want >= 3 && !getenv("GPL_EMF_MARCH")) emf_march = emf_auto;
     }
     nparts = fused ? mhd3d_march_blocks(g, march[1]) : mhd3d_blocks(g);
     if (pipelined) {

@@ -736,9 +736,9 @@ __device__ __forceinline__ R uct_val(const R *q, const R *e, const R *fa, const 
 // from the plane being processed, shared through L1/L2 by the tile and its
 // neighbours on the same XCD.
 // ---------------------------------------------------------------------------
-template <typename R, int LIMV, int L>
+template <typename R, int LIMV>
 __global__ __launch_bounds__(256)
-void k_emf_march(Box3 g, const double *__restrict__ Vs, const R *__restrict__ FD, R *__restrict__ E)
+void k_emf_march(Box3 g, int L, const double *__restrict__ Vs, const R *__restrict__ FD, R *__restrict__ E)
 {
   const int ntx = (g.nx + 63) >> 6, nty = (g.ny + 3) >> 2;
   const int t = xcd_tile(blockIdx.x, gridDim.x);
@@ -824,9 +824,12 @@ void k_emf_march(Box3 g, const double *__restrict__ Vs, const R *__restrict__ FD
 // the (x0-1, y0-1) corner) is one task per lane.  The loads of plane k+1
 // are issued before plane k is computed, so their latency hides behind it.
 // The z-stencils and the face records of plane k-1 stay in registers.
-template <typename R, int LIMV, int L>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 3 : 1)))
-void k_emf_tile(Box3 g, const double *__restrict__ Vs, const R *__restrict__ FD, R *__restrict__ E)
+// Registers: three waves per SIMD with the MC limiter (168 VGPRs); the van Leer
+// limiter's divisions need 230, and held to three waves they spilled 133 VGPRs
+// (192^3: 1086 us at three waves, 306 at two).
+template <typename R, int LIMV>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? (LIMV == MC_LIM ? 3 : 2) : 1)))
+void k_emf_tile(Box3 g, int L, const double *__restrict__ Vs, const R *__restrict__ FD, R *__restrict__ E)
 {
   constexpr int TX = 64, TY = 4;
   __shared__ R xs[4][TY][TX + 3];        // By, e[K][J], Bz, e[J][K] at x0-2 .. x0+64
@@ -1011,13 +1014,22 @@ void k_emf_tile(Box3 g, const double *__restrict__ Vs, const R *__restrict__ FD,
 }
 
 // The same edge EMFs with one thread per edge and every stencil value loaded
-// from memory (2D thread blocks over x-y; blockIdx.z is the plane).
+// from memory; blockIdx.z is the plane.  64 x 4 blocks over x-y, which share
+// the y stencils through L1, or (flat != 0, gridDim.y = 1) 256 consecutive
+// edges of the plane for rows that 64-wide blocks would leave partly idle
+// (emf_flat).  The kernel of boxes too small for the tiles (engine: emf_choice).
 template <typename R, int LIMV, int NQ = 3>
 __global__ __launch_bounds__(256)
-void k_emf_edge(Box3 g, const double *__restrict__ Vs, const R *__restrict__ FD, R *__restrict__ E)
+void k_emf_edge(Box3 g, int flat, const double *__restrict__ Vs, const R *__restrict__ FD,
+                R *__restrict__ E)
 {
   constexpr int NR = NQ == 4 ? 6 : 4;   // records per face: et, eb, then the weights' data
-  const int i = blockIdx.x*64 + (threadIdx.x & 63), j = blockIdx.y*4 + (threadIdx.x >> 6);
+  int i = blockIdx.x*64 + (threadIdx.x & 63), j = blockIdx.y*4 + (threadIdx.x >> 6);
+  if (flat) {
+    const int t = blockIdx.x*256 + threadIdx.x;
+    j = t / g.nx;
+    i = t - j*g.nx;
+  }
   const int k = blockIdx.z;
   if (i >= g.nx || j >= g.ny) return;
   const int nx = g.nx, ny = g.ny, nz = g.nz;
@@ -1181,6 +1193,10 @@ void k_finish(Box3 g, const R *__restrict__ E, const double *__restrict__ Vin,
   for (int nv = 0; nv < 8; nv++) sto(V + nv*n, c, (R)v[nv]);
 }
 
+// 64-wide blocks leave more than a fifth of their lanes idle on these rows
+// (80 x 95 x 66: 39 us with 64 x 4 blocks, 32 flat; 96^3: 51 against 43)
+static inline int emf_flat(int nx) { return ((nx + 63)/64)*64*4 > 5*nx; }
+
 // ---------------------------------------------------------------------------
 // Host-side launch helpers: one entry per kernel family, so that the host
 // orchestration can bracket each launch with timing events.
@@ -1243,35 +1259,19 @@ static void launch_t(int which, const Mhd3dBufs<R> &b, const Box3 &g, const Step
     break;
   }
   case K_EMF: {
+    const int flat = emf_flat(g.nx);
+    const dim3 ge = flat ? dim3((g.nx*g.ny + 255)/256, 1, g.nz) : dim3((g.nx + 63)/64, (g.ny + 3)/4, g.nz);
     if (SOLVER == 4) {                   // UCT_HLLD: six records per face, one edge per thread
-      hipLaunchKernelGGL((k_emf_edge<R, LIM, 4>), dim3((g.nx + 63)/64, (g.ny + 3)/4, g.nz), dim3(256), 0, s,
-                         g, b.Vin, b.FD, b.E);
+      hipLaunchKernelGGL((k_emf_edge<R, LIM, 4>), ge, dim3(256), 0, s, g, flat, b.Vin, b.FD, b.E);
     } else if (b.emf_march == 0) {
-      hipLaunchKernelGGL((k_emf_edge<R, LIM>), dim3((g.nx + 63)/64, (g.ny + 3)/4, g.nz), dim3(256), 0, s,
-                         g, b.Vin, b.FD, b.E);
-    } else if (b.emf_march == 4) {
-      const int nt = ((g.nx + 63)/64)*((g.ny + 3)/4)*((g.nz + 3)/4);
-      hipLaunchKernelGGL((k_emf_march<R, LIM, 4>), dim3(nt), dim3(256), 0, s, g, b.Vin, b.FD, b.E);
-    } else if (b.emf_march < 0) {        // LDS-staged tiles marching -emf_march planes
-      const int lt = -b.emf_march;
-      const int nt = ((g.nx + 63)/64)*((g.ny + 3)/4)*((nk + lt - 1)/lt);
-      if (lt == 4)
-        hipLaunchKernelGGL((k_emf_tile<R, LIM, 4>), dim3(nt), dim3(256), 0, s, g, b.Vin, b.FD, b.E);
-      else if (lt == 8)
-        hipLaunchKernelGGL((k_emf_tile<R, LIM, 8>), dim3(nt), dim3(256), 0, s, g, b.Vin, b.FD, b.E);
-      else if (lt == 16)
-        hipLaunchKernelGGL((k_emf_tile<R, LIM, 16>), dim3(nt), dim3(256), 0, s, g, b.Vin, b.FD, b.E);
-      else
-        hipLaunchKernelGGL((k_emf_tile<R, LIM, 32>), dim3(nt), dim3(256), 0, s, g, b.Vin, b.FD, b.E);
-    } else if (b.emf_march == 8) {
-      const int nt = ((g.nx + 63)/64)*((g.ny + 3)/4)*((g.nz + 7)/8);
-      hipLaunchKernelGGL((k_emf_march<R, LIM, 8>), dim3(nt), dim3(256), 0, s, g, b.Vin, b.FD, b.E);
-    } else if (b.emf_march == 32) {
-      const int nt = ((g.nx + 63)/64)*((g.ny + 3)/4)*((g.nz + 31)/32);
-      hipLaunchKernelGGL((k_emf_march<R, LIM, 32>), dim3(nt), dim3(256), 0, s, g, b.Vin, b.FD, b.E);
+      hipLaunchKernelGGL((k_emf_edge<R, LIM>), ge, dim3(256), 0, s, g, flat, b.Vin, b.FD, b.E);
     } else {
-      const int nt = ((g.nx + 63)/64)*((g.ny + 3)/4)*((g.nz + 15)/16);
-      hipLaunchKernelGGL((k_emf_march<R, LIM, 16>), dim3(nt), dim3(256), 0, s, g, b.Vin, b.FD, b.E);
+      const int l = b.emf_march < 0 ? -b.emf_march : b.emf_march;
+      const int nt = ((g.nx + 63)/64)*((g.ny + 3)/4)*((nk + l - 1)/l);
+      if (b.emf_march < 0)               // LDS-staged tiles
+        hipLaunchKernelGGL((k_emf_tile<R, LIM>), dim3(nt), dim3(256), 0, s, g, l, b.Vin, b.FD, b.E);
+      else                               // register march
+        hipLaunchKernelGGL((k_emf_march<R, LIM>), dim3(nt), dim3(256), 0, s, g, l, b.Vin, b.FD, b.E);
     }
     break;
   }

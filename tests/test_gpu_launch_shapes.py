@@ -47,3 +47,15 @@ def test_march_lengths_mixed(n, monkeypatch):
         got = _run(n, 4, 1e-3, precision="mixed")
         assert got[0] == ref[0]
         assert all(np.array_equal(a, b) for a, b in zip(got[1:], ref[1:])), march
+
+
+@pytest.mark.parametrize("n", [(15, 11, 9), (80, 10, 7), (130, 101, 79)])
+@pytest.mark.parametrize("lim", ["MC_LIM", "VANLEER_LIM"])
+def test_emf_choice_matches_tiles(n, lim, monkeypatch):
+    """The EMF kernel of the box's size (flat or 64 x 4 edges, tiles of 8 above
+    a million cells) against tiles of 16 planes."""
+    got = _run(n, 2, 1e-3, lim=lim)
+    monkeypatch.setenv("GPL_EMF_MARCH", "-16")
+    ref = _run(n, 2, 1e-3, lim=lim)
+    assert got[0] == ref[0] and got[0][0] == 0
+    assert all(np.array_equal(a, b) for a, b in zip(got[1:], ref[1:]))
