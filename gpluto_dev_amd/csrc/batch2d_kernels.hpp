@@ -185,7 +185,7 @@ void k2_sweepx(Batch2dBufs<R> b, R gamma, int want_cdt)
       if (want_cdt) b.Cdt[c0] = (R)(0.5*((double)cm + (double)cmn)/bx.dx);
     }
   }
-  if (e) atomicOr(b.err, e);
+  report_bits(b.err, e);
 }
 
 // ---------------------------------------------------------------------------
@@ -289,7 +289,7 @@ void k2_sweepy(Batch2dBufs<R> b, RKW w, int first_stage, int want_cdt, R gamma)
       if (lane == 0) b.cdt_part[it] = m;
     }
   }
-  if (e) atomicOr(b.err, e);
+  report_bits(b.err, e);
 }
 
 // ---------------------------------------------------------------------------
@@ -401,7 +401,7 @@ void k2_finish(Batch2dBufs<R> b, RKW w, int first_stage, double gmm1, double sma
 #pragma unroll
     for (int s = 0; s < 8; s++) b.V[s*n + c] = (R)v[s];
   }
-  if (eall) atomicOr(b.err, eall);
+  report_bits(b.err, eall);
 }
 
 // ---------------------------------------------------------------------------

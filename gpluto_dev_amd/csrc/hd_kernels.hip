@@ -149,7 +149,7 @@ void k_hd_sweep(HdBox g, const double *__restrict__ V, double *__restrict__ Vout
       if (want_cdt) cdt_max = cd;
     }
   }
-  if (e) atomicOr(err, e);
+  report_bits(err, e);
   if (LAST && want_cdt) {
     const double m = hd_block_max(cdt_max);
     if (threadIdx.x == 0) cdt_part[blockIdx.x] = m;

@@ -246,7 +246,7 @@ void k_sweep(Box3 g, const R *__restrict__ V, const double *__restrict__ Vs,
   Fd[4*n + c] = ff.f[7];
   CM[(size_t)D*n + c] = rmax(rabs(ff.Sl), rabs(ff.Sr));
   uct_store<R, D, SOLVER>(vl, vr, gamma, ff, FD + (size_t)D*uct_nrec<SOLVER>()*n, c, n);
-  if (ff.err && face_reported<D>(g, p.i, p.j, p.k)) atomicOr(err, ff.err);
+  if (ff.err && face_reported<D>(g, p.i, p.j, p.k)) report_bits(err, ff.err);
 }
 
 // ---------------------------------------------------------------------------
@@ -366,7 +366,7 @@ void k_sweepx_fused(Box3 g, const R *__restrict__ V, const double *__restrict__ 
   }
   if (want_cdt) sto(Cdt, c, (R)(0.5*((double)sF[5*nx + i] + (double)sF[5*nx + ip])/g.dx));
   if (ff.err && face_reported<0>(g, i, (int)(row % g.ny), (int)(row / g.ny)))
-    atomicOr(err, ff.err);
+    report_bits(err, ff.err);
 }
 
 // ---------------------------------------------------------------------------
@@ -533,7 +533,7 @@ void k_sweep_xy(Box3 g, int L, const R *__restrict__ V, const double *__restrict
 #pragma unroll
     for (int q = 0; q < 7; q++) { Vm[q] = Vc[q]; Vc[q] = Vp[q]; }
   }
-  if (e) atomicOr(err, e);
+  report_bits(err, e);
 }
 
 // ---------------------------------------------------------------------------
@@ -688,7 +688,7 @@ void k_sweep_march(Box3 g, int L, const R *__restrict__ V, const double *__restr
       for (int q = 0; q < 7; q++) { Vm[q] = Vc[q]; Vc[q] = Vp[q]; }
     }
   }
-  if (e) atomicOr(err, e);
+  report_bits(err, e);
   if (D == 2 && want_cdt) {
     const double m = block_max(cdt_max);
     if (threadIdx.x == 0) cdt_part[g.part0 + blockIdx.x] = m;
@@ -1176,7 +1176,7 @@ void k_finish(Box3 g, const R *__restrict__ E, const double *__restrict__ Vin,
       sto(U + 4*n, c, u8[7]);
     }
     if (is_active(g, p.i, p.j, p.k)) {
-      if (e) atomicOr(err, e);
+      report_bits(err, e);
       zone_report(zr, c, e);
     }
   } else {
@@ -1185,7 +1185,7 @@ void k_finish(Box3 g, const R *__restrict__ E, const double *__restrict__ Vin,
     if (e) {
 #pragma unroll
       for (int nv = 0; nv < 5; nv++) sto(U + nv*n, c, u[nv]);
-      if (is_active(g, p.i, p.j, p.k)) atomicOr(err, e);
+      if (is_active(g, p.i, p.j, p.k)) report_bits(err, e);
     }
     if (is_active(g, p.i, p.j, p.k)) zone_report(zr, c, e);
   }
