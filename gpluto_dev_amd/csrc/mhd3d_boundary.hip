@@ -20,112 +20,112 @@ namespace gpl {
 
 namespace {
 
-__device__ __forceinline__ size_t pid(const Box3 &g, int i, int j, int k)
-{
-  return (size_t)i + (size_t)g.nx*((size_t)j + (size_t)g.ny*k);
-}
-
-// one thread per (layer, a, b): layer 0, 1 the two ghost layers, layer 2 the
-// extra normal face of an upper periodic side
+// Both sides of direction dir (blockIdx.y: lower, upper), one thread per
+// transverse (a, b) of the padded box and both ghost layers.  The two sides
+// write different layers and read active ones, and everything a ghost cell
+// needs (its copied cells and tangential faces, the outflow side's normal faces
+// outward from the boundary, the field average) is computed from the source
+// layers in registers, so a direction is one launch without a barrier: three
+// launches a stage where a copy and a fill per side were twelve.  These
+// launches are latency, not bytes: 80 x 95 x 66, 81 us a stage in twelve,
+// 32 us in three.  The directions stay in turn: a later one reads the
+// ghosts of an earlier one in its corners.
 template <typename R>
 __global__ __launch_bounds__(256)
-void k_bnd_copy(Box3 g, int side, int type, R *__restrict__ V, double *__restrict__ Vs)
+void k_bnd_dir(Box3 g, int dir, int type_lo, int type_hi, R *__restrict__ V, double *__restrict__ Vs)
 {
-  const int dir = side >> 1, upper = side & 1;
+  const int upper = blockIdx.y, type = upper ? type_hi : type_lo;
   const int t1 = (dir + 1) % 3, t2 = (dir + 2) % 3;
   const int P[3] = {g.nx, g.ny, g.nz};
   const int na = P[t1], nb = P[t2];
   const int t = blockIdx.x*blockDim.x + threadIdx.x;
-  if (t >= 3*na*nb) return;
-  const int layer = t / (na*nb), r = t - layer*na*nb, b = r / na, a = r - b*na;
-  const int n = g.hi[dir] - g.lo[dir] + 1;
-  const int gi = upper ? g.hi[dir] + 1 + layer : layer;          // ghost index along dir
-  // reflective: the mirror image i0 - i, i0 = 2*lo - 1 or 2*hi + 1 (Src/boundary.cpp:939-945)
-  const int i0 = upper ? 2*g.hi[dir] + 1 : 2*g.lo[dir] - 1;
-  const int src = type == GPL_PERIODIC ? gi + (upper ? -n : n)
-                : type == GPL_REFLECTIVE ? i0 - gi : (upper ? g.hi[dir] : g.lo[dir]);
-  int p[3], q[3];
-  p[dir] = gi; p[t1] = a; p[t2] = b;
-  q[dir] = src; q[t1] = a; q[t2] = b;
-  const size_t N = (size_t)g.ncell;
-  const size_t cp = pid(g, p[0], p[1], p[2]), cq = pid(g, q[0], q[1], q[2]);
-  const bool cell = layer < 2 && a <= na - 2 && b <= nb - 2;    // BOX_LOOP over the ghost box
-  if (cell) {
-    for (int nv = 0; nv < 8; nv++) {
-      const R v = V[nv*N + cq];
-      // FlipSign (Src/boundary.cpp:840-925): a wall negates the normal velocity and field
-      V[nv*N + cp] = type == GPL_REFLECTIVE && (nv == 1 + dir || nv == 4 + dir) ? -v : v;
-    }
-  }
-  if (layer < 2) {
-    // tangential components: one more face along the component (BOX{I,J,K}_LOOP)
-    if (a <= na - 1 && b <= nb - 2) Vs[t1*N + cp] = Vs[t1*N + cq];
-    if (a <= na - 2 && b <= nb - 1) Vs[t2*N + cp] = Vs[t2*N + cq];
-  }
-  // periodic normal component: BOX_LOOP on the lower side, BOXI/J/K_LOOP (one
-  // more face, the spare layer) on the upper side
-  if (type == GPL_PERIODIC && a <= na - 2 && b <= nb - 2 && (layer < 2 || upper))
-    Vs[dir*N + cp] = Vs[dir*N + cq];
-  // reflective normal component, mirrored about the boundary face and
-  // negated: face i from i0 - i + 1 on the lower side, face i + 1 from i0 - i
-  // on the upper side
-  if (type == GPL_REFLECTIVE && layer < 2 && a <= na - 2 && b <= nb - 2) {
-    int t[3] = {p[0], p[1], p[2]}, f[3] = {q[0], q[1], q[2]};
-    if (!upper) f[dir] += 1;
-    else        t[dir] += 1;
-    Vs[dir*N + pid(g, t[0], t[1], t[2])] = -Vs[dir*N + pid(g, f[0], f[1], f[2])];
-  }
-}
-
-// one thread per transverse (a, b) of the ghost box: the outflow side's
-// normal faces outward from the boundary, then the ghost cells' field average
-template <typename R>
-__global__ __launch_bounds__(256)
-void k_bnd_fill(Box3 g, int side, int type, R *__restrict__ V, double *__restrict__ Vs)
-{
-  const int dir = side >> 1, upper = side & 1;
-  const int t1 = (dir + 1) % 3, t2 = (dir + 2) % 3;
-  const int P[3] = {g.nx, g.ny, g.nz};
-  const int na = P[t1] - 1, nb = P[t2] - 1;                       // cells 0 .. ntot-1
-  const int t = blockIdx.x*blockDim.x + threadIdx.x;
   if (t >= na*nb) return;
   const int b = t / na, a = t - b*na;
-  const size_t N = (size_t)g.ncell;
-  // face areas of the uniform Cartesian grid (Src/set_geometry.cpp:124,147,166)
-  const double A[3] = {1.0*g.dy*g.dz, g.dx*1.0*g.dz, g.dx*g.dy*1.0};
-  const double *B[3] = {Vs, Vs + N, Vs + 2*N};
-  double *Bn = Vs + dir*N;
-  if (type == GPL_OUTFLOW) {
-    for (int l = 0; l < 2; l++) {
-      const int i = upper ? g.hi[dir] + 1 + l : g.lo[dir] - 1 - l;
-      int p[3];
-      p[dir] = i; p[t1] = a; p[t2] = b;
-      double dB[3];
+  const size_t S[3] = {1, (size_t)g.nx, (size_t)g.nx*g.ny};
+  const size_t N = (size_t)g.ncell, at = a*S[t1] + b*S[t2], s1 = S[t1], s2 = S[t2], sd = S[dir];
+  const int lo = g.lo[dir], hi = g.hi[dir], n = hi - lo + 1;
+  const int g0 = upper ? hi + 1 : 0;            // ghost layers g0, g0 + 1
+  // source layer of ghost layer gi; reflective: the mirror image i0 - i,
+  // i0 = 2*lo - 1 or 2*hi + 1 (Src/boundary.cpp:939-945)
+  auto source = [&](int gi) {
+    return type == GPL_PERIODIC ? gi + (upper ? -n : n)
+         : type == GPL_REFLECTIVE ? (upper ? 2*hi + 1 : 2*lo - 1) - gi : (upper ? hi : lo);
+  };
+  double *B1 = Vs + t1*N, *B2 = Vs + t2*N, *Bn = Vs + dir*N;
+  const bool cell = a <= na - 2 && b <= nb - 2; // BOX_LOOP over the ghost box
+  double e1[2][2], e2[2][2];                    // tangential faces on both ends of the ghost cells
 #pragma unroll
-      for (int d = 0; d < 3; d++) {
-        int q[3] = {p[0], p[1], p[2]};
-        q[d] += 1;
-        dB[d] = A[d]*B[d][pid(g, q[0], q[1], q[2])] - A[d]*B[d][pid(g, p[0], p[1], p[2])];
+  for (int l = 0; l < 2; l++) {
+    const size_t cp = at + (g0 + l)*sd, cq = at + source(g0 + l)*sd;
+    // tangential components: one more face along the component (BOX{I,J,K}_LOOP)
+    if (b <= nb - 2) { e1[l][0] = B1[cq]; B1[cp] = e1[l][0]; }
+    if (a <= na - 2) { e2[l][0] = B2[cq]; B2[cp] = e2[l][0]; }
+    if (cell) {
+      e1[l][1] = B1[cq + s1];
+      e2[l][1] = B2[cq + s2];
+      constexpr int VAR[5] = {0, 1, 2, 3, 7};   // B1..3 are the field average below
+#pragma unroll
+      for (int q = 0; q < 5; q++) {
+        const int nv = VAR[q];
+        const R v = V[nv*N + cq];
+        // FlipSign (Src/boundary.cpp:840-925): a wall negates the normal velocity and field
+        V[nv*N + cp] = type == GPL_REFLECTIVE && nv == 1 + dir ? -v : v;
       }
-      // the two transverse terms in x, y, z order
-      const double ta = dir == 0 ? dB[1] : dB[0], tb = dir == 2 ? dB[1] : dB[2];
-      int q[3] = {p[0], p[1], p[2]};
-      q[dir] += 1;
-      if (!upper) Bn[pid(g, p[0], p[1], p[2])] = (A[dir]*Bn[pid(g, q[0], q[1], q[2])] + ta + tb)/A[dir];
-      else        Bn[pid(g, q[0], q[1], q[2])] = (A[dir]*Bn[pid(g, p[0], p[1], p[2])] - (ta + tb))/A[dir];
     }
   }
-  for (int l = 0; l < 2; l++) {
-    const int i = upper ? g.hi[dir] + 1 + l : l;
-    int p[3];
-    p[dir] = i; p[t1] = a; p[t2] = b;
-    const size_t c = pid(g, p[0], p[1], p[2]);
+  if (!cell) return;
+  // the normal faces f0 .. f0 + 2 that bound the two ghost cells
+  const int f0 = upper ? hi + 1 : 0;
+  double f[3];
+  if (type == GPL_PERIODIC) {
+    // BOX_LOOP on the lower side, BOXI/J/K_LOOP (one more face, the spare
+    // layer) on the upper side
 #pragma unroll
-    for (int d = 0; d < 3; d++) {
-      int q[3] = {p[0], p[1], p[2]};
-      q[d] += 1;
-      V[(4 + d)*N + c] = (R)(0.5*(B[d][c] + B[d][pid(g, q[0], q[1], q[2])]));
+    for (int l = 0; l < 3; l++)
+      f[l] = !upper && l == 2 ? Bn[at + lo*sd] : Bn[at + source(f0 + l)*sd];
+    Bn[at + f0*sd] = f[0];
+    Bn[at + (f0 + 1)*sd] = f[1];
+    if (upper) Bn[at + (f0 + 2)*sd] = f[2];
+  } else if (type == GPL_REFLECTIVE) {
+    // mirrored about the boundary face and negated: face i from i0 - i + 1 on
+    // the lower side, face i + 1 from i0 - i on the upper side
+    if (!upper) {
+      f[0] = -Bn[at + (source(0) + 1)*sd];
+      f[1] = -Bn[at + (source(1) + 1)*sd];
+      f[2] = Bn[at + lo*sd];
+      Bn[at] = f[0];
+      Bn[at + sd] = f[1];
+    } else {
+      f[0] = Bn[at + f0*sd];
+      f[1] = -Bn[at + source(hi + 1)*sd];
+      f[2] = -Bn[at + source(hi + 2)*sd];
+      Bn[at + (f0 + 1)*sd] = f[1];
+      Bn[at + (f0 + 2)*sd] = f[2];
     }
+  } else {
+    // outward from the boundary face with div B = 0; face areas of the uniform
+    // Cartesian grid (Src/set_geometry.cpp:124,147,166)
+    const double A[3] = {1.0*g.dy*g.dz, g.dx*1.0*g.dz, g.dx*g.dy*1.0};
+    f[upper ? 0 : 2] = Bn[at + (upper ? hi + 1 : lo)*sd];
+#pragma unroll
+    for (int l = 0; l < 2; l++) {
+      const int c = upper ? l : 1 - l;          // the ghost cell crossed, outward
+      const double d1 = A[t1]*e1[c][1] - A[t1]*e1[c][0];
+      const double d2 = A[t2]*e2[c][1] - A[t2]*e2[c][0];
+      // the two transverse terms in x, y, z order: (t1, t2) is (y, z), (z, x), (x, y)
+      const double ta = dir == 1 ? d2 : d1, tb = dir == 1 ? d1 : d2;
+      if (!upper) f[c] = (A[dir]*f[c + 1] + ta + tb)/A[dir];
+      else        f[c + 1] = (A[dir]*f[c] - (ta + tb))/A[dir];
+    }
+    Bn[at + (upper ? f0 + 1 : 0)*sd] = f[upper ? 1 : 0];
+    Bn[at + (upper ? f0 + 2 : 1)*sd] = f[upper ? 2 : 1];
+  }
+#pragma unroll
+  for (int l = 0; l < 2; l++) {
+    const size_t c = at + (g0 + l)*sd;
+    V[(4 + dir)*N + c] = (R)(0.5*(f[l] + f[l + 1]));
+    V[(4 + t1)*N + c] = (R)(0.5*(e1[l][0] + e1[l][1]));
+    V[(4 + t2)*N + c] = (R)(0.5*(e2[l][0] + e2[l][1]));
   }
 }
 
@@ -134,14 +134,11 @@ void k_bnd_fill(Box3 g, int side, int type, R *__restrict__ V, double *__restric
 template <typename R>
 void mhd3d_boundary(const Box3 &g, const int type[6], R *V, double *Vs, hipStream_t s)
 {
-  for (int side = 0; side < 6; side++) {
-    const int dir = side >> 1;
+  for (int dir = 0; dir < 3; dir++) {
     const int P[3] = {g.nx, g.ny, g.nz};
     const int na = P[(dir + 1) % 3], nb = P[(dir + 2) % 3];
-    hipLaunchKernelGGL((k_bnd_copy<R>), dim3((3*na*nb + 255)/256), dim3(256), 0, s,
-                       g, side, type[side], V, Vs);
-    hipLaunchKernelGGL((k_bnd_fill<R>), dim3(((na - 1)*(nb - 1) + 255)/256), dim3(256), 0, s,
-                       g, side, type[side], V, Vs);
+    hipLaunchKernelGGL((k_bnd_dir<R>), dim3((na*nb + 255)/256, 2), dim3(256), 0, s,
+                       g, dir, type[2*dir], type[2*dir + 1], V, Vs);
   }
 }
 
