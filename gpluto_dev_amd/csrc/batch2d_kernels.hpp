@@ -191,9 +191,9 @@ void k2_sweepx(Batch2dBufs<R> b, R gamma, int want_cdt)
 // ---------------------------------------------------------------------------
 // y sweep + RK combination of U + C_dt maximum per item
 // ---------------------------------------------------------------------------
-template <typename R, int LIM, int SOLVER, int L>
+template <typename R, int LIM, int SOLVER>
 __global__ __launch_bounds__(256)
-void k2_sweepy(Batch2dBufs<R> b, RKW w, int first_stage, int want_cdt, R gamma)
+void k2_sweepy(Batch2dBufs<R> b, int L, RKW w, int first_stage, int want_cdt, R gamma)
 {
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const size_t n = (size_t)b.ncell;
@@ -407,16 +407,16 @@ void k2_finish(Batch2dBufs<R> b, RKW w, int first_stage, double gmm1, double sma
 // ---------------------------------------------------------------------------
 // host launchers
 // ---------------------------------------------------------------------------
-template <typename R, int LIM, int SOLVER, int L>
+template <typename R, int LIM, int SOLVER>
 static void b2_launch_t(int phase, const Batch2dBufs<R> &b, RKW w, int first_stage, int want_dt,
-                        int blocks, double gamma, double small_rho, double small_prs, hipStream_t s)
+                        int march, int blocks, double gamma, double small_rho, double small_prs, hipStream_t s)
 {
   switch (phase) {
   case B2_SWEEP_X:
     hipLaunchKernelGGL((k2_sweepx<R, LIM, SOLVER>), dim3(blocks), dim3(256), 0, s, b, (R)gamma, want_dt);
     break;
   case B2_SWEEP_Y:
-    hipLaunchKernelGGL((k2_sweepy<R, LIM, SOLVER, L>), dim3(blocks), dim3(256), 0, s, b, w, first_stage,
+    hipLaunchKernelGGL((k2_sweepy<R, LIM, SOLVER>), dim3(blocks), dim3(256), 0, s, b, march, w, first_stage,
                        want_dt, (R)gamma);
     break;
   case B2_EMF:
@@ -431,31 +431,21 @@ static void b2_launch_t(int phase, const Batch2dBufs<R> &b, RKW w, int first_sta
   }
 }
 
-template <typename R, int LIM, int SOLVER>
-static void b2_launch_l(int phase, const Batch2dBufs<R> &b, RKW w, int first_stage, int want_dt,
-                        int march, int blocks, double gamma, double small_rho, double small_prs,
-                        hipStream_t s)
-{
-  if (march == 8)       b2_launch_t<R, LIM, SOLVER, 8>(phase, b, w, first_stage, want_dt, blocks, gamma, small_rho, small_prs, s);
-  else if (march == 32) b2_launch_t<R, LIM, SOLVER, 32>(phase, b, w, first_stage, want_dt, blocks, gamma, small_rho, small_prs, s);
-  else                  b2_launch_t<R, LIM, SOLVER, 16>(phase, b, w, first_stage, want_dt, blocks, gamma, small_rho, small_prs, s);
-}
-
 template <typename R>
 void batch2d_launch(int phase, const Batch2dBufs<R> &b, RKW w, int first_stage, int want_dt,
                     int limiter, int solver, int march, int blocks, double gamma,
                     double small_rho, double small_prs, hipStream_t s)
 {
   if (limiter == MC_LIM) {
-    if (solver == 4)      b2_launch_l<R, MC_LIM, 4>(phase, b, w, first_stage, want_dt, march, blocks, gamma, small_rho, small_prs, s);
-    else if (solver == 3) b2_launch_l<R, MC_LIM, 3>(phase, b, w, first_stage, want_dt, march, blocks, gamma, small_rho, small_prs, s);
-    else if (solver == 2) b2_launch_l<R, MC_LIM, 2>(phase, b, w, first_stage, want_dt, march, blocks, gamma, small_rho, small_prs, s);
-    else                  b2_launch_l<R, MC_LIM, 1>(phase, b, w, first_stage, want_dt, march, blocks, gamma, small_rho, small_prs, s);
+    if (solver == 4)      b2_launch_t<R, MC_LIM, 4>(phase, b, w, first_stage, want_dt, march, blocks, gamma, small_rho, small_prs, s);
+    else if (solver == 3) b2_launch_t<R, MC_LIM, 3>(phase, b, w, first_stage, want_dt, march, blocks, gamma, small_rho, small_prs, s);
+    else if (solver == 2) b2_launch_t<R, MC_LIM, 2>(phase, b, w, first_stage, want_dt, march, blocks, gamma, small_rho, small_prs, s);
+    else                  b2_launch_t<R, MC_LIM, 1>(phase, b, w, first_stage, want_dt, march, blocks, gamma, small_rho, small_prs, s);
   } else {
-    if (solver == 4)      b2_launch_l<R, VANLEER_LIM, 4>(phase, b, w, first_stage, want_dt, march, blocks, gamma, small_rho, small_prs, s);
-    else if (solver == 3) b2_launch_l<R, VANLEER_LIM, 3>(phase, b, w, first_stage, want_dt, march, blocks, gamma, small_rho, small_prs, s);
-    else if (solver == 2) b2_launch_l<R, VANLEER_LIM, 2>(phase, b, w, first_stage, want_dt, march, blocks, gamma, small_rho, small_prs, s);
-    else                  b2_launch_l<R, VANLEER_LIM, 1>(phase, b, w, first_stage, want_dt, march, blocks, gamma, small_rho, small_prs, s);
+    if (solver == 4)      b2_launch_t<R, VANLEER_LIM, 4>(phase, b, w, first_stage, want_dt, march, blocks, gamma, small_rho, small_prs, s);
+    else if (solver == 3) b2_launch_t<R, VANLEER_LIM, 3>(phase, b, w, first_stage, want_dt, march, blocks, gamma, small_rho, small_prs, s);
+    else if (solver == 2) b2_launch_t<R, VANLEER_LIM, 2>(phase, b, w, first_stage, want_dt, march, blocks, gamma, small_rho, small_prs, s);
+    else                  b2_launch_t<R, VANLEER_LIM, 1>(phase, b, w, first_stage, want_dt, march, blocks, gamma, small_rho, small_prs, s);
   }
 }
 

@@ -25,7 +25,8 @@ using namespace gpl;
 
 namespace {
 
-constexpr int kMarch[3] = {8, 16, 32};
+constexpr int kMarch[3] = {8, 16, 32};     // the autotuner's y-march lengths
+constexpr int kAuto = 3;                   // index of the length chosen by size (one box)
 constexpr int kBpc[4] = {2, 4, 8, 0};      // workgroups per CU; 0 = one per work group
 
 template <typename T>
@@ -75,9 +76,9 @@ struct gpl_batch {
   Item4 *xitems = nullptr;
   Item2 *tiles = nullptr;
   int nx_items = 0, ntiles = 0;
-  Item4 *yitems[3] = {nullptr, nullptr, nullptr};   // per march length
-  int *part_beg[3] = {nullptr, nullptr, nullptr};
-  int ny_items[3] = {0, 0, 0};
+  Item4 *yitems[4] = {};                            // per march length
+  int *part_beg[4] = {};
+  int ny_items[4] = {};
   // Box groups on streams of their own: group g holds boxes [gbox[g],
   // gbox[g+1]) with about the same number of cells.  The groups share no
   // cell, so their phases run side by side and fill each other's
@@ -88,8 +89,9 @@ struct gpl_batch {
   int gbox[kMaxGroups + 1] = {};
   hipStream_t gs[kMaxGroups] = {};
   hipEvent_t ev_fork = nullptr, ev_join[kMaxGroups] = {};
-  int xbeg[kMaxGroups + 1] = {}, tbeg[kMaxGroups + 1] = {}, ybeg[3][kMaxGroups + 1] = {};
+  int xbeg[kMaxGroups + 1] = {}, tbeg[kMaxGroups + 1] = {}, ybeg[4][kMaxGroups + 1] = {};
   // launch shape
+  int march[4] = {kMarch[0], kMarch[1], kMarch[2], 0};
   int march_idx = 1, bpc_idx = 2;
   bool tune_pending = true;
   double tuned_ms = 0.0;
@@ -105,8 +107,8 @@ static void batch_free(gpl_batch *b)
 {
   void *ptrs[] = {b->V, b->FD, b->E, b->dU, b->Cdt, b->U, b->Us, b->vs[0], b->vs[1], b->vs[2],
                   b->cdt_part, b->box, b->xitems, b->tiles,
-                  b->yitems[0], b->yitems[1], b->yitems[2], b->part_beg[0], b->part_beg[1],
-                  b->part_beg[2]};
+                  b->yitems[0], b->yitems[1], b->yitems[2], b->yitems[3], b->part_beg[0],
+                  b->part_beg[1], b->part_beg[2], b->part_beg[3]};
   for (void *p : ptrs) if (p) (void)hipFree(p);
   if (b->graph_exec) hipGraphExecDestroy(b->graph_exec);
   if (b->ev_fork) hipEventDestroy(b->ev_fork);
@@ -183,9 +185,15 @@ static int batch_init(gpl_batch *b, const gpl_config *cfg, int nbox, const int *
   b->nx_items = (int)xi.size();
   b->ntiles = (int)ti.size();
   int max_y = 0;
-  std::vector<int> yb[3];
-  for (int m = 0; m < 3; m++) {
-    const int L = kMarch[m];
+  // a batch tunes its march length among kMarch; one box behind a gpl_ctx
+  // takes the length of its size
+  std::vector<int> yb[4];
+  if (env) {
+    b->march_idx = kAuto;
+    b->march[kAuto] = march_length(b->fp64, 64LL*((b->hbox[0].nx + 63)/64), b->hbox[0].ny);
+  }
+  for (int m = env ? kAuto : 0; m < (env ? kAuto + 1 : 3); m++) {
+    const int L = b->march[m];
     std::vector<Item4> yi;
     std::vector<int> pb;
     for (int q = 0; q < nbox; q++) {
@@ -232,7 +240,8 @@ static int batch_init(gpl_batch *b, const gpl_config *cfg, int nbox, const int *
     for (int g = 0; g <= ng; g++) {
       b->xbeg[g] = xstart[b->gbox[g]];
       b->tbeg[g] = tstart[b->gbox[g]];
-      for (int m = 0; m < 3; m++) b->ybeg[m][g] = yb[m][b->gbox[g]];
+      for (int m = 0; m < 4; m++)
+        if (!yb[m].empty()) b->ybeg[m][g] = yb[m][b->gbox[g]];
     }
     b->gs[0] = b->stream;
     if (ng > 1 && hipEventCreateWithFlags(&b->ev_fork, hipEventDisableTiming) != hipSuccess) return GPL_EHIP;
@@ -505,7 +514,7 @@ static void enqueue_stage(gpl_batch *b, const double *uin, double *uout, double 
   q.FD = (R *)b->FD; q.E = (R *)b->E; q.dU = (R *)b->dU; q.Cdt = (R *)b->Cdt;
   q.err = b->err; q.ctl = b->ctl; q.box = b->box;
   q.ncell = b->ncell;
-  const int m = b->march_idx, march = kMarch[m];
+  const int m = b->march_idx, march = b->march[m];
   const gpl_config &c = b->cfg;
   // the box groups, each on its own stream; the kernels index the items of
   // their group and the C_dt partial slots that go with them
@@ -702,7 +711,7 @@ extern "C" int gpl_batch_set_tuning(gpl_batch *b, int march, int blocks_per_cu)
 extern "C" int gpl_batch_get_tuning(const gpl_batch *b, int *march, int *blocks_per_cu, double *step_ms)
 {
   if (!b) return GPL_EINVAL;
-  if (march) *march = kMarch[b->march_idx];
+  if (march) *march = b->march[b->march_idx];
   if (blocks_per_cu) *blocks_per_cu = kBpc[b->bpc_idx];
   if (step_ms) *step_ms = b->tuned_ms;
   return 0;

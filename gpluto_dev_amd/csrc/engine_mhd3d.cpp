@@ -42,42 +42,6 @@ int from_device_v(void *src, bool fp64, std::vector<double> &dst)
   return 0;
 }
 
-// Cells per lane of a march along an extent of n cells, for `across` cells in
-// the plane it crosses.  A lane solves L + 1 faces for its L cells, one after
-// the other, and loads its window first (about half a face's time).  Long
-// marches waste the fewest solves; on a small box they leave most of the chip
-// idle.
-//
-// FP64: one wavefront's Riemann solve already fills a SIMD's issue slots about
-// as well as two, so a launch takes ceil(blocks / CUs) (L + 1.5).  The shortest
-// such time over L <= 16 is taken, L = 16 unless another is 5% shorter (a box
-// that streams from HBM gains nothing from the model).  y and z march, us at
-// L = 16 -> at the rule's L: 64^3 54 + 57 -> 23 + 25 (L = 4), RMHD HLLD
-// 50x44x38 276 + 285 -> 59 + 59 (L = 2), 16^3 52 + 53 -> 11 + 12 (L = 1);
-// 128^3 100 + 106 against 108 + 113 at 8 and 117 + 127 at 4.
-//
-// FP32: four wavefronts per SIMD hide the load latency, so L is the largest of
-// 8, 4, 2, 1 that leaves 8192 wavefronts (512 for the last halving).  z march
-// and x+y kernel, us at 16 -> rule: 64^3 48 + 64 -> 16 + 20 (L = 2), 128^3
-// 81 + 110 -> 82 + 90 (L = 4), 192^3 280 + 270 -> 250 + 263 (L = 8).
-int march_length(bool fp64, long long across, int n)
-{
-  if (!fp64) {
-    int l = 8;
-    while (l > 1 && across*((n + l - 1)/l)/64 < (l > 2 ? 8192 : 512)) l /= 2;
-    return l;
-  }
-  constexpr int kCUs = 256, kBlock = 256;
-  int best = 16;
-  double tbest = 0.0;
-  for (int l = 16; l >= 1; l--) {
-    const long long blocks = (across*((n + l - 1)/l) + kBlock - 1)/kBlock;
-    const double t = (double)((blocks + kCUs - 1)/kCUs)*(l + 1.5);
-    if (l == 16 || t < 0.95*tbest) { best = l; tbest = t; }
-  }
-  return best;
-}
-
 // EMF kernel of a box (Mhd3dBufs::emf_march): 0 one edge per thread, -n LDS
 // tiles of 64 x 4 edges marching n planes.  A tile reads every HBM byte about
 // once, but its planes follow one another, so it needs enough tiles to fill the

@@ -59,3 +59,42 @@ def test_emf_choice_matches_tiles(n, lim, monkeypatch):
     ref = _run(n, 2, 1e-3, lim=lim)
     assert got[0] == ref[0] and got[0][0] == 0
     assert all(np.array_equal(a, b) for a, b in zip(got[1:], ref[1:]))
+
+
+@pytest.mark.parametrize("n", [(3, 70, 1), (65, 19, 1), (130, 37, 1), (128, 515, 1)])
+@pytest.mark.parametrize("sides", [(), ("outflow", "reflective", "reflective", "outflow", "periodic", "periodic")])
+def test_one_2d_box_matches_oracle(n, sides):
+    """One 2D box: the y march's length follows from its size."""
+    import oracle
+    vc, vs = ic.mhd_turbulence(n, 4)
+    g = StageUpdate(Definitions(dimensions=2), RuntimeSetup(n=n, sides=sides))
+    g.upload(vc, vs)
+    res = g.run(4, 5e-4)
+    gvc, gvs, _ = g.download()
+    g.close()
+    o = oracle.Oracle(phys="mhd", n=n, gamma=5 / 3, sides=sides or None)
+    o.set_state(vc, vs)
+    assert res == o.run(4, 5e-4)
+    ovc, ovs, _ = o.get_state()
+    assert np.array_equal(gvc, ovc) and np.array_equal(gvs, ovs)
+
+
+@pytest.mark.parametrize("n", [(3, 4, 5), (9, 3, 3)])
+@pytest.mark.parametrize("sides", [
+    ("outflow", "reflective", "reflective", "reflective", "outflow", "outflow"),
+    ("periodic", "periodic", "outflow", "reflective", "reflective", "outflow"),
+    ("reflective", "outflow", "periodic", "periodic", "periodic", "periodic")])
+def test_sides_of_the_smallest_boxes(n, sides):
+    """Every side type on boxes whose two ghost fills reach the same cells."""
+    import oracle
+    vc, vs = ic.mhd_turbulence(n, 4)
+    g = StageUpdate(Definitions(), RuntimeSetup(n=n, sides=sides))
+    g.upload(vc, vs)
+    res = g.run(3, 5e-4)
+    gvc, gvs, _ = g.download()
+    g.close()
+    o = oracle.Oracle(phys="mhd", n=n, gamma=5 / 3, sides=sides)
+    o.set_state(vc, vs)
+    assert res == o.run(3, 5e-4)
+    ovc, ovs, _ = o.get_state()
+    assert np.array_equal(gvc, ovc) and np.array_equal(gvs, ovs)
