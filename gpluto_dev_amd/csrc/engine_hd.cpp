@@ -20,15 +20,18 @@ public:
   EngineEnv env;
   HdBox g;
   size_t n = 0;
-  double *VA = nullptr, *VB = nullptr;   // [5][n] primitives, ping-pong across stages
-  double *U = nullptr, *U0 = nullptr, *dU = nullptr, *Cdt = nullptr, *cdt_part = nullptr;
-  int nparts = 0;
-  double *cur_v = nullptr;
+  // [5][n] primitives and conserved state, two buffers each: 2D and 3D ping-pong
+  // the primitives across stages and keep U^n in UA (stage 1 writes UB, the last
+  // stage UA); 1D, one launch a step, ping-pongs both across steps
+  double *VA = nullptr, *VB = nullptr, *UA = nullptr, *UB = nullptr;
+  double *cur_v = nullptr, *cur_u = nullptr;
+  double *cdt_part = nullptr;
+  unsigned *arrived = nullptr;   // arrival counters of the launch that ends a step
   double *diag = nullptr;     // diagnostics partials (DIAG_BLOCKS rows) and result row
 
   ~HdEngine() override
   {
-    void *ptrs[] = {VA, VB, U, U0, dU, Cdt, cdt_part, diag};
+    void *ptrs[] = {VA, VB, UA, UB, cdt_part, diag};
     for (void *p : ptrs) if (p) (void)hipFree(p);
   }
 
@@ -47,26 +50,24 @@ public:
     g.dx = (c.xend[0] - c.xbeg[0])/c.nx;
     g.dy = (c.xend[1] - c.xbeg[1])/c.ny;
     g.dz = (c.xend[2] - c.xbeg[2])/c.nz;
-    nparts = hd_blocks(g);
     int rc = 0;
     rc |= dev_alloc(bytes, (void **)&VA, 5*n*sizeof(double));
     rc |= dev_alloc(bytes, (void **)&VB, 5*n*sizeof(double));
-    rc |= dev_alloc(bytes, (void **)&U, 5*n*sizeof(double));
-    rc |= dev_alloc(bytes, (void **)&U0, 5*n*sizeof(double));
-    if (g.dims > 1) {
-      rc |= dev_alloc(bytes, (void **)&dU, 5*n*sizeof(double));
-      rc |= dev_alloc(bytes, (void **)&Cdt, n*sizeof(double));
-    }
-    rc |= dev_alloc(bytes, (void **)&cdt_part, (size_t)nparts*sizeof(double));
+    // the arrival counters follow U^n, so that the upload clears them
+    rc |= dev_alloc(bytes, (void **)&UA, 5*n*sizeof(double) + HD_ARRIVED*sizeof(unsigned));
+    arrived = (unsigned *)(UA + 5*n);
+    rc |= dev_alloc(bytes, (void **)&UB, 5*n*sizeof(double));
+    rc |= dev_alloc(bytes, (void **)&cdt_part, (size_t)hd_blocks(g, nstages())*sizeof(double));
     rc |= dev_alloc(bytes, (void **)&diag, (size_t)(DIAG_BLOCKS + 1)*DIAG_MAXQ*sizeof(double));
     cur_v = VA;
+    cur_u = UA;
     return rc ? GPL_ENOMEM : 0;
   }
 
   int upload(const double *vc, const double *const *, int layout) override
   {
     const Layout L = make_layout(cfg, layout);
-    std::vector<double> hv(5*n), hu(5*n);
+    std::vector<double> hv(5*n), hu(5*n + HD_ARRIVED*sizeof(unsigned)/sizeof(double));
     for (int k = 0; k < L.nz; k++)
       for (int j = 0; j < L.ny; j++)
         for (int i = 0; i < L.nx; i++) {
@@ -78,9 +79,10 @@ public:
           for (int nv = 0; nv < 5; nv++) { hv[nv*n + o] = v[nv]; hu[nv*n + o] = u[nv]; }
         }
     if (hipMemcpy(VA, hv.data(), 5*n*sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(U, hu.data(), 5*n*sizeof(double), hipMemcpyHostToDevice) != hipSuccess)
+        hipMemcpy(UA, hu.data(), hu.size()*sizeof(double), hipMemcpyHostToDevice) != hipSuccess)
       return GPL_EHIP;
     cur_v = VA;
+    cur_u = UA;
     return 0;
   }
 
@@ -98,7 +100,7 @@ public:
       double *dst = which == 0 ? vc : uc;
       if (!dst) continue;
       std::vector<double> h(5*n);
-      if (hipMemcpy(h.data(), which == 0 ? cur_v : U, 5*n*sizeof(double), hipMemcpyDeviceToHost) != hipSuccess)
+      if (hipMemcpy(h.data(), which == 0 ? cur_v : cur_u, 5*n*sizeof(double), hipMemcpyDeviceToHost) != hipSuccess)
         return GPL_EHIP;
       for (int nv = 0; nv < 5; nv++)
         for (int k = 0; k < L.nz; k++)
@@ -115,29 +117,38 @@ public:
     const RKW w1 = {0.0, 0.0, 1.0};
     const RKW w2 = cfg.time_stepping == GPL_RK3 ? RKW{0.75, 0.25, 0.25} : RKW{0.5, 0.5, 0.5};
     const RKW w3 = {1.0/3.0, 2.0/3.0, 2.0/3.0};
-    const int nst = cfg.time_stepping == GPL_RK3 ? 3 : 2;
-    static const int kid[3] = {K_HD_X, K_HD_Y, K_HD_Z};
+    const int nst = nstages();
     double *in = cur_v, *out = cur_v == VA ? VB : VA;
     if (zcnt) launch_zone_reset(zcnt, env.stream);
+    HdStep ctl = {env.ctl, arrived, cfg.cfl, cfg.cfl_max_var, advance_dt, 1};
+    if (g.dims == 1) {
+      double *uo = cur_u == UA ? UB : UA;
+      const HdBufs b = {in, out, cur_u, cur_u, uo, cdt_part, env.err, {zone_rep(0), zone_rep(1), zone_rep(2)}};
+      if (t) t->begin(K_HD_X);
+      hd_launch_step1d(b, g, ctl, nst, cfg.limiter, cfg.solver, cfg.gamma, cfg.small_rho, cfg.small_prs,
+                       env.stream);
+      if (t) t->end(K_HD_X);
+      cur_v = out;
+      cur_u = uo;
+      return;
+    }
+    const int kid = g.dims == 2 ? K_HD_Y : K_HD_Z;
     for (int st = 1; st <= nst; st++) {
       const RKW w = st == 1 ? w1 : (st == 2 ? w2 : w3);
-      HdBufs b = {in, out, U, U0, dU, Cdt, cdt_part, env.err, zone_rep(st - 1)};
-      for (int d = 0; d < g.dims; d++) {
-        if (t) t->begin(kid[d]);
-        hd_launch(d, b, g, env.ctl, w, st == 1, st == 1, cfg.limiter, cfg.solver, cfg.gamma,
-                  cfg.small_rho, cfg.small_prs, env.stream);
-        if (t) t->end(kid[d]);
-      }
+      const ZoneRep z = zone_rep(st - 1);
+      const HdBufs b = {in, out, st == 1 ? UA : UB, UA, st == nst ? UA : UB, cdt_part, env.err, {z, z, z}};
+      ctl.ends_step = st == nst;
+      if (t) t->begin(kid);
+      hd_launch_stage(b, g, ctl, w, st == 1, st == 1, cfg.limiter, cfg.solver, cfg.gamma, cfg.small_rho,
+                      cfg.small_prs, env.stream);
+      if (t) t->end(kid);
       double *tmp = in; in = out; out = tmp;
     }
-    if (t) t->begin(K_DT);
-    launch_dt(cdt_part, nparts, (double)g.dims, env.ctl, cfg.cfl, cfg.cfl_max_var, advance_dt,
-              env.stream);
-    if (t) t->end(K_DT);
     cur_v = in;
   }
 
-  int graph_period() const override { return cfg.time_stepping == GPL_RK3 ? 2 : 1; }
+  // 1D: one flip of the buffers a step; 2D, 3D: one flip a stage
+  int graph_period() const override { return g.dims == 1 || cfg.time_stepping == GPL_RK3 ? 2 : 1; }
   const void *state_key() const override { return cur_v; }
 
   int nvar() const override { return 5; }

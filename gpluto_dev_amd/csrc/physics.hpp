@@ -544,49 +544,50 @@ GPL_HD void hd_max_signal_speed(const R *v, R gamma, R &cmin, R &cmax)
 }
 
 // HLLC, Src/HD/hllc.cpp:54-250 (ideal EOS, Davis speeds, HLL_Speed hd.hpp:165).
-// out.f[0..4] = rho, m1, m2, m3, E fluxes.
+// out.f[0..4] = rho, m1, m2, m3, E fluxes.  The side whose flux is taken (left
+// of the fan, right of it, or the contact's upwind side) is selected first and
+// the conserved state and the flux are evaluated for it alone: the expressions
+// of the reference on the selected values, so the same bits, with one
+// PrimToCons (and its division by gamma - 1) and one Flux instead of two, and
+// about 40 registers less.
 template <typename R, int N>
 GPL_HD void hd_hllc(const R *vl, const R *vr, R gamma, FaceFlux<R> &out)
 {
   constexpr int VXn = 1 + N, VXt = 1 + (N + 1)%3, VXb = 1 + (N + 2)%3;
   const R gmm1 = gamma - R(1);
-  R ul[5], ur[5], fl[5], fr[5], sl_min, sl_max, sr_min, sr_max;
-  hd_prim_to_cons(vl, ul, gmm1);
-  hd_prim_to_cons(vr, ur, gmm1);
-  hd_flux<R, N>(vl, ul, fl);
-  hd_flux<R, N>(vr, ur, fr);
+  R sl_min, sl_max, sr_min, sr_max;
   hd_max_signal_speed<R, N>(vl, gamma, sl_min, sl_max);
   hd_max_signal_speed<R, N>(vr, gamma, sr_min, sr_max);
   const R Sl = rmin(sl_min, sr_min);
   const R Sr = rmax(sl_max, sr_max);
   out.Sl = Sl; out.Sr = Sr;
+  // contact speed (hllc.cpp:194-200); ul[VXn] = vl[0]*vl[VXn]
+  const R qL = vl[4] + vl[0]*vl[VXn]*(vl[VXn] - Sl);
+  const R qR = vr[4] + vr[0]*vr[VXn]*(vr[VXn] - Sr);
+  const R wL = vl[0]*(vl[VXn] - Sl);
+  const R wR = vr[0]*(vr[VXn] - Sr);
+  const R vs = (qR - qL)/(wR - wL);
+  const bool outL = Sl > R(0), outR = Sr < R(0);
+  const bool left = outL || (!outR && vs >= R(0));
+  R v[5], u[5], f[5];
+  for (int nv = 0; nv < 5; nv++) v[nv] = left ? vl[nv] : vr[nv];
+  const R S = left ? Sl : Sr;
+  hd_prim_to_cons(v, u, gmm1);
+  hd_flux<R, N>(v, u, f);
+  // star state (hllc.cpp:202-232)
+  R us[5];
+  us[0] = u[0]*(S - v[VXn])/(S - vs);
+  us[VXn] = us[0]*vs;
+  us[VXt] = us[0]*v[VXt];
+  us[VXb] = us[0]*v[VXb];
+  us[4] =   u[4]/v[0]
+          + (vs - v[VXn])*(vs + v[4]/(v[0]*(S - v[VXn])));
+  us[4] *= us[0];
   R *flux = out.f;
-  if (Sl > R(0)) {
-    for (int nv = 0; nv < 5; nv++) flux[nv] = fl[nv];
-  } else if (Sr < R(0)) {
-    for (int nv = 0; nv < 5; nv++) flux[nv] = fr[nv];
-  } else {
-    // contact speed (hllc.cpp:194-200)
-    const R qL = vl[4] + ul[VXn]*(vl[VXn] - Sl);
-    const R qR = vr[4] + ur[VXn]*(vr[VXn] - Sr);
-    const R wL = vl[0]*(vl[VXn] - Sl);
-    const R wR = vr[0]*(vr[VXn] - Sr);
-    const R vs = (qR - qL)/(wR - wL);
-    // star states of the side that is used (hllc.cpp:202-232)
-    const bool left = vs >= R(0);
-    const R *v = left ? vl : vr;
-    const R *u = left ? ul : ur;
-    const R *f = left ? fl : fr;
-    const R S = left ? Sl : Sr;
-    R us[5];
-    us[0] = u[0]*(S - v[VXn])/(S - vs);
-    us[VXn] = us[0]*vs;
-    us[VXt] = us[0]*v[VXt];
-    us[VXb] = us[0]*v[VXb];
-    us[4] =   u[4]/v[0]
-            + (vs - v[VXn])*(vs + v[4]/(v[0]*(S - v[VXn])));
-    us[4] *= us[0];
-    for (int nv = 0; nv < 5; nv++) flux[nv] = f[nv] + S*(us[nv] - u[nv]);
+  const bool fan = !outL && !outR;
+  for (int nv = 0; nv < 5; nv++) {
+    const R star = f[nv] + S*(us[nv] - u[nv]);
+    flux[nv] = fan ? star : f[nv];
   }
   uint32_t err = 0;
   for (int nv = 0; nv < 5; nv++) if (risnan(flux[nv])) err |= ERR_NAN | ERR_QUIT;

@@ -98,3 +98,60 @@ def test_sides_of_the_smallest_boxes(n, sides):
     assert res == o.run(3, 5e-4)
     ovc, ovs, _ = o.get_state()
     assert np.array_equal(gvc, ovc) and np.array_equal(gvs, ovs)
+
+
+HD_SIDES = ["periodic", "outflow", "reflective"]
+
+
+@pytest.mark.parametrize("n,ts,lim,solver", [
+    # 1D: one wavefront per block up to 16384 zones (56 or 52 zones each), four above
+    ((3, 1, 1), "RK2", "MC_LIM", "hllc"), ((5, 1, 1), "RK3", "VANLEER_LIM", "hll"),
+    ((52, 1, 1), "RK3", "MC_LIM", "hllc"), ((56, 1, 1), "RK2", "VANLEER_LIM", "hllc"),
+    ((113, 1, 1), "RK2", "MC_LIM", "hll"), ((16385, 1, 1), "RK3", "MC_LIM", "hllc"),
+    ((16617, 1, 1), "RK2", "MC_LIM", "hllc"),
+    # 2D: 63 columns per wavefront
+    ((3, 3, 1), "RK2", "MC_LIM", "hllc"), ((62, 7, 1), "RK3", "MC_LIM", "hll"),
+    ((63, 40, 1), "RK2", "VANLEER_LIM", "hllc"), ((64, 33, 1), "RK2", "MC_LIM", "hllc"),
+    ((127, 190, 1), "RK3", "VANLEER_LIM", "hllc"),
+    # 3D: 64 x 7 cells per block
+    ((3, 3, 3), "RK3", "MC_LIM", "hllc"), ((63, 8, 5), "RK2", "VANLEER_LIM", "hllc"),
+    ((64, 7, 4), "RK2", "MC_LIM", "hll"), ((65, 15, 33), "RK3", "MC_LIM", "hllc"),
+    ((66, 6, 70), "RK2", "MC_LIM", "hllc")])
+@pytest.mark.parametrize("sides", [0, 1, 2])
+def test_hd_launch_shapes_match_oracle(n, ts, lim, solver, sides):
+    """HD boxes at the edges of the kernels' blocks; every side type in turn on
+    every direction, from a noisy blast."""
+    import oracle
+    dims = 1 if n[1] == 1 else 2 if n[2] == 1 else 3
+    t = []
+    for d in range(3):
+        if d >= dims or sides == 0:
+            t += ["periodic", "periodic"]
+        else:
+            t += [HD_SIDES[1 + (sides + d) % 2], HD_SIDES[1 + (sides + d + 1) % 2]]
+    vc = ic.hd_blast(n, 6)
+    print(f"case n={n} {ts} {lim} {solver} {t}", flush=True)
+    g = StageUpdate(Definitions(physics="HD", dimensions=dims, time_stepping=ts, limiter=lim),
+                    RuntimeSetup(n=n, solver=solver, sides=tuple(t), gamma=1.4))
+    g.upload(vc)
+    dt0 = 0.02/max(n)
+    res = g.run(5, dt0)
+    more = g.run(2, -1.0)                      # goes on from the device's dt
+    inv = g.advance_step(dt0)
+    gvc, _, guc = g.download()
+    g.close()
+    o = oracle.Oracle(phys="hd", n=n, gamma=1.4, solver=solver, limiter=lim, time_stepping=int(ts[-1]),
+                      sides=t)
+    o.set_state(vc)
+    assert res == o.run(5, dt0)
+    dt = res[2]
+    err, time = 0, res[1]
+    for _ in range(2):
+        e, i = o.advance(dt)
+        err |= e
+        time += dt
+        dt = min(0.4/i, 1.1*dt)
+    assert more == (err, time, dt)
+    assert inv == o.advance(dt0)
+    ovc, _, ouc = o.get_state()
+    assert np.array_equal(gvc, ovc) and np.array_equal(guc, ouc)
