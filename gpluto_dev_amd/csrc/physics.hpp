@@ -140,7 +140,7 @@ struct FaceFlux {
 
 // HLLD, Src/MHD/hlld.cpp:62-500 (ideal EOS, no GLM, no background field)
 template <typename R, int N>
-GPL_HD void mhd_hlld(const R *vl, const R *vr, R gamma, FaceFlux<R> &out)
+GPL_HD void mhd_hlld_both(const R *vl, const R *vr, R gamma, FaceFlux<R> &out)
 {
   constexpr int VXn = 1 + N, VXt = 1 + (N + 1)%3, VXb = 1 + (N + 2)%3;
   constexpr int MXn = VXn, MXt = VXt, MXb = VXb;
@@ -281,6 +281,157 @@ GPL_HD void mhd_hlld(const R *vl, const R *vr, R gamma, FaceFlux<R> &out)
   uint32_t err = 0;
   for (int nv = 0; nv < 8; nv++) if (risnan(flux[nv])) err |= ERR_NAN | ERR_QUIT;
   out.err = err;
+}
+
+// The same solver for FP64, written so that the side whose flux is taken (left
+// of the fan, right of it, or the side of the contact that the decision tree of
+// Src/MHD/hlld.cpp:303-470 picks) is selected before what only that side needs:
+// its conserved state (a division by gamma - 1), its flux, its star energy (a
+// division), its double-star state and the final sum.  Every value is the
+// reference's expression on the selected operands, so the bits are the same; what
+// both sides need (speeds, star densities, transverse star fields and velocities)
+// stays as it is, and the HLL and HLLC fallbacks are branches that whole wavefronts
+// skip.  A wavefront with faces of both kinds no longer runs both sides, and the
+// two states and fluxes are not live together.  256^3, us a launch: x sweep 643 ->
+// 573, y sweep 760 -> 699 (the z sweep, 834, moves its bytes at the copy rate).
+// FP32 keeps the form above: its bits depend on what the compiler contracts.
+template <int N>
+GPL_HD void mhd_hlld_side(const double *vl, const double *vr, double gamma, FaceFlux<double> &out)
+{
+  constexpr int VXn = 1 + N, VXt = 1 + (N + 1)%3, VXb = 1 + (N + 2)%3;
+  constexpr int BXn = 4 + N, BXt = 4 + (N + 1)%3, BXb = 4 + (N + 2)%3;
+  constexpr int ENG = 7;
+  const double gmm1 = gamma - 1.0;
+  double sl_min, sl_max, sr_min, sr_max;
+  mhd_max_signal_speed<double, N>(vl, gamma, sl_min, sl_max);    // HLL_Speed, mhd.hpp:296
+  mhd_max_signal_speed<double, N>(vr, gamma, sr_min, sr_max);
+  const double Sl = rmin(sl_min, sr_min);
+  const double Sr = rmax(sl_max, sr_max);
+  out.Sl = Sl; out.Sr = Sr;
+  const double ptl = vl[7] + 0.5*(vl[4]*vl[4] + vl[5]*vl[5] + vl[6]*vl[6]);
+  const double ptr = vr[7] + 0.5*(vr[4]*vr[4] + vr[5]*vr[5] + vr[6]*vr[6]);
+  const double rdS = 1.0/(Sr - Sl);
+  const double Bx = (Sr*vr[BXn] - Sl*vl[BXn])*rdS;
+  const double sBx = Bx > 0.0 ? 1.0 : -1.0;
+  const double dul = Sl - vl[VXn], dur = Sr - vr[VXn];
+  double SM, pts;
+  {
+    const double scrh = 1.0/(dur*vr[0] - dul*vl[0]);
+    SM = (dur*(vr[0]*vr[VXn]) - dul*(vl[0]*vl[VXn]) - ptr + ptl)*scrh;
+    pts =   dur*vr[0]*ptl - dul*vl[0]*ptr
+          + vl[0]*vr[0]*dur*dul*(vr[VXn] - vl[VXn]);
+    pts *= scrh;
+  }
+  const double rsl = vl[0]*dul/(Sl - SM), rsr = vr[0]*dur/(Sr - SM);   // star densities
+  const double sqrL = sqrt(rsl), sqrR = sqrt(rsr);
+  double S1L = SM - rabs(Bx)/sqrL;
+  double S1R = SM + rabs(Bx)/sqrR;
+  const bool outL = Sl >= 0.0, outR = !outL && Sr <= 0.0;
+  const bool hll = !outL && !outR && (rsl < 0.0 || rsr < 0.0);
+  const bool fan = !outL && !outR && !hll;
+  // transverse fields of the star states
+  double btL, bbL, btR, bbR;
+  {
+    const double kL = (vl[0]*dul*dul - Bx*Bx)/(vl[0]*dul*(Sl - SM) - Bx*Bx);
+    const double kR = (vr[0]*dur*dur - Bx*Bx)/(vr[0]*dur*(Sr - SM) - Bx*Bx);
+    btL = vl[BXt]*kL; bbL = vl[BXb]*kL;
+    btR = vr[BXt]*kR; bbR = vr[BXb]*kR;
+  }
+  if (fan && (((S1L - Sl) < 1.e-4*(SM - Sl)) || ((S1R - Sr) > -1.e-4*(Sr - SM)))) {
+    // HLLC: the transverse fields of the HLL average
+    const double ftl = vl[BXt]*vl[VXn] - vl[BXn]*vl[VXt], fbl = vl[BXb]*vl[VXn] - vl[BXn]*vl[VXb];
+    const double ftr = vr[BXt]*vr[VXn] - vr[BXn]*vr[VXt], fbr = vr[BXb]*vr[VXn] - vr[BXn]*vr[VXb];
+    double ut = Sr*vr[BXt] - Sl*vl[BXt] + ftl - ftr;  ut *= rdS;
+    double ub = Sr*vr[BXb] - Sl*vl[BXb] + fbl - fbr;  ub *= rdS;
+    btL = btR = ut;
+    bbL = bbR = ub;
+    S1L = S1R = SM;
+  }
+  double vsL, vsR, wsL, wsR;
+  {
+    const double mL = Bx/(vl[0]*dul), mR = Bx/(vr[0]*dur);
+    vsL = vl[VXt] - mL*(btL - vl[BXt]);
+    vsR = vr[VXt] - mR*(btR - vr[BXt]);
+    wsL = vl[VXb] - mL*(bbL - vl[BXb]);
+    wsR = vr[VXb] - mR*(bbR - vr[BXb]);
+  }
+  // the decision tree: inL / inR are the single-star regions
+  const bool inL = S1L >= 0.0, inR = !inL && S1R <= 0.0;
+  const bool left = outL || (!outR && (inL || (!inR && SM >= 0.0)));
+  const bool two = fan && !inL && !inR;
+  // transverse velocity and field of the double-star states, common to both sides
+  double vss = 0.0, wss = 0.0, btt = 0.0, bbb = 0.0;
+  if (two) {
+    const double q = sqrL + sqrR;
+    vss = sqrL*vsL + sqrR*vsR + (btR - btL)*sBx;
+    vss /= q;
+    wss = sqrL*wsL + sqrR*wsR + (bbR - bbL)*sBx;
+    wss /= q;
+    btt = sqrL*btR + sqrR*btL + sqrL*sqrR*(vsR - vsL)*sBx;
+    btt /= q;
+    bbb = sqrL*bbR + sqrR*bbL + sqrL*sqrR*(wsR - wsL)*sBx;
+    bbb /= q;
+  }
+  // the side that is taken
+  double v[8], u[8], f[8], pt;
+  for (int nv = 0; nv < 8; nv++) v[nv] = left ? vl[nv] : vr[nv];
+  mhd_prim_to_cons(v, u, gmm1);
+  mhd_flux<double, N>(v, u, f, pt);
+  double *flux = out.f;
+  for (int nv = 0; nv < 8; nv++) flux[nv] = f[nv];
+  if (fan) {
+    const double S = left ? Sl : Sr, d = left ? dul : dur, S1 = left ? S1L : S1R;
+    const double sq = left ? sqrL : sqrR;
+    const double vs = left ? vsL : vsR, ws = left ? wsL : wsR, bt = left ? btL : btR, bb = left ? bbL : bbR;
+    double us[8], uss[8];
+    us[0] = left ? rsl : rsr;
+    us[VXn] = us[0]*SM;
+    us[VXt] = us[0]*vs;
+    us[VXb] = us[0]*ws;
+    us[BXn] = Bx;
+    us[BXt] = bt;
+    us[BXb] = bb;
+    double scrh  = v[VXn]*Bx + v[VXt]*u[BXt] + v[VXb]*u[BXb];
+    scrh -= SM*Bx + vs*bt + ws*bb;
+    us[ENG]  = d*u[ENG] - pt*v[VXn] + pts*SM + Bx*scrh;
+    us[ENG] /= S - SM;
+    if (two) {
+      uss[0] = us[0];
+      uss[VXn] = uss[0]*SM;
+      uss[VXt] = uss[0]*vss;
+      uss[VXb] = uss[0]*wss;
+      uss[BXn] = Bx;
+      uss[BXt] = btt;
+      uss[BXb] = bbb;
+      double e2 = SM*Bx + vs*bt + ws*bb;
+      e2 -= SM*Bx + vss*btt + wss*bbb;
+      // left: E* - sqrL e sBx, right: E* + sqrR e sBx
+      const double c = sq*e2*sBx;
+      uss[ENG] = left ? us[ENG] - c : us[ENG] + c;
+      for (int nv = 0; nv < 8; nv++) flux[nv] = flux[nv] + S1*(uss[nv] - us[nv]);
+    }
+    for (int nv = 0; nv < 8; nv++) flux[nv] = flux[nv] + S*(us[nv] - u[nv]);
+  } else if (hll) {
+    double ul[8], ur[8], fl[8], fr[8], p;
+    mhd_prim_to_cons(vl, ul, gmm1);
+    mhd_prim_to_cons(vr, ur, gmm1);
+    mhd_flux<double, N>(vl, ul, fl, p);
+    mhd_flux<double, N>(vr, ur, fr, p);
+    for (int nv = 0; nv < 8; nv++) {
+      flux[nv]  = Sl*Sr*(ur[nv] - ul[nv]) + Sr*fl[nv] - Sl*fr[nv];
+      flux[nv] *= rdS;
+    }
+  }
+  const bool nan = __builtin_isunordered(flux[0], flux[1]) | __builtin_isunordered(flux[2], flux[3]) |
+                   __builtin_isunordered(flux[4], flux[5]) | __builtin_isunordered(flux[6], flux[7]);
+  out.err = nan ? ERR_NAN | ERR_QUIT : 0u;
+}
+
+template <typename R, int N>
+GPL_HD void mhd_hlld(const R *vl, const R *vr, R gamma, FaceFlux<R> &out)
+{
+  if constexpr (sizeof(R) == sizeof(double)) mhd_hlld_side<N>(vl, vr, gamma, out);
+  else mhd_hlld_both<R, N>(vl, vr, gamma, out);
 }
 
 // HLL with Davis speeds (Src/MHD/hll.cpp; formula as Src/MHD/hlld.cpp:452-461)
