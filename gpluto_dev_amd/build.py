@@ -50,6 +50,7 @@ SOURCES = [("mhd3d_fp64.hip", MFMA_VGPR),
            ("engine_mhd3d.cpp", []),
            ("engine_hd.cpp", []),
            ("dbl_io.cpp", []),
+           ("host_copy.cpp", []),
            ("gpl_api.cpp", [])]
 
 

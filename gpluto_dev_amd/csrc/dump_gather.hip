@@ -1,7 +1,9 @@
-// The dbl dump image of a 3D MHD/RMHD box, gathered on the device in the
+// The active zones of one variable for a download (launch_field_gather), and
+// the dbl dump image of a 3D MHD/RMHD box, gathered on the device in the
 // file's own order (Src/write_data.cpp:136-159 with FillOutputBuffer
 // :564-607): the eight primitives over the active zones, i fastest, then
 // Bx1s, Bx2s, Bx3s with nx+1, ny+1, nz+1 faces along their direction.
+#include "host_copy.hpp"
 #include "mhd3d.hpp"
 
 namespace gpl {
@@ -61,5 +63,29 @@ template void mhd3d_dump_gather<double>(const Box3 &, const int *, const int *, 
                                         const double *, double *, hipStream_t);
 template void mhd3d_dump_gather<float>(const Box3 &, const int *, const int *, const float *,
                                        const double *, double *, hipStream_t);
+
+namespace {
+
+template <typename R>
+__global__ __launch_bounds__(256)
+void k_field_gather(FieldGeom g, const R *__restrict__ src, size_t e0, size_t count, double *__restrict__ dst)
+{
+  const size_t t = (size_t)blockIdx.x*blockDim.x + threadIdx.x;
+  if (t >= count) return;
+  const size_t e = e0 + t, r = e / g.n[0];
+  const int i = (int)(e - r*g.n[0]), k = (int)(r / g.n[1]), j = (int)(r - (size_t)k*g.n[1]);
+  dst[t] = (double)src[g.off + (size_t)(i + g.lo[0]) +
+                       (size_t)g.sx*((size_t)(j + g.lo[1]) + (size_t)g.sy*(k + g.lo[2]))];
+}
+
+}  // namespace
+
+void launch_field_gather(const FieldGeom &g, const void *src, bool f32, size_t e0, size_t count,
+                         double *dst, hipStream_t s)
+{
+  const dim3 nb((unsigned)((count + 255)/256));
+  if (f32) hipLaunchKernelGGL((k_field_gather<float>), nb, dim3(256), 0, s, g, (const float *)src, e0, count, dst);
+  else     hipLaunchKernelGGL((k_field_gather<double>), nb, dim3(256), 0, s, g, (const double *)src, e0, count, dst);
+}
 
 }  // namespace gpl

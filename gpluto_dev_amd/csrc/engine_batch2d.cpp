@@ -11,6 +11,7 @@
 #include "batch2d.hpp"
 #include "diagnostics.hpp"
 #include "engine.hpp"
+#include "host_copy.hpp"
 #include "physics.hpp"
 
 #include <hip/hip_runtime.h>
@@ -101,6 +102,7 @@ struct gpl_batch {
   int graph_shape = -1;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   double last_run_ms = 0.0;
+  HostCopy copy;        // downloads in the active layout
 };
 
 static void batch_free(gpl_batch *b)
@@ -444,6 +446,25 @@ static int gpl_batch_download_impl(gpl_batch *b, int box, double *vc, double *co
   const int NX = d.nx, NY = d.ny;
   const size_t m = (size_t)NX*NY, nc = (size_t)b->ncell;
   const size_t rs = b->fp64 ? sizeof(double) : sizeof(float);
+  if (!L.ary) {
+    const FieldGeom fg = {(size_t)d.off, NX, NY, {d.lo[0], d.lo[1], 0}, {L.nx, L.ny, 1}, !b->padded};
+    const size_t na = (size_t)L.nx*L.ny;
+    auto prim = [&](int q) { return (const void *)((const char *)b->V + q*nc*rs); };
+    std::vector<FieldOut> out;
+    if (vc) for (int q = 0; q < 8; q++) out.push_back({prim(q), !b->fp64, vc + q*na});
+    if (vs) for (int c = 0; c < 2; c++) if (vs[c]) out.push_back({b->vs[b->cur] + c*nc, false, vs[c]});
+    // B1, B2 of Uc are the face averages (= Vc's)
+    const int map[8] = {0, 1, 2, 3, -1, -1, 4, 5};
+    if (uc)
+      for (int q = 0; q < 8; q++) {
+        if (map[q] >= 0) out.push_back({b->U + map[q]*nc, false, uc + q*na});
+        else             out.push_back({prim(q), !b->fp64, uc + q*na});
+      }
+    const size_t had = b->copy.device_bytes();
+    const int rc = b->copy.fetch(fg, out, b->stream);
+    b->bytes += b->copy.device_bytes() - had;
+    return rc;
+  }
   std::vector<double> hv(8*m), hu(6*m), hs(2*m);
   for (int s = 0; s < 8; s++) {
     const char *src = (const char *)b->V + (s*nc + d.off)*rs;
@@ -747,7 +768,10 @@ public:
   }
   int download(double *vc, double *const *vs, double *uc, int layout) override
   {
-    return gpl_batch_download_impl(b, 0, vc, vs, uc, layout);
+    const size_t had = b->bytes;
+    const int rc = gpl_batch_download_impl(b, 0, vc, vs, uc, layout);
+    bytes += b->bytes - had;
+    return rc;
   }
   void enqueue_step(int advance_dt, LaunchTimer *) override { ::enqueue_step(b, advance_dt); }
   int graph_period() const override { return ::graph_period(b); }

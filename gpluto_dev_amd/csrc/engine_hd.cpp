@@ -96,6 +96,13 @@ public:
   int download(double *vc, double *const *, double *uc, int layout) override
   {
     const Layout L = make_layout(cfg, layout);
+    if (!L.ary) {
+      const FieldGeom fg = {0, L.nx, L.ny, {0, 0, 0}, {L.nx, L.ny, L.nz}, true};
+      std::vector<FieldOut> out;
+      if (vc) for (int q = 0; q < 5; q++) out.push_back({cur_v + q*n, false, vc + q*n});
+      if (uc) for (int q = 0; q < 5; q++) out.push_back({cur_u + q*n, false, uc + q*n});
+      return fetch(fg, out, env.stream);
+    }
     for (int which = 0; which < 2; which++) {
       double *dst = which == 0 ? vc : uc;
       if (!dst) continue;

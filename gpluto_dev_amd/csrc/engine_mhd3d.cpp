@@ -322,6 +322,23 @@ public:
   {
     const Layout L = make_layout(cfg, layout);
     const int nx = L.nx, ny = L.ny, nz = L.nz;
+    if (!L.ary) {
+      const FieldGeom fg = {0, g.nx, g.ny, {g.lo[0], g.lo[1], g.lo[2]}, {nx, ny, nz}, !padded};
+      const size_t na3 = (size_t)nx*ny*nz, rs = fp64 ? sizeof(double) : sizeof(float);
+      auto prim = [&](int q) { return (const void *)((const char *)V + q*n*rs); };
+      std::vector<FieldOut> out;
+      if (vc) for (int q = 0; q < 8; q++) out.push_back({prim(q), !fp64, vc + q*na3});
+      if (vsh)
+        for (int d = 0; d < 3; d++) if (vsh[d]) out.push_back({vs[cur] + d*n, false, vsh[d]});
+      // the cell-centred field of Uc is the face average (= Vc's B1..3)
+      const int map[8] = {0, 1, 2, 3, -1, -1, -1, 4};
+      if (uc)
+        for (int q = 0; q < 8; q++) {
+          if (map[q] >= 0) out.push_back({U + map[q]*n, false, uc + q*na3});
+          else             out.push_back({prim(q), !fp64, uc + q*na3});
+        }
+      return fetch(fg, out, env.stream);
+    }
     std::vector<double> hv(8*n);
     if ((vc || uc) && from_device_v(V, fp64, hv)) return GPL_EHIP;
     if (vc) {

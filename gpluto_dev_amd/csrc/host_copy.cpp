@@ -1,0 +1,206 @@
+// Device-to-host transfer of state arrays: see host_copy.hpp.
+#include "host_copy.hpp"
+#include "../../include/gpluto_amd.h"
+
+#include <atomic>
+#include <condition_variable>
+#include <cstring>
+#include <mutex>
+#include <thread>
+
+namespace gpl {
+
+namespace {
+
+// Moves chunks from pinned memory to the caller's arrays: the calling thread and
+// up to kHelpers more, each taking pieces of the chunk on offer.  Helpers that
+// cannot be started are simply missing.
+class Movers {
+public:
+  explicit Movers(size_t total)
+  {
+    // a helper pays for itself from some megabytes on
+    const int want = total >= (size_t(32) << 20) ? kHelpers : (total >= (size_t(4) << 20) ? 2 : 0);
+    try {
+      helpers.reserve(want);
+      for (int q = 0; q < want; q++) helpers.emplace_back([this] { serve(); });
+    } catch (...) {
+    }
+  }
+  ~Movers()
+  {
+    {
+      std::lock_guard<std::mutex> l(m);
+      quit = true;
+    }
+    cv.notify_all();
+    for (auto &t : helpers) t.join();
+  }
+  void move(void *dst, const void *src, size_t bytes)
+  {
+    if (helpers.empty()) { memcpy(dst, src, bytes); return; }
+    {
+      std::lock_guard<std::mutex> l(m);
+      to = (char *)dst; from = (const char *)src; size = bytes;
+      next.store(0);
+      busy = (int)helpers.size();
+      round++;
+    }
+    cv.notify_all();
+    work();
+    std::unique_lock<std::mutex> l(m);
+    idle.wait(l, [this] { return busy == 0; });
+  }
+
+private:
+  static constexpr int kHelpers = 7;
+  static constexpr size_t kPiece = size_t(1) << 20;
+  void work()
+  {
+    for (;;) {
+      const size_t o = next.fetch_add(kPiece);
+      if (o >= size) return;
+      memcpy(to + o, from + o, size - o < kPiece ? size - o : kPiece);
+    }
+  }
+  void serve()
+  {
+    unsigned long seen = 0;
+    std::unique_lock<std::mutex> l(m);
+    for (;;) {
+      cv.wait(l, [&] { return quit || round != seen; });
+      if (quit) return;
+      seen = round;
+      l.unlock();
+      work();
+      l.lock();
+      if (--busy == 0) idle.notify_one();
+    }
+  }
+  std::vector<std::thread> helpers;
+  std::mutex m;
+  std::condition_variable cv, idle;
+  std::atomic<size_t> next{0};
+  char *to = nullptr;
+  const char *from = nullptr;
+  size_t size = 0;
+  unsigned long round = 0;
+  int busy = 0;
+  bool quit = false;
+};
+
+// part of a run of fields that are adjacent on both sides
+struct Piece {
+  const void *src;
+  bool f32;
+  size_t e0, count;  // elements of the field
+  double *dst;
+  size_t at;         // offset in its slot, doubles
+};
+
+}  // namespace
+
+HostCopy::~HostCopy()
+{
+  if (pin) (void)hipHostFree(pin);
+  if (dev) (void)hipFree(dev);
+  for (hipEvent_t e : done) if (e) (void)hipEventDestroy(e);
+}
+
+int HostCopy::reserve(size_t slot, bool gather)
+{
+  const size_t want = kSlots*slot*sizeof(double);
+  for (int q = 0; q < kSlots; q++)
+    if (!done[q] && hipEventCreateWithFlags(&done[q], hipEventDisableTiming) != hipSuccess) return GPL_EHIP;
+  if (pin_cap < want) {
+    if (pin) (void)hipHostFree(pin);
+    pin = nullptr;
+    pin_cap = 0;
+    if (hipHostMalloc((void **)&pin, want, hipHostMallocDefault) != hipSuccess) { pin = nullptr; return GPL_ENOMEM; }
+    pin_cap = want;
+  }
+  if (gather && dev_cap < want) {
+    if (dev) (void)hipFree(dev);
+    dev = nullptr;
+    dev_cap = 0;
+    if (hipMalloc((void **)&dev, want) != hipSuccess) { dev = nullptr; return GPL_ENOMEM; }
+    dev_cap = want;
+  }
+  return 0;
+}
+
+int HostCopy::fetch(const FieldGeom &g, const std::vector<FieldOut> &out, hipStream_t s)
+{
+  const size_t n = (size_t)g.n[0]*g.n[1]*g.n[2], total = n*out.size();
+  if (!total) return 0;
+  bool gather = !g.whole;
+  for (const FieldOut &f : out) gather = gather || f.f32;
+  // a small state goes through all slots at once, with one wait, a larger one in
+  // slots of an eighth of it, 16 MiB at most
+  const bool once = total <= (size_t(1) << 17);
+  if (once && !gather) {
+    // up to a megabyte the runtime's own staging is as fast and needs no buffer
+    for (size_t q = 0; q < out.size();) {
+      size_t run = 1;                          // fields that follow one another on both sides
+      while (q + run < out.size() && out[q + run].dst == out[q].dst + run*n &&
+             (const double *)out[q + run].src == (const double *)out[q].src + run*n)
+        run++;
+      if (hipMemcpyAsync(out[q].dst, (const double *)out[q].src + g.off, run*n*sizeof(double),
+                         hipMemcpyDeviceToHost, s) != hipSuccess)
+        return GPL_EHIP;
+      q += run;
+    }
+    return hipStreamSynchronize(s) == hipSuccess ? 0 : GPL_EHIP;
+  }
+  size_t slot = once ? (total + kSlots - 1)/kSlots : (total + 7)/8;
+  if (slot > kChunk) slot = kChunk;
+  if (int rc = reserve(slot, gather)) return rc;
+  const size_t hold = once ? slot*kSlots : slot;   // doubles of a group
+  // groups of pieces, one group per slot; without a gather, fields that follow
+  // one another on both sides make one piece
+  std::vector<std::vector<Piece>> groups;
+  size_t used = hold;
+  for (const FieldOut &f : out)
+    for (size_t e = 0; e < n;) {
+      if (used == hold) { groups.emplace_back(); used = 0; }
+      const size_t c = n - e < hold - used ? n - e : hold - used;
+      Piece *last = groups.back().empty() ? nullptr : &groups.back().back();
+      if (last && last->dst + last->count == f.dst + e &&
+          (gather ? false : (const double *)last->src + last->e0 + last->count == (const double *)f.src + e))
+        last->count += c;
+      else
+        groups.back().push_back({f.src, f.f32, e, c, f.dst + e, used});
+      e += c;
+      used += c;
+    }
+  const int ng = (int)groups.size();
+  Movers movers(total*sizeof(double));
+  auto send = [&](int k) -> bool {
+    double *hp = pin + (size_t)(k % kSlots)*slot, *dp = dev + (size_t)(k % kSlots)*slot;
+    size_t sum = 0;
+    for (const Piece &p : groups[k]) {
+      if (gather) launch_field_gather(g, p.src, p.f32, p.e0, p.count, dp + p.at, s);
+      else if (hipMemcpyAsync(hp + p.at, (const double *)p.src + g.off + p.e0, p.count*sizeof(double),
+                              hipMemcpyDeviceToHost, s) != hipSuccess)
+        return false;
+      sum += p.count;
+    }
+    if (gather && (hipGetLastError() != hipSuccess ||
+                   hipMemcpyAsync(hp, dp, sum*sizeof(double), hipMemcpyDeviceToHost, s) != hipSuccess))
+      return false;
+    return hipEventRecord(done[k % kSlots], s) == hipSuccess;
+  };
+  bool ok = true;
+  int sent = 0;
+  for (int k = 0; k < ng && ok; k++) {
+    while (ok && sent < ng && sent < k + kSlots) { ok = send(sent); sent++; }
+    ok = ok && hipEventSynchronize(done[k % kSlots]) == hipSuccess;
+    if (!ok) break;
+    const double *hp = pin + (size_t)(k % kSlots)*slot;
+    for (const Piece &p : groups[k]) movers.move(p.dst, hp + p.at, p.count*sizeof(double));
+  }
+  if (!ok) (void)hipStreamSynchronize(s);     // nothing is in flight into the buffers afterwards
+  return ok ? 0 : GPL_EHIP;
+}
+
+}  // namespace gpl

@@ -1,0 +1,58 @@
+// Device-to-host transfer of state arrays into a caller's (pageable) arrays.
+//
+// A field is one variable over the active zones, i fastest.  Fields are cut into
+// chunks; a chunk is copied into one of kSlots pinned buffers (through a device
+// buffer that a gather kernel fills where the stored array is FP32 or holds
+// ghost layers), and while later chunks are on their way, helper threads move it
+// to the caller's array.  256^3, the eleven arrays of Vc and Vs (1.48 GB): 422
+// ms with pageable copies into host vectors and element loops, 27.6 this way (a
+// pinned copy alone is 26); 128^3 55 -> 3.7, 192^3 mixed 222 -> 12.4.
+//
+// The buffers belong to one context (no sharing between contexts or threads),
+// are allocated at its first transfer, at most kSlots chunks of 16 MiB pinned and,
+// if a gather is needed, as much on the device, and are freed with it.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+#include <vector>
+
+namespace gpl {
+
+// Where the active zones lie in a stored array: element (i, j, k) at
+// off + (i + lo[0]) + sx*((j + lo[1]) + sy*(k + lo[2])).
+struct FieldGeom {
+  size_t off;
+  int sx, sy;
+  int lo[3], n[3];
+  bool whole;        // the array is the active zones and nothing else
+};
+
+struct FieldOut {
+  const void *src;   // device array, at element 0 of the box's storage (before off)
+  bool f32;          // float, else double
+  double *dst;       // host array of n[0]*n[1]*n[2] doubles
+};
+
+class HostCopy {
+public:
+  ~HostCopy();
+  // Every field of `out` to the host, behind the work already on the stream;
+  // returns when the arrays are filled.  0, GPL_ENOMEM or GPL_EHIP.
+  int fetch(const FieldGeom &g, const std::vector<FieldOut> &out, hipStream_t s);
+  size_t device_bytes() const { return dev_cap; }
+
+private:
+  static constexpr int kSlots = 4;
+  static constexpr size_t kChunk = size_t(1) << 21;   // doubles per slot at most: 16 MiB
+  int reserve(size_t chunk, bool gather);
+  double *pin = nullptr, *dev = nullptr;
+  size_t pin_cap = 0, dev_cap = 0;                     // bytes
+  hipEvent_t done[kSlots] = {};
+};
+
+// dst[t] = element e0 + t of the field, in FP64
+void launch_field_gather(const FieldGeom &g, const void *src, bool f32, size_t e0, size_t count,
+                         double *dst, hipStream_t s);
+
+}  // namespace gpl
