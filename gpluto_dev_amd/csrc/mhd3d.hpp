@@ -61,6 +61,11 @@ void mhd3d_launch(int which, const Mhd3dBufs<R> &b, const Box3 &g, const StepCtl
                   int first_stage, int want_dt, int limiter, int solver, double gamma,
                   double small_rho, double small_prs, hipStream_t s);
 
+// mhd3d_launch<double>'s RMHD and van Leer sweeps and EMFs, built without loop
+// hoisting of constants (mhd3d_fp64_nohoist.hip)
+void mhd3d_launch_nohoist(int which, const Mhd3dBufs<double> &b, const Box3 &g, const StepCtl *ctl, RKW w,
+                          int first_stage, int want_dt, int limiter, int solver, double gamma, hipStream_t s);
+
 // Ghost-zone fill of a padded box (non-periodic sides), side by side;
 // type[s] = GPL_PERIODIC, GPL_OUTFLOW or GPL_REFLECTIVE for X1-beg, ..., X3-end.
 // dbl dump image of the box (active cells, faces 0..n along each direction;

@@ -1201,14 +1201,75 @@ static inline int emf_flat(int nx) { return ((nx + 63)/64)*64*4 > 5*nx; }
 // Host-side launch helpers: one entry per kernel family, so that the host
 // orchestration can bracket each launch with timing events.
 // ---------------------------------------------------------------------------
+// The fused sweeps: x, and the y and z marches.
 template <typename R, int LIM, int SOLVER, int PH>
-static void launch_t(int which, const Mhd3dBufs<R> &b, const Box3 &g, const StepCtl *ctl, RKW w,
-                     int first_stage, int want_dt, double gamma, double small_rho,
-                     double small_prs, hipStream_t s)
+static void launch_sweep(int which, const Mhd3dBufs<R> &b, const Box3 &g, const StepCtl *ctl, RKW w,
+                         int first_stage, int want_dt, double gamma, hipStream_t s)
+{
+  const int T = 256;
+  const int nk = g.ke - g.kb;          // planes of the launch
+  if (which == K_SWEEPX_F) {
+    const size_t shm = 14*(size_t)g.nx*sizeof(R);
+    hipLaunchKernelGGL((k_sweepx_fused<R, LIM, SOLVER, PH>), dim3(g.ny*nk), dim3(g.nx), shm, s,
+                       g, b.V, b.Vin, b.FD, b.dU, b.Cdt, ctl, (R)gamma, want_dt, b.err);
+  } else if (which == K_SWEEPY_F) {
+    const int L = b.march[0], nt = g.nx*nk*((g.ny + L - 1)/L);
+    hipLaunchKernelGGL((k_sweep_march<R, 1, LIM, SOLVER, PH>), dim3((nt + T - 1)/T), dim3(T), 0, s,
+                       g, L, b.V, b.Vin, b.FD, b.dU, b.Cdt, b.Uin, b.U, b.U0, ctl, w, first_stage, want_dt,
+                       b.cdt_part, (R)gamma, b.err);
+  } else {
+    const int L = b.march[1], nt = g.nx*g.ny*((nk + L - 1)/L);
+    hipLaunchKernelGGL((k_sweep_march<R, 2, LIM, SOLVER, PH>), dim3((nt + T - 1)/T), dim3(T), 0, s,
+                       g, L, b.V, b.Vin, b.FD, b.dU, b.Cdt, b.Uin, b.U, b.U0, ctl, w, first_stage, want_dt,
+                       b.cdt_part, (R)gamma, b.err);
+  }
+}
+
+template <typename R, int LIM>
+static void launch_emf(const Mhd3dBufs<R> &b, const Box3 &g, int solver, hipStream_t s)
+{
+  const int nk = g.ke - g.kb;
+  const int flat = emf_flat(g.nx);
+  const dim3 ge = flat ? dim3((g.nx*g.ny + 255)/256, 1, g.nz) : dim3((g.nx + 63)/64, (g.ny + 3)/4, g.nz);
+  if (solver == 4) {                   // UCT_HLLD: six records per face, one edge per thread
+    hipLaunchKernelGGL((k_emf_edge<R, LIM, 4>), ge, dim3(256), 0, s, g, flat, b.Vin, b.FD, b.E);
+  } else if (b.emf_march == 0) {
+    hipLaunchKernelGGL((k_emf_edge<R, LIM>), ge, dim3(256), 0, s, g, flat, b.Vin, b.FD, b.E);
+  } else {
+    const int l = b.emf_march < 0 ? -b.emf_march : b.emf_march;
+    const int nt = ((g.nx + 63)/64)*((g.ny + 3)/4)*((nk + l - 1)/l);
+    if (b.emf_march < 0)               // LDS-staged tiles
+      hipLaunchKernelGGL((k_emf_tile<R, LIM>), dim3(nt), dim3(256), 0, s, g, l, b.Vin, b.FD, b.E);
+    else                               // register march
+      hipLaunchKernelGGL((k_emf_march<R, LIM>), dim3(nt), dim3(256), 0, s, g, l, b.Vin, b.FD, b.E);
+  }
+}
+
+template <typename R, int PH>
+static void launch_finish(const Mhd3dBufs<R> &b, const Box3 &g, const StepCtl *ctl, RKW w,
+                          int first_stage, double gamma, double small_rho, double small_prs, hipStream_t s)
+{
+  const int T = 256;
+  const dim3 nb(((g.ke - g.kb)*g.nx*g.ny + T - 1)/T);
+  // the RMHD mapper takes gamma, the MHD one gamma - 1
+  if (PH == 1 && b.net)
+    hipLaunchKernelGGL((k_finish<R, PH, PH == 1>), nb, dim3(T), 0, s,
+                       g, b.E, b.Vin, b.Vout, b.Bs0, b.U, b.V, ctl, w, first_stage, gamma,
+                       small_rho, small_prs, b.err, b.net, b.zr);
+  else
+    hipLaunchKernelGGL((k_finish<R, PH, false>), nb, dim3(T), 0, s,
+                       g, b.E, b.Vin, b.Vout, b.Bs0, b.U, b.V, ctl, w, first_stage,
+                       PH == 1 ? gamma : gamma - 1.0, small_rho, small_prs, b.err, nullptr, b.zr);
+}
+
+// The unfused kernels and the fused x+y march: ideal MHD (the RMHD x+y kernel
+// would hold more registers than a wavefront has; the engine never selects it).
+template <typename R, int LIM, int SOLVER>
+static void launch_mhd(int which, const Mhd3dBufs<R> &b, const Box3 &g, const StepCtl *ctl, RKW w,
+                       int first_stage, int want_dt, double gamma, hipStream_t s)
 {
   const int T = 256;
   const int nb = (g.ncell + T - 1)/T;
-  const int nk = g.ke - g.kb;          // planes of the fused kernels' launch
   switch (which) {
   case K_SWEEP_X:
     hipLaunchKernelGGL((k_sweep<R, 0, LIM, SOLVER>), dim3(nb), dim3(T), 0, s,
@@ -1227,104 +1288,65 @@ static void launch_t(int which, const Mhd3dBufs<R> &b, const Box3 &g, const Step
                        g, b.F, b.CM, b.Uin, b.U, b.U0, ctl, w, first_stage,
                        want_dt ? b.cdt_part : nullptr);
     break;
-  case K_SWEEPX_F: {
-    const size_t shm = 14*(size_t)g.nx*sizeof(R);
-    hipLaunchKernelGGL((k_sweepx_fused<R, LIM, SOLVER, PH>), dim3(g.ny*nk), dim3(g.nx), shm, s,
-                       g, b.V, b.Vin, b.FD, b.dU, b.Cdt, ctl, (R)gamma, want_dt, b.err);
-    break;
-  }
   case K_SWEEPXY_F: {
-    // ideal MHD only: the RMHD x+y kernel would hold more registers than a
-    // wavefront has (the engine never selects it for RMHD)
-    if constexpr (PH == 0) {
-      const size_t shm = 20*(size_t)g.nx*sizeof(R);
-      const int L = b.march[0], nb = g.nz*((g.ny + L - 1)/L);
-      hipLaunchKernelGGL((k_sweep_xy<R, LIM, SOLVER, PH>), dim3(nb), dim3(g.nx), shm, s,
-                         g, L, b.V, b.Vin, b.FD, b.dU, b.Cdt, ctl, (R)gamma, want_dt, b.err);
-    }
+    const size_t shm = 20*(size_t)g.nx*sizeof(R);
+    const int L = b.march[0], nl = g.nz*((g.ny + L - 1)/L);
+    hipLaunchKernelGGL((k_sweep_xy<R, LIM, SOLVER, 0>), dim3(nl), dim3(g.nx), shm, s,
+                       g, L, b.V, b.Vin, b.FD, b.dU, b.Cdt, ctl, (R)gamma, want_dt, b.err);
     break;
   }
-  case K_SWEEPY_F: {
-    const int L = b.march[0], nt = g.nx*nk*((g.ny + L - 1)/L);
-    hipLaunchKernelGGL((k_sweep_march<R, 1, LIM, SOLVER, PH>), dim3((nt + T - 1)/T), dim3(T), 0, s,
-                       g, L, b.V, b.Vin, b.FD, b.dU, b.Cdt, b.Uin, b.U, b.U0, ctl, w, first_stage, want_dt,
-                       b.cdt_part, (R)gamma, b.err);
-    break;
-  }
-  case K_SWEEPZ_F: {
-    const int L = b.march[1], nt = g.nx*g.ny*((nk + L - 1)/L);
-    hipLaunchKernelGGL((k_sweep_march<R, 2, LIM, SOLVER, PH>), dim3((nt + T - 1)/T), dim3(T), 0, s,
-                       g, L, b.V, b.Vin, b.FD, b.dU, b.Cdt, b.Uin, b.U, b.U0, ctl, w, first_stage, want_dt,
-                       b.cdt_part, (R)gamma, b.err);
-    break;
-  }
-  case K_EMF: {
-    const int flat = emf_flat(g.nx);
-    const dim3 ge = flat ? dim3((g.nx*g.ny + 255)/256, 1, g.nz) : dim3((g.nx + 63)/64, (g.ny + 3)/4, g.nz);
-    if (SOLVER == 4) {                   // UCT_HLLD: six records per face, one edge per thread
-      hipLaunchKernelGGL((k_emf_edge<R, LIM, 4>), ge, dim3(256), 0, s, g, flat, b.Vin, b.FD, b.E);
-    } else if (b.emf_march == 0) {
-      hipLaunchKernelGGL((k_emf_edge<R, LIM>), ge, dim3(256), 0, s, g, flat, b.Vin, b.FD, b.E);
-    } else {
-      const int l = b.emf_march < 0 ? -b.emf_march : b.emf_march;
-      const int nt = ((g.nx + 63)/64)*((g.ny + 3)/4)*((nk + l - 1)/l);
-      if (b.emf_march < 0)               // LDS-staged tiles
-        hipLaunchKernelGGL((k_emf_tile<R, LIM>), dim3(nt), dim3(256), 0, s, g, l, b.Vin, b.FD, b.E);
-      else                               // register march
-        hipLaunchKernelGGL((k_emf_march<R, LIM>), dim3(nt), dim3(256), 0, s, g, l, b.Vin, b.FD, b.E);
-    }
-    break;
-  }
-  case K_FINISH:
-    // the RMHD mapper takes gamma, the MHD one gamma - 1
-    if (PH == 1 && b.net)
-      hipLaunchKernelGGL((k_finish<R, PH, PH == 1>), dim3((nk*g.nx*g.ny + T - 1)/T), dim3(T), 0, s,
-                         g, b.E, b.Vin, b.Vout, b.Bs0, b.U, b.V, ctl, w, first_stage, gamma,
-                         small_rho, small_prs, b.err, b.net, b.zr);
-    else
-      hipLaunchKernelGGL((k_finish<R, PH, false>), dim3((nk*g.nx*g.ny + T - 1)/T), dim3(T), 0, s,
-                         g, b.E, b.Vin, b.Vout, b.Bs0, b.U, b.V, ctl, w, first_stage,
-                         PH == 1 ? gamma : gamma - 1.0, small_rho, small_prs, b.err, nullptr, b.zr);
-    break;
   default:
     break;
   }
 }
 
+// by Riemann solver (4 is HLLD with the UCT_HLLD EMF)
+template <typename R, int LIM, int PH>
+static void launch_sweep_by(int which, const Mhd3dBufs<R> &b, const Box3 &g, const StepCtl *ctl, RKW w,
+                            int first_stage, int want_dt, int solver, double gamma, hipStream_t s)
+{
+  if constexpr (PH == 0)
+    if (solver == 4) return launch_sweep<R, LIM, 4, PH>(which, b, g, ctl, w, first_stage, want_dt, gamma, s);
+  if (solver == 3) return launch_sweep<R, LIM, 3, PH>(which, b, g, ctl, w, first_stage, want_dt, gamma, s);
+  if (solver == 2) return launch_sweep<R, LIM, 2, PH>(which, b, g, ctl, w, first_stage, want_dt, gamma, s);
+  launch_sweep<R, LIM, 1, PH>(which, b, g, ctl, w, first_stage, want_dt, gamma, s);
+}
+template <typename R, int LIM>
+static void launch_mhd_by(int which, const Mhd3dBufs<R> &b, const Box3 &g, const StepCtl *ctl, RKW w,
+                          int first_stage, int want_dt, int solver, double gamma, hipStream_t s)
+{
+  if (solver == 4)      launch_mhd<R, LIM, 4>(which, b, g, ctl, w, first_stage, want_dt, gamma, s);
+  else if (solver == 3) launch_mhd<R, LIM, 3>(which, b, g, ctl, w, first_stage, want_dt, gamma, s);
+  else if (solver == 2) launch_mhd<R, LIM, 2>(which, b, g, ctl, w, first_stage, want_dt, gamma, s);
+  else                  launch_mhd<R, LIM, 1>(which, b, g, ctl, w, first_stage, want_dt, gamma, s);
+}
+
+#if !defined(GPL_MHD3D_NOHOIST)
 template <typename R>
 void mhd3d_launch(int which, const Mhd3dBufs<R> &b, const Box3 &g, const StepCtl *ctl, RKW w,
                   int first_stage, int want_dt, int limiter, int solver, double gamma,
                   double small_rho, double small_prs, hipStream_t s)
 {
-  if constexpr (std::is_same<R, double>::value) {
-    if (b.phys == 1) {            // RMHD: HLL, HLLC or HLLD, FP64 only
-      if (solver == 3) {
-        if (limiter == MC_LIM) launch_t<R, MC_LIM, 3, 1>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
-        else                   launch_t<R, VANLEER_LIM, 3, 1>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
-      } else if (solver == 2) {
-        if (limiter == MC_LIM) launch_t<R, MC_LIM, 2, 1>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
-        else                   launch_t<R, VANLEER_LIM, 2, 1>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
-      } else {
-        if (limiter == MC_LIM) launch_t<R, MC_LIM, 1, 1>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
-        else                   launch_t<R, VANLEER_LIM, 1, 1>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
-      }
-      return;
-    }
+  constexpr bool F64 = std::is_same<R, double>::value;
+  const bool mc = limiter == MC_LIM;
+  if (which == K_FINISH) {
+    if constexpr (F64)
+      if (b.phys == 1) return launch_finish<R, 1>(b, g, ctl, w, first_stage, gamma, small_rho, small_prs, s);
+    return launch_finish<R, 0>(b, g, ctl, w, first_stage, gamma, small_rho, small_prs, s);
   }
-  if (solver == 4) {               // HLLD with the UCT_HLLD EMF
-    if (limiter == MC_LIM) launch_t<R, MC_LIM, 4, 0>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
-    else                   launch_t<R, VANLEER_LIM, 4, 0>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
-    return;
-  }
-  if (limiter == MC_LIM) {
-    if (solver == 3)      launch_t<R, MC_LIM, 3, 0>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
-    else if (solver == 2) launch_t<R, MC_LIM, 2, 0>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
-    else                  launch_t<R, MC_LIM, 1, 0>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
+  const bool sweep = which == K_SWEEPX_F || which == K_SWEEPY_F || which == K_SWEEPZ_F;
+  if constexpr (F64) {
+    if (which == K_EMF || (sweep && (!mc || b.phys == 1)))
+      return mhd3d_launch_nohoist(which, b, g, ctl, w, first_stage, want_dt, limiter, solver, gamma, s);
+    if (sweep) return launch_sweep_by<R, MC_LIM, 0>(which, b, g, ctl, w, first_stage, want_dt, solver, gamma, s);
   } else {
-    if (solver == 3)      launch_t<R, VANLEER_LIM, 3, 0>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
-    else if (solver == 2) launch_t<R, VANLEER_LIM, 2, 0>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
-    else                  launch_t<R, VANLEER_LIM, 1, 0>(which, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
+    if (which == K_EMF) return mc ? launch_emf<R, MC_LIM>(b, g, solver, s) : launch_emf<R, VANLEER_LIM>(b, g, solver, s);
+    if (sweep && mc) return launch_sweep_by<R, MC_LIM, 0>(which, b, g, ctl, w, first_stage, want_dt, solver, gamma, s);
+    if (sweep) return launch_sweep_by<R, VANLEER_LIM, 0>(which, b, g, ctl, w, first_stage, want_dt, solver, gamma, s);
   }
+  if (mc) launch_mhd_by<R, MC_LIM>(which, b, g, ctl, w, first_stage, want_dt, solver, gamma, s);
+  else    launch_mhd_by<R, VANLEER_LIM>(which, b, g, ctl, w, first_stage, want_dt, solver, gamma, s);
 }
+#endif
 
 }  // namespace gpl
