@@ -25,6 +25,13 @@
 //    acos x = 2 phi (x > 0) or pi - 2 phi (x < 0) with sin^2 phi = h =
 //    (1 - |x|)/2 (exact), phi = phi0 - (sin^2 phi0 - h)/sin(2 phi0),
 //    phi0 = acos(|x|)/2, which keeps full relative accuracy as x -> +-1.
+// Both functions try a quick phase first: about 2^-73 in plain doubles with an
+// error bound, and a test whether that decides the rounding.  It nearly always
+// does, so the double-double evaluation is a branch that wavefronts skip.  RMHD
+// HLL at 128^3, us per x, y, z sweep, which solve two quartics per face: 154, 194,
+// 210 with double-double forms and the library's acos as the seed, 132, 169, 186
+// with the quick phase and a seed of 2^-38 (the z sweep 229 where the compiler
+// hoists the constants out of the march: mhd3d_fp64_nohoist.hip).
 // Explicit fma() calls are the error-free products; they are exact on both
 // sides regardless of -ffp-contract.
 #pragma once
@@ -119,11 +126,62 @@ GPL_CR_HD void dd_sincos(double x, dd &s, dd &c)
   c = dd_add(dd_add(C, dd_mul(C, cw)), dd_mul(S, msr));
 }
 
+// The quick phase (Ziv's strategy; Muller, "Elementary Functions", ch. 10): sin
+// and cos of x as unevaluated sums sh + sl and ch + cl with |sl| < 2^-23, in plain
+// double arithmetic with exact products and sums where a rounding would count.
+// With |r| <= 2^-7, the corrections being S cw + C r w for sin x (w = sin r/r - 1,
+// cw = cos r - 1), the largest rounded terms are r w <= 2^-23.6 (relative error of
+// w 2^-51.2: 2^-74.8) and the last addition (2^-76.6): absolute error below 2^-73.5
+// for both; for k = 0 (S = 0, C = 1) sin x = r + r w has relative error below
+// 2^-67.8.
+struct sincos_sum { double sh, sl, ch, cl; int k; };
+GPL_CR_HD sincos_sum quick_sincos(double x)
+{
+  sincos_sum q;
+  q.k = (int)(x*64.0 + 0.5);
+  const double r = x - q.k*0.015625;              // exact
+  const double zh = r*r, zl = fma(r, r, -zh);
+  const double w = zh*fma(zh, fma(zh, fma(zh, 1.0/362880.0, -1.0/5040.0), 1.0/120.0), -1.0/6.0);
+  const double rw = r*w;
+  const double hz = -0.5*zh;                       // cos r - 1 = hz + t
+  const double t = fma(zh*zh, fma(zh, fma(zh, 1.0/40320.0, -1.0/720.0), 1.0/24.0), -0.5*zl);
+  const double *row = table_row(q.k);
+  const double S = row[0], Sl = row[1], C = row[2], Cl = row[3];
+  {
+    const dd p = two_prod(C, r), h = two_prod(S, hz);
+    const dd a = fast_two_sum(S, p.hi);            // S >= |C r|, or S = 0 (k = 0)
+    const dd b = fast_two_sum(a.hi, h.hi);
+    double lo = fma(Sl, hz, fma(Cl, r, Sl));
+    lo = fma(S, t, lo + (p.lo + h.lo)) + (a.lo + b.lo);
+    q.sh = b.hi;
+    q.sl = fma(C, rw, lo);
+  }
+  {
+    const dd p = two_prod(S, -r), h = two_prod(C, hz);
+    const dd a = two_sum(C, p.hi);                 // C passes through 0
+    const dd b = two_sum(a.hi, h.hi);
+    double lo = fma(Cl, hz, fma(Sl, -r, Cl));
+    lo = fma(C, t, lo + (p.lo + h.lo)) + (a.lo + b.lo);
+    q.ch = b.hi;
+    q.cl = fma(-S, rw, lo);
+  }
+  return q;
+}
+constexpr double kE72 = 0x1p-72, kE71 = 0x1p-71, kE66 = 0x1p-66, kE65 = 0x1p-65;
+
 // sin(x) and cos(x) correctly rounded for 0 <= x <= 2.19 (the resolvent
-// cubic's theta lies in [0, pi/3]); other arguments (NaN) take the library's.
+// cubic's theta lies in [0, pi/3]); other arguments (NaN) give NaN.
+// The quick phase decides unless hi + (lo - e) and hi + (lo + e) round apart, e
+// its error bound (about once in 2^14 arguments); then the double-double form.
 GPL_CR_HD void sincos_cr(double x, double *sn, double *cs)
 {
-  if (!(x >= 0.0 && x <= 2.19)) { sincos(x, sn, cs); return; }
+  if (!(x >= 0.0 && x <= 2.19)) { *sn = *cs = __builtin_nan(""); return; }
+  const sincos_sum q = quick_sincos(x);
+  const double es = q.k ? kE72 : q.sh*kE66;
+  const double s1 = q.sh + (q.sl + es), c1 = q.ch + (q.cl + kE72);
+  *sn = s1;
+  *cs = c1;
+  if (s1 == q.sh + (q.sl - es) && c1 == q.ch + (q.cl - kE72)) return;
   dd s, c;
   dd_sincos(x, s, c);
   *sn = s.hi + s.lo;
@@ -165,12 +223,61 @@ GPL_CR_HD double acos_seed(double x)
   return 0.5*t;
 }
 
-// acos(x) correctly rounded for -1 <= x <= 1; NaN takes the library's.
+// A seed for the quick phase, one polynomial for either form: asin(z) = z + z y P(y),
+// y = z^2 <= 1/4, with z = |x| or sqrt((1 - |x|)/2), P the Chebyshev interpolant of
+// degree 7 of (asin(z)/z - 1)/y (relative error of the seed 2^-38).
+GPL_CR_HD double quick_acos_seed(double x)
+{
+  const double ax = fabs(x), h = (1.0 - ax)*0.5;
+  const bool mid = ax <= 0.5;
+  const double y = mid ? x*x : h;
+  const double z = mid ? x : sqrt(h);
+  double P = 0.02930523970533579;
+  P = fma(P, y, 0.0054431851027481075);
+  P = fma(P, y, 0.019306260869368045);
+  P = fma(P, y, 0.022132443623426794);
+  P = fma(P, y, 0.030397634130580702);
+  P = fma(P, y, 0.044642358484883196);
+  P = fma(P, y, 0.07500000598829049);
+  P = fma(P, y, 0.16666666665495086);
+  const double a = fma(z*y, P, z);
+  return mid ? kPiHi*0.5 - a : a;
+}
+
+// The same step from the quick phase, with one division for either form; false
+// if the bound of its error leaves two roundings.  The step's own second-order
+// term is below 2^-77 (relative to phi for |x| > 1/2).  |x| <= 1/2: the error of cos
+// over sin theta >= 0.86, below 2^-73.  |x| > 1/2: that of sin^2 over sin 2 phi,
+// below 2^-73, for k = 0 phi 2^-67.8.
+GPL_CR_HD bool quick_acos(double x, double seed, double *res)
+{
+  const sincos_sum q = quick_sincos(seed);
+  const dd s = fast_two_sum(q.sh, q.sl);
+  const double ax = fabs(x), h = (1.0 - ax)*0.5;
+  const bool mid = ax <= 0.5;
+  dd s2 = two_prod(s.hi, s.hi);
+  s2.lo += 2.0*s.hi*s.lo;
+  const double num = mid ? (q.ch - x) + q.cl : (h - s2.hi) - s2.lo;
+  const double den = mid ? s.hi : 2.0*s.hi*(q.ch + q.cl);
+  const double delta = num/den;
+  const double e = q.k ? kE71 : seed*kE65;
+  const bool neg = !mid && x < 0.0;
+  dd t = two_sum(kPiHi, -2.0*seed);
+  t.lo += kPiLo - 2.0*delta;
+  const double hi = neg ? t.hi : seed, lo = neg ? t.lo : delta, err = neg ? 2.0*e : e;
+  const double r1 = hi + (lo + err), r2 = hi + (lo - err);
+  *res = !mid && !neg ? 2.0*r1 : r1;
+  return r1 == r2;
+}
+
+// acos(x) correctly rounded for -1 <= x <= 1, else NaN.
 GPL_CR_HD double acos_cr(double x)
 {
-  if (!(x >= -1.0 && x <= 1.0)) return acos(x);
+  if (!(x >= -1.0 && x <= 1.0)) return __builtin_nan("");
   if (x == 1.0) return 0.0;
   if (x == -1.0) return kPiHi;
+  double r;
+  if (quick_acos(x, quick_acos_seed(x), &r)) return r;
   return acos_refine(x, acos_seed(x));
 }
 

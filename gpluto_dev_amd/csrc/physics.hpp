@@ -961,7 +961,20 @@ GPL_HD bool rmhd_quartic_extremes(double b, double c, double d, double e, double
   z[1] = -0.25*b + sz1 - sz2 - sz3;
   z[2] = -0.25*b - sz1 + sz2 - sz3;
   z[3] = -0.25*b - sz1 - sz2 + sz3;
-  // SortArray (insertion sort, strict >): the extremes of the sorted list
+  // SortArray (insertion sort, strict >): the ends of the sorted list, the first
+  // of the smallest and the last of the largest.  With a NaN among them (infinite
+  // roots) the order depends on the comparisons made: the sort itself.
+  const double zs = z[0] + z[1] + z[2] + z[3];
+  if (zs == zs) {
+    double lo = z[0], hi = z[0];
+    for (int j = 1; j < 4; j++) {
+      lo = lo > z[j] ? z[j] : lo;
+      hi = hi > z[j] ? hi : z[j];
+    }
+    zmin = lo;
+    zmax = hi;
+    return true;
+  }
   for (int j = 1; j < 4; j++) {
     const double f = z[j];
     int i = j - 1;

@@ -94,4 +94,49 @@ long long crm_compare(int mode, long long n, unsigned long long seed, double lo,
   return total.load();
 }
 
+// The quick phase against the double-double forms on argument()'s modes: the
+// number of results that differ; out[0] the largest error of quick_sincos as a
+// fraction of the bound its rounding test takes, out[1] the number of arguments
+// whose rounding it leaves to the double-double form.
+long long crm_quick(int mode, long long n, unsigned long long seed, double lo, double hi,
+                    int nthreads, double *out)
+{
+  using namespace gpl::cr;
+  std::atomic<long long> differ{0}, left{0};
+  std::vector<double> worst(std::max(1, nthreads), 0.0);
+  std::vector<std::thread> pool;
+  for (int t = 0; t < (int)worst.size(); t++) {
+    pool.emplace_back([&, t]() {
+      long long nd = 0, nl = 0;
+      for (long long i = t; i < n; i += (long long)worst.size()) {
+        double x = argument(mode, (uint64_t)i, seed, lo, hi);
+        if (mode == 0 || mode == 1) {
+          if (x == 1.0 || x == -1.0) continue;
+          double r;
+          const double exact = acos_refine(x, acos_seed(x));
+          if (!quick_acos(x, quick_acos_seed(x), &r)) nl++;
+          else if (r != exact) nd++;
+          if (acos_cr(x) != exact) nd++;
+          x = acos_seed(x);
+        }
+        dd s, c;
+        dd_sincos(x, s, c);
+        const sincos_sum q = quick_sincos(x);
+        const double es = fabs(((q.sh - s.hi) + q.sl) - s.lo)/(q.k ? kE72 : q.sh*kE66);
+        const double ec = fabs(((q.ch - c.hi) + q.cl) - c.lo)/kE72;
+        worst[t] = std::max(worst[t], std::max(x > 0.0 ? es : 0.0, ec));
+        double sn, cs;
+        sincos_cr(x, &sn, &cs);
+        if (sn != s.hi + s.lo || cs != c.hi + c.lo) nd++;
+      }
+      differ += nd;
+      left += nl;
+    });
+  }
+  for (auto &th : pool) th.join();
+  out[0] = *std::max_element(worst.begin(), worst.end());
+  out[1] = (double)left.load();
+  return differ.load();
+}
+
 }  // extern "C"
