@@ -92,6 +92,30 @@ inline int march_length(bool fp64, long long across, int n)
   return best;
 }
 
+// Whole columns per block for a y or z sweep of columns of n cells (FP64), or 0
+// for the march of `march` cells.  A block of c columns solves every face once,
+// c*n lanes side by side; rows of fewer than 4 cells (32 bytes) waste too much of
+// each cache line and blocks over 256 lanes stall on their barriers (64^3, y + z:
+// 17 + 20 us with 4 columns, 21 + 24 with 2 and with 8).  In units of one wavefront's
+// solve the busiest CU takes ceil(blocks / CUs) ceil(c n / 64) against the march's
+// (L + 1.5) per wavefront; the columns are taken where that is 10% less.  Step, us,
+// march -> columns: MHD HLLD 16^3 62 -> 55, 64^3 152 -> 138, 128x64^2 266 -> 242,
+// 128^2x64 (ratio 0.91, refused) 500 -> 516; RMHD HLL 64^3 245 -> 199, HLLD 64^3
+// 504 -> 376, HLLD van Leer RK3 50x44x38 455 -> 314.
+inline int sweep_columns(int nx, int na, int n, int march)
+{
+  constexpr int kCUs = 256, kBlock = 256;
+  const long long mb = ((long long)nx*na*((n + march - 1)/march) + kBlock - 1)/kBlock;
+  double best = 0.9*(double)((mb + kCUs - 1)/kCUs)*(kBlock/64)*(march + 1.5);
+  int x = 0;
+  for (int c = 4; c <= 8 && c*n <= kBlock; c++) {
+    const long long blocks = (long long)((nx + c - 1)/c)*na;
+    const double t = (double)((blocks + kCUs - 1)/kCUs)*((c*n + 63)/64);
+    if (t < best) { best = t; x = c; }
+  }
+  return x;
+}
+
 // invDt_hyp = max over the partial maxima / DIMENSIONS; with advance != 0
 // also NextTimeStep and time += dt on the device.
 void launch_dt(const double *part, int nparts, double dims, StepCtl *ctl, double cfl,

@@ -83,6 +83,7 @@ public:
   // cells per lane of the y march (rows per block of the x+y kernel) and of
   // the z march (march_length)
   int march[2] = {16, 16};
+  int cols[2] = {0, 0};        // whole columns per block instead (sweep_columns)
   // x and y sweeps in one row-marching kernel: the mixed form, where it saves
   // HBM traffic (its three LDS rows must fit in 64 KB); the FP64 sweeps are
   // VALU-bound and run faster as two kernels
@@ -198,7 +199,12 @@ public:
       }
       if (!pipelined && want >= 3 && !getenv("GPL_EMF_MARCH")) emf_march = emf_auto;
     }
-    nparts = fused ? mhd3d_march_blocks(g, march[1]) : mhd3d_blocks(g);
+    if (fp64 && fused && !fused_xy && !pipelined && !getenv("GPL_MARCH")) {
+      cols[0] = sweep_columns(g.nx, g.nz, g.ny, march[0]);
+      cols[1] = sweep_columns(g.nx, g.ny, g.nz, march[1]);
+    }
+    nparts = !fused ? mhd3d_blocks(g) : cols[1] ? (g.nx + cols[1] - 1)/cols[1]*g.ny
+                                                : mhd3d_march_blocks(g, march[1]);
     if (pipelined) {
       // C_dt partial slots: each slab's z march writes its own range
       slab_part0.resize(nslab);
@@ -402,7 +408,7 @@ public:
     b.F = (R *)F; b.CM = (R *)CM; b.FD = (R *)FD; b.E = (R *)E;
     b.dU = (R *)dU; b.Cdt = (R *)Cdt;
     b.cdt_part = cdt_part; b.err = env.err;
-    b.march[0] = march[0]; b.march[1] = march[1];
+    for (int d = 0; d < 2; d++) { b.march[d] = march[d]; b.cols[d] = cols[d]; }
     b.emf_march = emf_march;
     b.phys = rmhd ? 1 : 0;
     b.net = net_on ? net : nullptr;

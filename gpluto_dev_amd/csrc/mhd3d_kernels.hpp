@@ -695,6 +695,108 @@ void k_sweep_march(Box3 g, int L, const R *__restrict__ V, const double *__restr
   }
 }
 
+// ---------------------------------------------------------------------------
+// y / z sweep of short columns: a block holds X whole periodic columns, a lane
+// one cell and its lower face, shared through LDS as in k_sweepx_fused: every
+// face solved once, no march.
+// A march of L solves L + 1 faces one after the other; on a small box L is small
+// and the chip waits for that chain (HLLD 64^3, L = 4, y + z 20 + 24 us against
+// 17 + 20; RMHD HLLD 64^3 85 + 88 against 55 + 55).  Issue-bound as the x sweep,
+// 164 - 168 registers (HLLD), three wavefronts per SIMD where the march has one.
+// From about 128^3 on the march's unbroken rows of x win: 96 + 112 us against
+// 165 + 214.  sweep_columns draws the line.
+// ---------------------------------------------------------------------------
+template <typename R, int D, int LIM, int SOLVER, int PH>
+__global__ __launch_bounds__(256)
+void k_sweep_cols(Box3 g, int X, const R *__restrict__ V, const double *__restrict__ Vs,
+                  R *__restrict__ FD, R *__restrict__ dU, R *__restrict__ Cdt,
+                  const double *Uin, double *U, const double *U0,
+                  const StepCtl *__restrict__ ctl, RKW w, int first_stage, int want_cdt,
+                  double *__restrict__ cdt_part, R gamma, uint32_t *__restrict__ err)
+{
+  static_assert(D == 1 || D == 2, "columns along y or z");
+  extern __shared__ __align__(16) unsigned char gpl_smem[];
+  constexpr int BXn = 4 + D;
+  constexpr int VAR[7] = {0, 1, 2, 3, 4, D == 1 ? 6 : 5, 7};
+  const int t = threadIdx.x, T = blockDim.x;
+  R *sV = (R *)gpl_smem;           // [7][T] primitives
+  R *sD = sV + 7*T;                // [7][T] state at the upper face made by the cell
+  const int nd = D == 1 ? g.ny : g.nz;
+  const int ntx = (g.nx + X - 1)/X;
+  const int b = xcd_tile(blockIdx.x, gridDim.x);
+  const int a = b / ntx;           // the other transverse index
+  const int r = t / X, it = (b - a*ntx)*X + t - r*X;
+  const bool own = it < g.nx && r < nd;         // the other lanes repeat a cell
+  const int p = r < nd ? r : nd - 1, i = it < g.nx ? it : g.nx - 1;
+  const unsigned c = D == 1 ? i + (unsigned)g.nx*(p + g.ny*a) : i + (unsigned)g.nx*(a + g.ny*p);
+  const size_t n = (size_t)g.ncell;
+  const int tm = p > 0 ? t - X : t + (nd - 1)*X;
+  const int tp = p < nd - 1 ? t + X : t - (nd - 1)*X;
+  R v0[7];
+#pragma unroll
+  for (int q = 0; q < 7; q++) { v0[q] = ldo(V + VAR[q]*n, c); sV[q*T + t] = v0[q]; }
+  const R bn = (R)ldo(Vs + D*n, c);
+  __syncthreads();
+  R lo[7], hi[7];                  // the cell's states at its lower and upper face
+#pragma unroll
+  for (int q = 0; q < 7; q++) {
+    const R dv = plm_slope<R, LIM>(sV[q*T + tm], v0[q], sV[q*T + tp]);
+    lo[q] = v0[q] - R(0.5)*dv;
+    hi[q] = v0[q] + R(0.5)*dv;
+  }
+  if (PH == 1 && superluminal(lo, hi)) {
+#pragma unroll
+    for (int q = 0; q < 7; q++) lo[q] = hi[q] = v0[q];
+  }
+#pragma unroll
+  for (int q = 0; q < 7; q++) sD[q*T + t] = hi[q];
+  __syncthreads();
+  R vl[8], vr[8];
+#pragma unroll
+  for (int q = 0; q < 7; q++) { vl[VAR[q]] = sD[q*T + tm]; vr[VAR[q]] = lo[q]; }
+  vl[BXn] = vr[BXn] = bn;
+  FaceFlux<R> ff;
+  riemann<R, D, SOLVER, PH>(vl, vr, gamma, ff, g);
+  if (own) uct_store<R, D, SOLVER>(vl, vr, gamma, ff, FD + (size_t)D*uct_nrec<SOLVER>()*n, c, n);
+  const bool rep = D == 1 ? face_reported<1>(g, i, p, a) : face_reported<2>(g, i, a, p);
+  const uint32_t e = own && rep ? ff.err : 0;
+  __syncthreads();                 // everyone is done with sV/sD
+  R *sF = sV;                      // [6][T]: hydro flux and cmax of the lower face
+  sF[0*T + t] = ff.f[0]; sF[1*T + t] = ff.f[1]; sF[2*T + t] = ff.f[2];
+  sF[3*T + t] = ff.f[3]; sF[4*T + t] = ff.f[7];
+  sF[5*T + t] = rmax(rabs(ff.Sl), rabs(ff.Sr));
+  __syncthreads();
+  double cdt = -1.0;
+  if (own) {
+    const double ddx = D == 1 ? g.dy : g.dz, dtdx = ctl->dt/ddx;
+#pragma unroll
+    for (int nv = 0; nv < 5; nv++) {
+      double rr = -dtdx*((double)sF[nv*T + tp] - (double)sF[nv*T + t]);
+      if (PH == 0) rr += 0.0;
+      double du = (double)ldo((const R *)(dU + nv*n), c);
+      du += rr;
+      if (D == 1) {
+        sto(dU + nv*n, c, (R)du);
+      } else if (first_stage) {
+        sto(U + nv*n, c, ldo(Uin + nv*n, c) + w.wR*du);
+      } else {
+        sto(U + nv*n, c, w.w0*ldo(U0 + nv*n, c) + w.w1*ldo(Uin + nv*n, c) + w.wR*du);
+      }
+    }
+    if (want_cdt) {
+      double cd = (double)ldo((const R *)Cdt, c);
+      cd += 0.5*((double)sF[5*T + t] + (double)sF[5*T + tp])/ddx;
+      if (D == 1) sto(Cdt, c, (R)cd);
+      else if (is_active(g, i, a, p)) cdt = cd;
+    }
+  }
+  report_bits(err, e);
+  if (D == 2 && want_cdt) {
+    const double m = block_max(cdt);
+    if (t == 0) cdt_part[blockIdx.x] = m;
+  }
+}
+
 // PLM of a scalar column for the EMF average (array_reconstruct.cpp:167-205):
 // left state at the interface between q1 and q2 from (q0,q1,q2), right state
 // from (q1,q2,q3).
@@ -1201,13 +1303,30 @@ static inline int emf_flat(int nx) { return ((nx + 63)/64)*64*4 > 5*nx; }
 // Host-side launch helpers: one entry per kernel family, so that the host
 // orchestration can bracket each launch with timing events.
 // ---------------------------------------------------------------------------
-// The fused sweeps: x, and the y and z marches.
+// The fused sweeps: x, and the y and z marches or whole columns (FP64).
 template <typename R, int LIM, int SOLVER, int PH>
 static void launch_sweep(int which, const Mhd3dBufs<R> &b, const Box3 &g, const StepCtl *ctl, RKW w,
                          int first_stage, int want_dt, double gamma, hipStream_t s)
 {
   const int T = 256;
   const int nk = g.ke - g.kb;          // planes of the launch
+  if constexpr (sizeof(R) == 8) {
+    const int d = which == K_SWEEPZ_F, X = which == K_SWEEPX_F ? 0 : b.cols[d];
+    if (X > 0) {
+      const int nd = d ? g.nz : g.ny, tt = (X*nd + 63)/64*64;
+      const int grid = (g.nx + X - 1)/X*(d ? g.ny : g.nz);
+      const size_t shm = 14*(size_t)tt*sizeof(R);
+      if (d == 0)
+        hipLaunchKernelGGL((k_sweep_cols<R, 1, LIM, SOLVER, PH>), dim3(grid), dim3(tt), shm, s,
+                           g, X, b.V, b.Vin, b.FD, b.dU, b.Cdt, b.Uin, b.U, b.U0, ctl, w, first_stage,
+                           want_dt, b.cdt_part, (R)gamma, b.err);
+      else
+        hipLaunchKernelGGL((k_sweep_cols<R, 2, LIM, SOLVER, PH>), dim3(grid), dim3(tt), shm, s,
+                           g, X, b.V, b.Vin, b.FD, b.dU, b.Cdt, b.Uin, b.U, b.U0, ctl, w, first_stage,
+                           want_dt, b.cdt_part, (R)gamma, b.err);
+      return;
+    }
+  }
   if (which == K_SWEEPX_F) {
     const size_t shm = 14*(size_t)g.nx*sizeof(R);
     hipLaunchKernelGGL((k_sweepx_fused<R, LIM, SOLVER, PH>), dim3(g.ny*nk), dim3(g.nx), shm, s,

@@ -155,3 +155,33 @@ def test_hd_launch_shapes_match_oracle(n, ts, lim, solver, sides):
     assert inv == o.advance(dt0)
     ovc, _, ouc = o.get_state()
     assert np.array_equal(gvc, ovc) and np.array_equal(guc, ouc)
+
+
+@pytest.mark.parametrize("n,phys,solver,lim,sides", [
+    ((5, 3, 4), "MHD", "hlld", "MC_LIM", ()),                    # columns shorter than a wavefront's rows
+    ((9, 64, 5), "MHD", "hll", "VANLEER_LIM", ()),               # the longest column, 4 per block
+    ((33, 17, 64), "MHD", "hlld", "MC_LIM", ()),                 # remainders in x and in the last wavefront
+    ((13, 65, 32), "MHD", "hllc", "MC_LIM", ()),                 # y marches, z in columns of 8
+    ((18, 14, 21), "MHD", "hlld", "VANLEER_LIM", ("outflow", "reflective", "outflow", "outflow",
+                                                  "reflective", "reflective")),
+    ((21, 30, 11), "RMHD", "hll", "MC_LIM", ()),
+    ((14, 19, 38), "RMHD", "hlld", "VANLEER_LIM", ()),
+])
+def test_columns_match_marches(n, phys, solver, lim, sides, monkeypatch):
+    """y and z sweeps of whole columns against marches of 4: the same bits, dt
+    and error word included."""
+    rel = phys == "RMHD"
+    state = ic.rmhd_turbulence(n, 5, lorentz_max=2.0, sigma=0.3) if rel else ic.mhd_turbulence(n, 5)
+    res = []
+    for march in ("", "4"):
+        if march:
+            monkeypatch.setenv("GPL_MARCH", march)
+        print(f"case n={n} {phys} {solver} {lim} {sides} march={march}", flush=True)
+        g = StageUpdate(Definitions(physics=phys, time_stepping="RK3", limiter=lim),
+                        RuntimeSetup(n=n, solver=solver, sides=tuple(sides), cfl=0.2,
+                                     gamma=4 / 3 if rel else 5 / 3))
+        g.upload(*state)
+        res.append((g.run(3, 1e-3), *g.download()))
+        g.close()
+    assert res[0][0] == res[1][0]
+    assert all(np.array_equal(a, b) for a, b in zip(res[0][1:], res[1][1:]))
