@@ -116,6 +116,24 @@ inline int sweep_columns(int nx, int na, int n, int march)
   return x;
 }
 
+// Rows per block of the 3D x sweep: the fewest whose wavefronts on the busiest CU,
+// ceil(blocks / CUs) ceil(rows nx / 64), are 5% fewer than with fewer rows, blocks
+// of at most 256 lanes.  x sweep, us, one row -> this many: 20x70x90 20 -> 12
+// (3 rows), 72x80x66 27 -> 22 (3), 79x94x65 (75x90x61 with ghosts) 32 -> 26 (3),
+// 96^3 43 -> 38 (2).
+inline int sweep_rows(int nx, long long nrows)
+{
+  constexpr int kCUs = 256, kBlock = 256;
+  int rows = 1;
+  double best = 0.0;
+  for (int m = 1; m == 1 || m*nx <= kBlock; m++) {
+    const long long blocks = (nrows + m - 1)/m;
+    const double t = (double)((blocks + kCUs - 1)/kCUs)*((m*nx + 63)/64);
+    if (m == 1 || t < 0.95*best) { best = t; rows = m; }
+  }
+  return rows;
+}
+
 // invDt_hyp = max over the partial maxima / DIMENSIONS; with advance != 0
 // also NextTimeStep and time += dt on the device.
 void launch_dt(const double *part, int nparts, double dims, StepCtl *ctl, double cfl,

@@ -83,6 +83,7 @@ public:
   // cells per lane of the y march (rows per block of the x+y kernel) and of
   // the z march (march_length)
   int march[2] = {16, 16};
+  int rows = 1;                // rows per block of the x sweep (sweep_rows)
   int cols[2] = {0, 0};        // whole columns per block instead (sweep_columns)
   // x and y sweeps in one row-marching kernel: the mixed form, where it saves
   // HBM traffic (its three LDS rows must fit in 64 KB); the FP64 sweeps are
@@ -199,6 +200,7 @@ public:
       }
       if (!pipelined && want >= 3 && !getenv("GPL_EMF_MARCH")) emf_march = emf_auto;
     }
+    rows = sweep_rows(g.nx, (long long)g.ny*g.nz);
     if (fp64 && fused && !fused_xy && !pipelined && !getenv("GPL_MARCH")) {
       cols[0] = sweep_columns(g.nx, g.nz, g.ny, march[0]);
       cols[1] = sweep_columns(g.nx, g.ny, g.nz, march[1]);
@@ -408,6 +410,7 @@ public:
     b.F = (R *)F; b.CM = (R *)CM; b.FD = (R *)FD; b.E = (R *)E;
     b.dU = (R *)dU; b.Cdt = (R *)Cdt;
     b.cdt_part = cdt_part; b.err = env.err;
+    b.rows = rows;
     for (int d = 0; d < 2; d++) { b.march[d] = march[d]; b.cols[d] = cols[d]; }
     b.emf_march = emf_march;
     b.phys = rmhd ? 1 : 0;

@@ -50,6 +50,7 @@ struct Mhd3dBufs {
   double *cdt_part;
   uint32_t *err;
   int march[2];    // cells per lane of the y march (and rows per block of the x+y kernel), of the z march
+  int rows;        // x-rows per block of the x sweep
   int cols[2];     // y and z sweep by that many whole columns per block (0: the march)
   int emf_march;   // EMF kernel: 0 one edge per thread, n > 0 register z-march of n, -n LDS tiles marching n
   int phys;        // 0: ideal MHD, 1: relativistic MHD (FP64, fused kernels)

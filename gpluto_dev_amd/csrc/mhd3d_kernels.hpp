@@ -300,7 +300,9 @@ void k_rhs_update(Box3 g, const R *__restrict__ F, const R *__restrict__ CM,
 }
 
 // ---------------------------------------------------------------------------
-// Fused x sweep: one block per periodic x-row (blockDim.x == nx <= 512).
+// Fused x sweep: `rows` whole periodic x-rows per block (nx <= 512).
+// Issue-bound (HLLD at 256^3 35 ps per cell); idle lanes of a row's last wavefront
+// cost as much as busy ones, so sweep_rows packs several rows into a block.
 // DataToSweep/Reconstruct (plm_states.cpp:99-189) with every cell's slope
 // computed once and shared through LDS, HLLD (hlld.cpp:100-500), CT store,
 // and RightHandSide's x part (rhs.cpp:384-386, 523): dUc = rhs_x
@@ -308,29 +310,40 @@ void k_rhs_update(Box3 g, const R *__restrict__ F, const R *__restrict__ CM,
 // ---------------------------------------------------------------------------
 template <typename R, int LIM, int SOLVER, int PH>
 __global__ __launch_bounds__(512)
-void k_sweepx_fused(Box3 g, const R *__restrict__ V, const double *__restrict__ Vs,
+void k_sweepx_fused(Box3 g, int rows, const R *__restrict__ V, const double *__restrict__ Vs,
                     R *__restrict__ FD, R *__restrict__ dU, R *__restrict__ Cdt,
                     const StepCtl *__restrict__ ctl, R gamma, int want_cdt,
                     uint32_t *__restrict__ err)
 {
   extern __shared__ __align__(16) unsigned char gpl_smem[];
-  const int nx = g.nx, i = threadIdx.x;
-  R *sV = (R *)gpl_smem;           // [7][nx] primitives of the row
-  R *sD = sV + 7*nx;               // [7][nx] left state vL(i+1) made by cell i
+  const int nx = g.nx, t = threadIdx.x, T = blockDim.x;
+  R *sV = (R *)gpl_smem;           // [7][T] primitives of the rows
+  R *sD = sV + 7*T;                // [7][T] left state vL(i+1) made by cell i
   const size_t n = (size_t)g.ncell;
-  const unsigned row = blockIdx.x + (unsigned)g.ny*g.kb;   // j + ny*k
+  // row j + ny*k; the lanes past the last row or the block's rows repeat a cell
+  int ln = 0, i = t;
+  bool own = true;
+  unsigned row = blockIdx.x*rows + (unsigned)g.ny*g.kb;
+  if (rows > 1) {
+    const int left = g.ny*g.ke - (int)row, m = rows < left ? rows : left;
+    ln = t / nx;
+    own = ln < m;
+    ln = own ? ln : m - 1;
+    i = own ? t - ln*nx : 0;
+    row += ln;
+  }
   const unsigned c = i + nx*row;
-  const int im = i == 0 ? nx - 1 : i - 1, ip = i == nx - 1 ? 0 : i + 1;
+  const int o = ln*nx, im = o + (i == 0 ? nx - 1 : i - 1), ip = o + (i == nx - 1 ? 0 : i + 1);
   constexpr int VAR[7] = {0, 1, 2, 3, 5, 6, 7};   // B1 comes from the face
   R v0[7], dv[7];
 #pragma unroll
-  for (int q = 0; q < 7; q++) { v0[q] = ldo(V + VAR[q]*n, c); sV[q*nx + i] = v0[q]; }
+  for (int q = 0; q < 7; q++) { v0[q] = ldo(V + VAR[q]*n, c); sV[q*T + t] = v0[q]; }
   const R bn = (R)ldo(Vs, c);
   __syncthreads();
   R lo[7], hi[7];                  // this cell's vR(i) and vL(i+1)
 #pragma unroll
   for (int q = 0; q < 7; q++) {
-    dv[q] = plm_slope<R, LIM>(sV[q*nx + im], v0[q], sV[q*nx + ip]);
+    dv[q] = plm_slope<R, LIM>(sV[q*T + im], v0[q], sV[q*T + ip]);
     lo[q] = v0[q] - R(0.5)*dv[q];
     hi[q] = v0[q] + R(0.5)*dv[q];
   }
@@ -339,32 +352,33 @@ void k_sweepx_fused(Box3 g, const R *__restrict__ V, const double *__restrict__ 
     for (int q = 0; q < 7; q++) lo[q] = hi[q] = v0[q];
   }
 #pragma unroll
-  for (int q = 0; q < 7; q++) sD[q*nx + i] = hi[q];
+  for (int q = 0; q < 7; q++) sD[q*T + t] = hi[q];
   __syncthreads();
   R vl[8], vr[8];
 #pragma unroll
   for (int q = 0; q < 7; q++) {
-    vl[VAR[q]] = sD[q*nx + im];
+    vl[VAR[q]] = sD[q*T + im];
     vr[VAR[q]] = lo[q];
   }
   vl[4] = vr[4] = bn;
   FaceFlux<R> ff;
   riemann<R, 0, SOLVER, PH>(vl, vr, gamma, ff, g);
-  uct_store<R, 0, SOLVER>(vl, vr, gamma, ff, FD, c, n);
+  if (own) uct_store<R, 0, SOLVER>(vl, vr, gamma, ff, FD, c, n);
   __syncthreads();                 // everyone is done with sV/sD
-  R *sF = sV;                      // [6][nx]: hydro flux and cmax of face i
-  sF[0*nx + i] = ff.f[0]; sF[1*nx + i] = ff.f[1]; sF[2*nx + i] = ff.f[2];
-  sF[3*nx + i] = ff.f[3]; sF[4*nx + i] = ff.f[7];
-  sF[5*nx + i] = rmax(rabs(ff.Sl), rabs(ff.Sr));
+  R *sF = sV;                      // [6][T]: hydro flux and cmax of face i
+  sF[0*T + t] = ff.f[0]; sF[1*T + t] = ff.f[1]; sF[2*T + t] = ff.f[2];
+  sF[3*T + t] = ff.f[3]; sF[4*T + t] = ff.f[7];
+  sF[5*T + t] = rmax(rabs(ff.Sl), rabs(ff.Sr));
   __syncthreads();
+  if (!own) return;
   const double dtdx = ctl->dt/g.dx;
 #pragma unroll
   for (int nv = 0; nv < 5; nv++) {
-    double r = -dtdx*((double)sF[nv*nx + ip] - (double)sF[nv*nx + i]);
+    double r = -dtdx*((double)sF[nv*T + ip] - (double)sF[nv*T + t]);
     if (PH == 0) r += 0.0;         // MHD adds src[] = 0 (rhs.cpp:519); RMHD+CT has no source
     sto(dU + nv*n, c, (R)r);
   }
-  if (want_cdt) sto(Cdt, c, (R)(0.5*((double)sF[5*nx + i] + (double)sF[5*nx + ip])/g.dx));
+  if (want_cdt) sto(Cdt, c, (R)(0.5*((double)sF[5*T + t] + (double)sF[5*T + ip])/g.dx));
   if (ff.err && face_reported<0>(g, i, (int)(row % g.ny), (int)(row / g.ny)))
     report_bits(err, ff.err);
 }
@@ -1328,9 +1342,10 @@ static void launch_sweep(int which, const Mhd3dBufs<R> &b, const Box3 &g, const 
     }
   }
   if (which == K_SWEEPX_F) {
-    const size_t shm = 14*(size_t)g.nx*sizeof(R);
-    hipLaunchKernelGGL((k_sweepx_fused<R, LIM, SOLVER, PH>), dim3(g.ny*nk), dim3(g.nx), shm, s,
-                       g, b.V, b.Vin, b.FD, b.dU, b.Cdt, ctl, (R)gamma, want_dt, b.err);
+    const int rows = b.rows, tt = rows > 1 ? (rows*g.nx + 63)/64*64 : g.nx;
+    const size_t shm = 14*(size_t)tt*sizeof(R);
+    hipLaunchKernelGGL((k_sweepx_fused<R, LIM, SOLVER, PH>), dim3((g.ny*nk + rows - 1)/rows), dim3(tt), shm, s,
+                       g, rows, b.V, b.Vin, b.FD, b.dU, b.Cdt, ctl, (R)gamma, want_dt, b.err);
   } else if (which == K_SWEEPY_F) {
     const int L = b.march[0], nt = g.nx*nk*((g.ny + L - 1)/L);
     hipLaunchKernelGGL((k_sweep_march<R, 1, LIM, SOLVER, PH>), dim3((nt + T - 1)/T), dim3(T), 0, s,

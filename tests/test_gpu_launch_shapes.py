@@ -185,3 +185,15 @@ def test_columns_match_marches(n, phys, solver, lim, sides, monkeypatch):
         g.close()
     assert res[0][0] == res[1][0]
     assert all(np.array_equal(a, b) for a, b in zip(res[0][1:], res[1][1:]))
+
+
+@pytest.mark.parametrize("n", [(5, 21, 37), (20, 23, 29), (72, 17, 19)])
+def test_rows_per_block_match_oracle(n):
+    """x sweeps of 4, 3 and 2 rows per block, the last block short of a row."""
+    import oracle
+    (err, t, dt), vc, vs, _ = _run(n, 3, 1e-3)
+    o = oracle.Oracle(phys="mhd", n=n, gamma=5 / 3)
+    o.set_state(*ic.mhd_turbulence(n, 17))
+    assert (err, t, dt) == o.run(3, 1e-3)
+    ovc, ovs, _ = o.get_state()
+    assert np.array_equal(vc, ovc) and np.array_equal(vs, ovs)
