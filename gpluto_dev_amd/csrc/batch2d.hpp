@@ -28,9 +28,26 @@ struct BoxDesc {
 // Work items.  Sweep items are one wavefront each:
 //   x: {box, row j, first cell i0, cells in the segment (<= 63)}
 //   y: {box, first column i0 (64 lanes), segment index, unused}
-// Cell tiles (EMF, face update): {box, first cell within the box}, 256 cells.
+// Cell tiles (EMF, face update): {box, tile within the box, x fastest}.
 struct Item4 { int box, a, b, c; };
-struct Item2 { int box, start; };
+struct Item2 { int box, tile; };
+
+// Cells (w, h) of a tile in a box nx cells wide, for blocks of 320 or 192 lanes:
+// 32 x 8 or 32 x 4, in a narrower box whole rows; (w + 1)(h + 1) edges at most one
+// per lane, at most 256 or 128 cells.
+constexpr int kTileLanes = 320, kTileLanesSmall = 192;
+struct Tile2 { int w, h; };
+__host__ __device__ inline Tile2 tile2d(int nx, int lanes)
+{
+  const int w = nx < 32 ? nx : 32;
+  const int h = (lanes == kTileLanes ? 256 : 128)/w, he = lanes/(w + 1) - 1;
+  return {w, h < he ? h : he};
+}
+inline int tile_count(int nx, int ny, int lanes)
+{
+  const Tile2 t = tile2d(nx, lanes);
+  return (nx + t.w - 1)/t.w*((ny + t.h - 1)/t.h);
+}
 
 template <typename R>
 struct Batch2dBufs {
@@ -46,7 +63,7 @@ struct Batch2dBufs {
   const double *Bs0; // [2][ncell] faces at the start of the step (second stage on)
   R *FD;             // [2][4][ncell] UCT face data et, eb, min(0,Sl), max(0,Sr); UCT_HLLD:
                      // [2][6][ncell] et, eb, aL, aR, dL, dR
-  R *E;              // [ncell] Ez at the lower-left corner of every cell
+  R *E;              // [ncell] Ez at the lower-left corner of every cell (two launches)
   R *dU;             // [6][ncell] x-sweep flux divergence
   R *Cdt;            // [ncell]    x-sweep C_dt
   double *cdt_part;  // one C_dt maximum per y item
@@ -56,12 +73,13 @@ struct Batch2dBufs {
   const Item4 *xitems;
   const Item4 *yitems;
   const Item2 *tiles;
+  int tile_lanes;    // lanes per block of the one-launch EMF and update (0: two launches, tiles of 256 cells)
   int nx_items, ny_items, ntiles;
   int ncell;
   ZoneRep zr;        // this stage's zone-by-zone reports (zr.err null: off)
 };
 
-enum Batch2dPhase { B2_SWEEP_X = 0, B2_SWEEP_Y, B2_EMF, B2_FINISH };
+enum Batch2dPhase { B2_SWEEP_X = 0, B2_SWEEP_Y, B2_EMF, B2_FINISH, B2_CT };
 
 // Launch one phase as a persistent grid of 'blocks' workgroups of 256
 // threads; 'march' is the y-segment length the y items were built for.

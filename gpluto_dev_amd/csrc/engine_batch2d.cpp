@@ -76,6 +76,7 @@ struct gpl_batch {
   BoxDesc *box = nullptr;
   Item4 *xitems = nullptr;
   Item2 *tiles = nullptr;
+  int tile_lanes = kTileLanes;
   int nx_items = 0, ntiles = 0;
   Item4 *yitems[4] = {};                            // per march length
   int *part_beg[4] = {};
@@ -161,6 +162,15 @@ static int batch_init(gpl_batch *b, const gpl_config *cfg, int nbox, const int *
   for (int q = 0; q < 4; q++) b->side[q] = side_type(*cfg, q);
   b->padded = !all_periodic(*cfg);
   const int pad = b->padded ? 5 : 0, lo = b->padded ? 2 : 0;
+  // EMF and update in one launch while its blocks of 320 lanes are all in flight at
+  // once, four per CU (512^2 step 116 us in two launches, 108 in one; 768^2, 2.25
+  // rounds of blocks, 210 and 227; 1024^2, four rounds, 397 and 394); in smaller tiles
+  // where half of the CUs would get none (64^2 41.8 -> 40.8, 128^2 44.7 -> 43.5)
+  {
+    long long nt = 0;
+    for (int q = 0; q < nbox; q++) nt += tile_count(nx[q] + pad, ny[q] + pad, kTileLanes);
+    b->tile_lanes = nt > 4LL*b->ncu ? 0 : 2*nt > b->ncu ? kTileLanes : kTileLanesSmall;
+  }
   for (int q = 0; q < nbox; q++) {
     BoxDesc d;
     d.nx = nx[q] + pad; d.ny = ny[q] + pad; d.off = off;
@@ -176,7 +186,8 @@ static int batch_init(gpl_batch *b, const gpl_config *cfg, int nbox, const int *
     tstart.push_back((int)ti.size());
     for (int j = 0; j < d.ny; j++)
       for (int i0 = 0; i0 < d.nx; i0 += 63) xi.push_back({q, j, i0, d.nx - i0 < 63 ? d.nx - i0 : 63});
-    for (int s = 0; s < d.nx*d.ny; s += 256) ti.push_back({q, s});
+    const int nt = b->tile_lanes ? tile_count(d.nx, d.ny, b->tile_lanes) : (d.nx*d.ny + 255)/256;
+    for (int s = 0; s < nt; s++) ti.push_back({q, s});
     off += d.nx*d.ny;
   }
   const size_t nc = (size_t)b->ncell, rs = b->fp64 ? sizeof(double) : sizeof(float);
@@ -257,7 +268,7 @@ static int batch_init(gpl_batch *b, const gpl_config *cfg, int nbox, const int *
   rc |= dev_alloc(b->bytes, (void **)&b->Us, 6*nc*sizeof(double));
   for (int q = 0; q < 3; q++) rc |= dev_alloc(b->bytes, (void **)&b->vs[q], 2*nc*sizeof(double));
   rc |= dev_alloc(b->bytes, &b->FD, 2*(b->ksolver == 4 ? 6 : 4)*nc*rs);
-  rc |= dev_alloc(b->bytes, &b->E, nc*rs);
+  if (!b->tile_lanes) rc |= dev_alloc(b->bytes, &b->E, nc*rs);
   rc |= dev_alloc(b->bytes, &b->dU, 6*nc*rs);
   rc |= dev_alloc(b->bytes, &b->Cdt, nc*rs);
   rc |= dev_alloc(b->bytes, (void **)&b->cdt_part, (size_t)max_y*sizeof(double));
@@ -533,6 +544,7 @@ static void enqueue_stage(gpl_batch *b, const double *uin, double *uout, double 
   q.V = (R *)b->V; q.Uin = uin; q.U = uout; q.U0 = b->U;
   q.Vin = vin; q.Vout = vout; q.Bs0 = vbase;
   q.FD = (R *)b->FD; q.E = (R *)b->E; q.dU = (R *)b->dU; q.Cdt = (R *)b->Cdt;
+  q.tile_lanes = b->tile_lanes;
   q.err = b->err; q.ctl = b->ctl; q.box = b->box;
   q.ncell = b->ncell;
   const int m = b->march_idx, march = b->march[m];
@@ -555,10 +567,11 @@ static void enqueue_stage(gpl_batch *b, const double *uin, double *uout, double 
                       c.gamma, c.small_rho, c.small_prs, st);
     batch2d_launch<R>(B2_SWEEP_Y, q, w, first_stage, first_stage, c.limiter, b->ksolver, march, gy,
                       c.gamma, c.small_rho, c.small_prs, st);
-    batch2d_launch<R>(B2_EMF, q, w, first_stage, first_stage, c.limiter, b->ksolver, march, gt,
-                      c.gamma, c.small_rho, c.small_prs, st);
-    batch2d_launch<R>(B2_FINISH, q, w, first_stage, first_stage, c.limiter, b->ksolver, march, gt,
-                      c.gamma, c.small_rho, c.small_prs, st);
+    for (int ph : {b->tile_lanes ? B2_CT : B2_EMF, B2_FINISH}) {
+      batch2d_launch<R>(ph, q, w, first_stage, first_stage, c.limiter, b->ksolver, march, gt,
+                        c.gamma, c.small_rho, c.small_prs, st);
+      if (ph == B2_CT) break;
+    }
   }
 }
 

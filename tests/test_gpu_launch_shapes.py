@@ -197,3 +197,24 @@ def test_rows_per_block_match_oracle(n):
     assert (err, t, dt) == o.run(3, 1e-3)
     ovc, ovs, _ = o.get_state()
     assert np.array_equal(vc, ovc) and np.array_equal(vs, ovs)
+
+
+@pytest.mark.parametrize("n,lim", [((4, 300, 1), "MC_LIM"), ((31, 9, 1), "VANLEER_LIM"), ((32, 8, 1), "MC_LIM"),
+                                   ((33, 17, 1), "MC_LIM"), ((65, 7, 1), "VANLEER_LIM"),
+                                   ((301, 190, 1), "MC_LIM"), ((520, 513, 1), "MC_LIM")])
+def test_2d_tiles_match_oracle(n, lim):
+    """The 2D EMF and update tiles: narrow boxes of whole rows, one tile, remainders of
+    a cell or a row; the larger tiles; a box past one round of blocks (two launches)."""
+    import oracle
+    vc, vs = ic.mhd_turbulence(n, 17)
+    print(f"case n={n} {lim}", flush=True)
+    g = StageUpdate(Definitions(dimensions=2, limiter=lim), RuntimeSetup(n=n))
+    g.upload(vc, vs)
+    res = g.run(3, 1e-3)
+    gvc, gvs, _ = g.download()
+    g.close()
+    o = oracle.Oracle(phys="mhd", n=n, gamma=5 / 3, limiter=lim)
+    o.set_state(vc, vs)
+    assert res == o.run(3, 1e-3)
+    ovc, ovs, _ = o.get_state()
+    assert np.array_equal(gvc, ovc) and np.array_equal(gvs, ovs)
