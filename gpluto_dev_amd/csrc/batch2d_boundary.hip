@@ -26,7 +26,8 @@ namespace {
 // the 3D fill (mhd3d_boundary.hip) the sides write different layers, read
 // active ones, and what a ghost cell needs is computed from the source layers in
 // registers: two launches a stage where a copy and a fill per side were eight
-// (one 306 x 195 box: 44 us a stage in eight, 15 us in two).
+// (one 306 x 195 box: 44 us a stage in eight, 15 us in two, 12 us with every load
+// before the first store).
 template <typename R>
 __global__ __launch_bounds__(256)
 void k2_bnd_dir(const BoxDesc *__restrict__ box, int dir, int type_lo, int type_hi, R *__restrict__ V,
@@ -51,56 +52,61 @@ void k2_bnd_dir(const BoxDesc *__restrict__ box, int dir, int type_lo, int type_
   double *Bt = Vs + tr*N, *Bn = Vs + dir*N;
   const bool cell = a <= na - 2;                // BOX_LOOP over the ghost box
   double e[2][2];                               // tangential faces on both ends of the ghost cells
+  constexpr int VAR[6] = {0, 1, 2, 3, 6, 7};    // B1, B2 are the field average below
+  R v[2][6];
+  const int f0 = upper ? hi + 1 : 0;            // the normal faces f0 .. f0 + 2 bound the two ghost cells
+  double f[3] = {0.0, 0.0, 0.0};
+  // every load before the first store: the arrays are filled in place, so a store
+  // would hold the loads after it back by a trip to memory each
 #pragma unroll
   for (int l = 0; l < 2; l++) {
-    const size_t cp = at + (g0 + l)*sd, cq = at + source(g0 + l)*sd;
-    // the tangential component: one more face along it (BOX{I,J}_LOOP)
+    // one cell across: the upper side's second layer repeats its first
+    const size_t cq = at + (type == GPL_PERIODIC && upper && n == 1 ? hi : source(g0 + l))*sd;
     e[l][0] = Bt[cq];
-    Bt[cp] = e[l][0];
     if (cell) {
       e[l][1] = Bt[cq + st];
-      constexpr int VAR[6] = {0, 1, 2, 3, 6, 7};   // B1, B2 are the field average below
 #pragma unroll
-      for (int q = 0; q < 6; q++) {
-        const int nv = VAR[q];
-        const R v = V[nv*N + cq];
-        V[nv*N + cp] = type == GPL_REFLECTIVE && nv == 1 + dir ? -v : v;
-      }
+      for (int q = 0; q < 6; q++) v[l][q] = V[VAR[q]*N + cq];
+    }
+  }
+  if (cell) {
+    if (type == GPL_PERIODIC) {
+#pragma unroll
+      for (int l = 0; l < 3; l++)
+        f[l] = !upper && l == 2 ? Bn[at + lo*sd] : Bn[at + source(f0 + l)*sd];
+    } else if (type == GPL_REFLECTIVE) {
+      // mirrored about the boundary face and negated: face i from i0 - i + 1 on
+      // the lower side, face i + 1 from i0 - i on the upper side
+      f[upper ? 0 : 2] = Bn[at + (upper ? f0 : lo)*sd];
+      f[upper ? 1 : 0] = -Bn[at + (upper ? source(hi + 1) : source(0) + 1)*sd];
+      f[upper ? 2 : 1] = -Bn[at + (upper ? source(hi + 2) : source(1) + 1)*sd];
+    } else {
+      f[upper ? 0 : 2] = Bn[at + (upper ? hi + 1 : lo)*sd];
+    }
+  }
+#pragma unroll
+  for (int l = 0; l < 2; l++) {
+    const size_t cp = at + (g0 + l)*sd;
+    Bt[cp] = e[l][0];                           // one more face along it (BOX{I,J}_LOOP)
+    if (cell) {
+#pragma unroll
+      for (int q = 0; q < 6; q++)
+        V[VAR[q]*N + cp] = type == GPL_REFLECTIVE && VAR[q] == 1 + dir ? -v[l][q] : v[l][q];
     }
   }
   if (!cell) return;
-  // the normal faces f0 .. f0 + 2 that bound the two ghost cells
-  const int f0 = upper ? hi + 1 : 0;
-  double f[3];
   if (type == GPL_PERIODIC) {
     // BOX_LOOP on the lower side, one more face (the spare layer) on the upper
-#pragma unroll
-    for (int l = 0; l < 3; l++)
-      f[l] = !upper && l == 2 ? Bn[at + lo*sd] : Bn[at + source(f0 + l)*sd];
     Bn[at + f0*sd] = f[0];
     Bn[at + (f0 + 1)*sd] = f[1];
     if (upper) Bn[at + (f0 + 2)*sd] = f[2];
   } else if (type == GPL_REFLECTIVE) {
-    // mirrored about the boundary face and negated: face i from i0 - i + 1 on
-    // the lower side, face i + 1 from i0 - i on the upper side
-    if (!upper) {
-      f[0] = -Bn[at + (source(0) + 1)*sd];
-      f[1] = -Bn[at + (source(1) + 1)*sd];
-      f[2] = Bn[at + lo*sd];
-      Bn[at] = f[0];
-      Bn[at + sd] = f[1];
-    } else {
-      f[0] = Bn[at + f0*sd];
-      f[1] = -Bn[at + source(hi + 1)*sd];
-      f[2] = -Bn[at + source(hi + 2)*sd];
-      Bn[at + (f0 + 1)*sd] = f[1];
-      Bn[at + (f0 + 2)*sd] = f[2];
-    }
+    Bn[at + (upper ? f0 + 1 : 0)*sd] = f[upper ? 1 : 0];
+    Bn[at + (upper ? f0 + 2 : 1)*sd] = f[upper ? 2 : 1];
   } else {
     // outward from the boundary face with div B = 0; face areas of the uniform
     // Cartesian grid in 2D (Src/set_geometry.cpp:124,147)
     const double A[2] = {1.0*d.dy, d.dx*1.0};
-    f[upper ? 0 : 2] = Bn[at + (upper ? hi + 1 : lo)*sd];
 #pragma unroll
     for (int l = 0; l < 2; l++) {
       const int c = upper ? l : 1 - l;          // the ghost cell crossed, outward

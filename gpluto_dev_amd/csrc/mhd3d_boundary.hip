@@ -28,8 +28,8 @@ namespace {
 // layers in registers, so a direction is one launch without a barrier: three
 // launches a stage where a copy and a fill per side were twelve.  These
 // launches are latency, not bytes: 80 x 95 x 66, 81 us a stage in twelve,
-// 32 us in three.  The directions stay in turn: a later one reads the
-// ghosts of an earlier one in its corners.
+// 32 us in three, 26 us with every load before the first store.  The directions
+// stay in turn: a later one reads the ghosts of an earlier one in its corners.
 template <typename R>
 __global__ __launch_bounds__(256)
 void k_bnd_dir(Box3 g, int dir, int type_lo, int type_hi, R *__restrict__ V, double *__restrict__ Vs)
@@ -54,59 +54,66 @@ void k_bnd_dir(Box3 g, int dir, int type_lo, int type_hi, R *__restrict__ V, dou
   double *B1 = Vs + t1*N, *B2 = Vs + t2*N, *Bn = Vs + dir*N;
   const bool cell = a <= na - 2 && b <= nb - 2; // BOX_LOOP over the ghost box
   double e1[2][2], e2[2][2];                    // tangential faces on both ends of the ghost cells
+  constexpr int VAR[5] = {0, 1, 2, 3, 7};       // B1..3 are the field average below
+  R v[2][5];
+  const int f0 = upper ? hi + 1 : 0;            // the normal faces f0 .. f0 + 2 bound the two ghost cells
+  double f[3] = {0.0, 0.0, 0.0};
+  // every load before the first store: the arrays are filled in place, so a store
+  // would hold the loads after it back by a trip to memory each
 #pragma unroll
   for (int l = 0; l < 2; l++) {
-    const size_t cp = at + (g0 + l)*sd, cq = at + source(g0 + l)*sd;
-    // tangential components: one more face along the component (BOX{I,J,K}_LOOP)
-    if (b <= nb - 2) { e1[l][0] = B1[cq]; B1[cp] = e1[l][0]; }
-    if (a <= na - 2) { e2[l][0] = B2[cq]; B2[cp] = e2[l][0]; }
+    const size_t cq = at + source(g0 + l)*sd;
+    if (b <= nb - 2) e1[l][0] = B1[cq];
+    if (a <= na - 2) e2[l][0] = B2[cq];
     if (cell) {
       e1[l][1] = B1[cq + s1];
       e2[l][1] = B2[cq + s2];
-      constexpr int VAR[5] = {0, 1, 2, 3, 7};   // B1..3 are the field average below
 #pragma unroll
-      for (int q = 0; q < 5; q++) {
-        const int nv = VAR[q];
-        const R v = V[nv*N + cq];
-        // FlipSign (Src/boundary.cpp:840-925): a wall negates the normal velocity and field
-        V[nv*N + cp] = type == GPL_REFLECTIVE && nv == 1 + dir ? -v : v;
-      }
+      for (int q = 0; q < 5; q++) v[l][q] = V[VAR[q]*N + cq];
+    }
+  }
+  if (cell) {
+    if (type == GPL_PERIODIC) {
+#pragma unroll
+      for (int l = 0; l < 3; l++)
+        f[l] = !upper && l == 2 ? Bn[at + lo*sd] : Bn[at + source(f0 + l)*sd];
+    } else if (type == GPL_REFLECTIVE) {
+      // mirrored about the boundary face and negated: face i from i0 - i + 1 on
+      // the lower side, face i + 1 from i0 - i on the upper side
+      f[upper ? 0 : 2] = Bn[at + (upper ? f0 : lo)*sd];
+      f[upper ? 1 : 0] = -Bn[at + (upper ? source(hi + 1) : source(0) + 1)*sd];
+      f[upper ? 2 : 1] = -Bn[at + (upper ? source(hi + 2) : source(1) + 1)*sd];
+    } else {
+      f[upper ? 0 : 2] = Bn[at + (upper ? hi + 1 : lo)*sd];
+    }
+  }
+#pragma unroll
+  for (int l = 0; l < 2; l++) {
+    const size_t cp = at + (g0 + l)*sd;
+    // tangential components: one more face along the component (BOX{I,J,K}_LOOP)
+    if (b <= nb - 2) B1[cp] = e1[l][0];
+    if (a <= na - 2) B2[cp] = e2[l][0];
+    if (cell) {
+      // FlipSign (Src/boundary.cpp:840-925): a wall negates the normal velocity and field
+#pragma unroll
+      for (int q = 0; q < 5; q++)
+        V[VAR[q]*N + cp] = type == GPL_REFLECTIVE && VAR[q] == 1 + dir ? -v[l][q] : v[l][q];
     }
   }
   if (!cell) return;
-  // the normal faces f0 .. f0 + 2 that bound the two ghost cells
-  const int f0 = upper ? hi + 1 : 0;
-  double f[3];
   if (type == GPL_PERIODIC) {
     // BOX_LOOP on the lower side, BOXI/J/K_LOOP (one more face, the spare
     // layer) on the upper side
-#pragma unroll
-    for (int l = 0; l < 3; l++)
-      f[l] = !upper && l == 2 ? Bn[at + lo*sd] : Bn[at + source(f0 + l)*sd];
     Bn[at + f0*sd] = f[0];
     Bn[at + (f0 + 1)*sd] = f[1];
     if (upper) Bn[at + (f0 + 2)*sd] = f[2];
   } else if (type == GPL_REFLECTIVE) {
-    // mirrored about the boundary face and negated: face i from i0 - i + 1 on
-    // the lower side, face i + 1 from i0 - i on the upper side
-    if (!upper) {
-      f[0] = -Bn[at + (source(0) + 1)*sd];
-      f[1] = -Bn[at + (source(1) + 1)*sd];
-      f[2] = Bn[at + lo*sd];
-      Bn[at] = f[0];
-      Bn[at + sd] = f[1];
-    } else {
-      f[0] = Bn[at + f0*sd];
-      f[1] = -Bn[at + source(hi + 1)*sd];
-      f[2] = -Bn[at + source(hi + 2)*sd];
-      Bn[at + (f0 + 1)*sd] = f[1];
-      Bn[at + (f0 + 2)*sd] = f[2];
-    }
+    Bn[at + (upper ? f0 + 1 : 0)*sd] = f[upper ? 1 : 0];
+    Bn[at + (upper ? f0 + 2 : 1)*sd] = f[upper ? 2 : 1];
   } else {
     // outward from the boundary face with div B = 0; face areas of the uniform
     // Cartesian grid (Src/set_geometry.cpp:124,147,166)
     const double A[3] = {1.0*g.dy*g.dz, g.dx*1.0*g.dz, g.dx*g.dy*1.0};
-    f[upper ? 0 : 2] = Bn[at + (upper ? hi + 1 : lo)*sd];
 #pragma unroll
     for (int l = 0; l < 2; l++) {
       const int c = upper ? l : 1 - l;          // the ghost cell crossed, outward
