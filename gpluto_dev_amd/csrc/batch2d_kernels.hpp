@@ -189,10 +189,13 @@ void k2_sweepx(Batch2dBufs<R> b, R gamma, int want_cdt)
 }
 
 // ---------------------------------------------------------------------------
-// y sweep + RK combination of U + C_dt maximum per item
+// y sweep + RK combination of U + C_dt maximum per item.  FP64 is held to two
+// wavefronts per SIMD: HLLD is 2 registers over (2 spilled, 12 B), and a batch that
+// fills the chip needs the second one (64 boxes, 3.2 M cells: step 1.265 -> 1.124
+// ms); one box that does not pays for the spill (512^2 107.3 -> 108.7 us).
 // ---------------------------------------------------------------------------
 template <typename R, int LIM, int SOLVER>
-__global__ __launch_bounds__(256)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 2 : 1)))
 void k2_sweepy(Batch2dBufs<R> b, int L, RKW w, int first_stage, int want_cdt, R gamma)
 {
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
