@@ -25,6 +25,7 @@
 //  finish: CT_Update (ct_update.cpp:181-258), the staggered RK combination
 //    (rk_step.cpp:378-385,540-552), B1/B2 = face averages
 //    (ct_field_average.cpp:182-184) and ConsToPrim (mappers3D.cpp:104-194).
+//    One launch with the EMF while its blocks are all in flight at once.
 // This header holds the templates; batch2d_fp64.hip and batch2d_mixed.hip
 // instantiate them with their own compiler flags.
 #pragma once

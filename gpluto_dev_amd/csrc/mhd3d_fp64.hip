@@ -1,5 +1,6 @@
 // FP64 drop-in instantiation of the 3D MHD stage kernels.  Built with
 // -ffp-contract=off so every product and sum is rounded as in the reference.
+// The RMHD and van Leer sweeps and the EMFs are in mhd3d_fp64_nohoist.hip.
 #include "mhd3d_kernels.hpp"
 
 namespace gpl {

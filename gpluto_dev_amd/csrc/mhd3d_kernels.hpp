@@ -19,13 +19,14 @@
 // Two kernel paths compute the same numbers:
 //  * fused (nx <= 512): one kernel per sweep direction reconstructs, solves
 //    the Riemann problem and accumulates the flux divergence in place, with no
-//    interface flux written to HBM -- x: one block per periodic x-row, the row
+//    interface flux written to HBM -- x: one or more periodic x-rows per block,
 //    staged in LDS; y, z: each thread marches a register window along the
-//    column; the z kernel also applies the RK combination of U;
+//    column, or (small FP64 boxes) a block holds whole columns in LDS; the z
+//    kernel also applies the RK combination of U;
 //  * split: one thread per interface, fluxes through HBM, a separate
 //    divergence/RK kernel (any box).
-// This header holds the templates; mhd3d_fp64.hip and mhd3d_mixed.hip
-// instantiate them with their own compiler flags.
+// This header holds the templates; mhd3d_fp64.hip, mhd3d_fp64_nohoist.hip and
+// mhd3d_mixed.hip instantiate them with their own compiler flags.
 #pragma once
 #include <type_traits>
 #include "c2p_net.hpp"
