@@ -107,24 +107,69 @@ HostCopy::~HostCopy()
   for (hipEvent_t e : done) if (e) (void)hipEventDestroy(e);
 }
 
-int HostCopy::reserve(size_t slot, bool gather)
+bool HostCopy::reserve(size_t slot, bool gather)
 {
   const size_t want = kSlots*slot*sizeof(double);
   for (int q = 0; q < kSlots; q++)
-    if (!done[q] && hipEventCreateWithFlags(&done[q], hipEventDisableTiming) != hipSuccess) return GPL_EHIP;
+    if (!done[q] && hipEventCreateWithFlags(&done[q], hipEventDisableTiming) != hipSuccess) {
+      done[q] = nullptr;
+      return false;
+    }
   if (pin_cap < want) {
     if (pin) (void)hipHostFree(pin);
     pin = nullptr;
     pin_cap = 0;
-    if (hipHostMalloc((void **)&pin, want, hipHostMallocDefault) != hipSuccess) { pin = nullptr; return GPL_ENOMEM; }
+    if (hipHostMalloc((void **)&pin, want, hipHostMallocDefault) != hipSuccess) { pin = nullptr; return false; }
     pin_cap = want;
   }
   if (gather && dev_cap < want) {
     if (dev) (void)hipFree(dev);
     dev = nullptr;
     dev_cap = 0;
-    if (hipMalloc((void **)&dev, want) != hipSuccess) { dev = nullptr; return GPL_ENOMEM; }
+    if (hipMalloc((void **)&dev, want) != hipSuccess) { dev = nullptr; return false; }
     dev_cap = want;
+  }
+  return true;
+}
+
+int HostCopy::fetch_whole(const FieldGeom &g, const std::vector<FieldOut> &out, hipStream_t s)
+{
+  const size_t n = (size_t)g.n[0]*g.n[1]*g.n[2];
+  for (size_t q = 0; q < out.size();) {
+    size_t run = 1;                            // fields that follow one another on both sides
+    while (q + run < out.size() && out[q + run].dst == out[q].dst + run*n &&
+           (const double *)out[q + run].src == (const double *)out[q].src + run*n)
+      run++;
+    if (hipMemcpyAsync(out[q].dst, (const double *)out[q].src + g.off, run*n*sizeof(double),
+                       hipMemcpyDeviceToHost, s) != hipSuccess)
+      return GPL_EHIP;
+    q += run;
+  }
+  return hipStreamSynchronize(s) == hipSuccess ? 0 : GPL_EHIP;
+}
+
+int HostCopy::fetch_rows(const FieldGeom &g, const std::vector<FieldOut> &out, hipStream_t s)
+{
+  // whole stored rows of a plane at a time, about 2 MiB or one row
+  const int most = (int)(kRows/(size_t)g.sx), rows = most < 1 ? 1 : (most < g.n[1] ? most : g.n[1]);
+  std::vector<double> buf((size_t)rows*g.sx);
+  for (const FieldOut &f : out) {
+    const size_t es = f.f32 ? sizeof(float) : sizeof(double);
+    for (int k = 0; k < g.n[2]; k++)
+      for (int j0 = 0; j0 < g.n[1]; j0 += rows) {
+        const int m = g.n[1] - j0 < rows ? g.n[1] - j0 : rows;
+        const size_t at = g.off + (size_t)g.sx*((size_t)(j0 + g.lo[1]) + (size_t)g.sy*(k + g.lo[2]));
+        if (hipMemcpyAsync(buf.data(), (const char *)f.src + at*es, (size_t)m*g.sx*es, hipMemcpyDeviceToHost,
+                           s) != hipSuccess ||
+            hipStreamSynchronize(s) != hipSuccess)
+          return GPL_EHIP;
+        for (int j = 0; j < m; j++) {
+          double *d = f.dst + ((size_t)k*g.n[1] + j0 + j)*g.n[0];
+          const size_t o = (size_t)j*g.sx + g.lo[0];
+          if (f.f32) for (int i = 0; i < g.n[0]; i++) d[i] = (double)((const float *)buf.data())[o + i];
+          else       memcpy(d, buf.data() + o, (size_t)g.n[0]*sizeof(double));
+        }
+      }
   }
   return 0;
 }
@@ -138,23 +183,14 @@ int HostCopy::fetch(const FieldGeom &g, const std::vector<FieldOut> &out, hipStr
   // a small state goes through all slots at once, with one wait, a larger one in
   // slots of an eighth of it, 16 MiB at most
   const bool once = total <= (size_t(1) << 17);
-  if (once && !gather) {
-    // up to a megabyte the runtime's own staging is as fast and needs no buffer
-    for (size_t q = 0; q < out.size();) {
-      size_t run = 1;                          // fields that follow one another on both sides
-      while (q + run < out.size() && out[q + run].dst == out[q].dst + run*n &&
-             (const double *)out[q + run].src == (const double *)out[q].src + run*n)
-        run++;
-      if (hipMemcpyAsync(out[q].dst, (const double *)out[q].src + g.off, run*n*sizeof(double),
-                         hipMemcpyDeviceToHost, s) != hipSuccess)
-        return GPL_EHIP;
-      q += run;
-    }
-    return hipStreamSynchronize(s) == hipSuccess ? 0 : GPL_EHIP;
-  }
+  // up to a megabyte the runtime's own staging is as fast and needs no buffer
+  if (once && !gather) return fetch_whole(g, out, s);
   size_t slot = once ? (total + kSlots - 1)/kSlots : (total + 7)/8;
   if (slot > kChunk) slot = kChunk;
-  if (int rc = reserve(slot, gather)) return rc;
+  if (!reserve(slot, gather)) {
+    (void)hipGetLastError();                   // dealt with here: not for a later check to find
+    return gather ? fetch_rows(g, out, s) : fetch_whole(g, out, s);
+  }
   const size_t hold = once ? slot*kSlots : slot;   // doubles of a group
   // groups of pieces, one group per slot; without a gather, fields that follow
   // one another on both sides make one piece

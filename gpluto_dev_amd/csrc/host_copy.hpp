@@ -10,7 +10,9 @@
 //
 // The buffers belong to one context (no sharing between contexts or threads),
 // are allocated at its first transfer, at most kSlots chunks of 16 MiB pinned and,
-// if a gather is needed, as much on the device, and are freed with it.
+// if a gather is needed, as much on the device, and are freed with it.  Where they
+// cannot be had (a full card, a limit on locked memory) the transfer takes neither:
+// pageable copies, unpacked on the host where a gather would be needed.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -38,14 +40,17 @@ class HostCopy {
 public:
   ~HostCopy();
   // Every field of `out` to the host, behind the work already on the stream;
-  // returns when the arrays are filled.  0, GPL_ENOMEM or GPL_EHIP.
+  // returns when the arrays are filled.  0 or GPL_EHIP.
   int fetch(const FieldGeom &g, const std::vector<FieldOut> &out, hipStream_t s);
   size_t device_bytes() const { return dev_cap; }
 
 private:
   static constexpr int kSlots = 4;
   static constexpr size_t kChunk = size_t(1) << 21;   // doubles per slot at most: 16 MiB
-  int reserve(size_t chunk, bool gather);
+  static constexpr size_t kRows = size_t(1) << 18;    // doubles of fetch_rows' host buffer
+  bool reserve(size_t chunk, bool gather);
+  int fetch_whole(const FieldGeom &g, const std::vector<FieldOut> &out, hipStream_t s);   // no gather needed
+  int fetch_rows(const FieldGeom &g, const std::vector<FieldOut> &out, hipStream_t s);
   double *pin = nullptr, *dev = nullptr;
   size_t pin_cap = 0, dev_cap = 0;                     // bytes
   hipEvent_t done[kSlots] = {};

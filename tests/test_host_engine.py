@@ -1,0 +1,74 @@
+"""The library's host side (C ABI, engines, transfers) on the CPU: built with
+host memory for device memory and recorded kernel launches (tests/host/
+host_engine.cpp), so that what an engine allocates, copies and asks its kernels
+for can be checked without a GPU."""
+import ctypes as C
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+from gpluto_dev_amd import _lib
+from gpluto_dev_amd.stage import Definitions, RuntimeSetup, StageUpdate
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LIB = os.path.join(ROOT, "tests", "_build", "libhost_engine.so")
+UNLIMITED = 2 ** 64 - 1
+WALLS = ("outflow", "reflective", "periodic", "periodic", "outflow", "outflow")
+
+
+@pytest.fixture(scope="module")
+def he():
+    subprocess.run(["make", "-s", "-C", os.path.join(ROOT, "tests", "host")], check=True)
+    was = _lib.LIB_PATH, _lib._lib
+    _lib.LIB_PATH, _lib._lib = LIB, None
+    L = _lib.load()
+    L.he_limits.argtypes = [C.c_size_t, C.c_size_t]
+    L.he_held.restype = C.c_size_t
+    yield L
+    _lib.LIB_PATH, _lib._lib = was
+
+
+def _domain(n, physics="MHD", precision="fp64", sides=(), **kw):
+    dims = 1 if n[1] == 1 else 2 if n[2] == 1 else 3
+    return StageUpdate(Definitions(physics=physics, dimensions=dims, **kw),
+                       RuntimeSetup(n=n, sides=sides, solver="hllc" if physics == "HD" else "hlld"),
+                       precision=precision)
+
+
+def _fill(d, seed=3):
+    rng = np.random.default_rng(seed)
+    sh = tuple(reversed(d.n))
+    vs = None if not d.mhd else 0.1*rng.random((d._nfaces,) + sh)
+    d.upload(1.0 + 0.1*rng.random((d.nvar,) + sh), vs)
+
+
+@pytest.mark.parametrize("n,physics,precision,sides", [
+    ((41, 43, 47), "MHD", "fp64", ()),               # whole FP64 fields
+    ((9, 8, 7), "MHD", "mixed", ()),                 # FP32: unpacked on the host
+    ((41, 43, 47), "MHD", "mixed", ()),
+    ((23, 30, 31), "MHD", "fp64", WALLS),            # ghost layers
+    ((23, 30, 31), "MHD", "mixed", WALLS),
+    ((517, 530, 1), "MHD", "mixed", WALLS),          # a plane in several pieces
+    ((60, 61, 50), "HD", "fp64", ())])
+def test_download_without_staging_memory(he, n, physics, precision, sides):
+    """A download needs neither pinned nor device memory of its own: what the
+    buffers of its usual path cannot get, it does without, and leaves no error
+    behind."""
+    d = _domain(n, physics, precision, sides)
+    _fill(d)
+    want = d.download()
+    d.close()
+    for pinned in (0, 1 << 20, UNLIMITED):
+        d = _domain(n, physics, precision, sides)
+        _fill(d)
+        he.he_limits(he.he_held(0), pinned)
+        try:
+            got = d.download()
+        finally:
+            he.he_limits(UNLIMITED, UNLIMITED)
+        assert he.he_last_error() == 0
+        d.close()
+        assert all(a is None and b is None or np.array_equal(a, b) for a, b in zip(got, want))
+    assert he.he_held(0) == 0 and he.he_held(1) == 0
