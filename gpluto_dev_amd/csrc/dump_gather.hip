@@ -80,12 +80,13 @@ void k_field_gather(FieldGeom g, const R *__restrict__ src, size_t e0, size_t co
 
 }  // namespace
 
-void launch_field_gather(const FieldGeom &g, const void *src, bool f32, size_t e0, size_t count,
-                         double *dst, hipStream_t s)
+hipError_t launch_field_gather(const FieldGeom &g, const void *src, bool f32, size_t e0, size_t count,
+                               double *dst, hipStream_t s)
 {
-  const dim3 nb((unsigned)((count + 255)/256));
-  if (f32) hipLaunchKernelGGL((k_field_gather<float>), nb, dim3(256), 0, s, g, (const float *)src, e0, count, dst);
-  else     hipLaunchKernelGGL((k_field_gather<double>), nb, dim3(256), 0, s, g, (const double *)src, e0, count, dst);
+  // the launch's own result: the thread's last error may be an older call's
+  void *args[] = {const_cast<FieldGeom *>(&g), &src, &e0, &count, &dst};
+  const void *kernel = f32 ? (const void *)k_field_gather<float> : (const void *)k_field_gather<double>;
+  return hipLaunchKernel(kernel, dim3((unsigned)((count + 255)/256)), dim3(256), args, 0, s);
 }
 
 }  // namespace gpl

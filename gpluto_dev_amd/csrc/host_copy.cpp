@@ -215,15 +215,14 @@ int HostCopy::fetch(const FieldGeom &g, const std::vector<FieldOut> &out, hipStr
     double *hp = pin + (size_t)(k % kSlots)*slot, *dp = dev + (size_t)(k % kSlots)*slot;
     size_t sum = 0;
     for (const Piece &p : groups[k]) {
-      if (gather) launch_field_gather(g, p.src, p.f32, p.e0, p.count, dp + p.at, s);
-      else if (hipMemcpyAsync(hp + p.at, (const double *)p.src + g.off + p.e0, p.count*sizeof(double),
-                              hipMemcpyDeviceToHost, s) != hipSuccess)
-        return false;
+      const hipError_t e = gather
+          ? launch_field_gather(g, p.src, p.f32, p.e0, p.count, dp + p.at, s)
+          : hipMemcpyAsync(hp + p.at, (const double *)p.src + g.off + p.e0, p.count*sizeof(double),
+                           hipMemcpyDeviceToHost, s);
+      if (e != hipSuccess) return false;
       sum += p.count;
     }
-    if (gather && (hipGetLastError() != hipSuccess ||
-                   hipMemcpyAsync(hp, dp, sum*sizeof(double), hipMemcpyDeviceToHost, s) != hipSuccess))
-      return false;
+    if (gather && hipMemcpyAsync(hp, dp, sum*sizeof(double), hipMemcpyDeviceToHost, s) != hipSuccess) return false;
     return hipEventRecord(done[k % kSlots], s) == hipSuccess;
   };
   bool ok = true;

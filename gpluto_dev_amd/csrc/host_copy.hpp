@@ -57,7 +57,7 @@ private:
 };
 
 // dst[t] = element e0 + t of the field, in FP64
-void launch_field_gather(const FieldGeom &g, const void *src, bool f32, size_t e0, size_t count,
-                         double *dst, hipStream_t s);
+hipError_t launch_field_gather(const FieldGeom &g, const void *src, bool f32, size_t e0, size_t count,
+                               double *dst, hipStream_t s);
 
 }  // namespace gpl

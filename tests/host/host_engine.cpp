@@ -188,8 +188,8 @@ template void launch_diagnostics<double>(const DiagBox &, const double *, const 
 template void launch_diagnostics<float>(const DiagBox &, const float *, const double *, double *, double *, hipStream_t);
 int net_pack_upload(const float *, float *, NetPack *, hipStream_t) { return GPL_EUNSUPPORTED; }
 
-void launch_field_gather(const FieldGeom &g, const void *src, bool f32, size_t e0, size_t count, double *dst,
-                         hipStream_t)
+hipError_t launch_field_gather(const FieldGeom &g, const void *src, bool f32, size_t e0, size_t count, double *dst,
+                               hipStream_t)
 {
   for (size_t t = 0; t < count; t++) {
     const size_t e = e0 + t, r = e / g.n[0];
@@ -198,6 +198,7 @@ void launch_field_gather(const FieldGeom &g, const void *src, bool f32, size_t e
                      (size_t)g.sx*((size_t)(j + g.lo[1]) + (size_t)g.sy*(k + g.lo[2]));
     dst[t] = f32 ? (double)((const float *)src)[o] : ((const double *)src)[o];
   }
+  return hipSuccess;
 }
 
 }  // namespace gpl

@@ -72,3 +72,19 @@ def test_download_without_staging_memory(he, n, physics, precision, sides):
         d.close()
         assert all(a is None and b is None or np.array_equal(a, b) for a, b in zip(got, want))
     assert he.he_held(0) == 0 and he.he_held(1) == 0
+
+
+@pytest.mark.parametrize("precision,sides", [("mixed", ()), ("fp64", WALLS)])
+def test_download_after_an_unrelated_error(he, precision, sides):
+    """An error that an earlier HIP call of the thread left behind is not the
+    download's."""
+    d = _domain((23, 30, 31), precision=precision, sides=sides)
+    _fill(d)
+    want = d.download()
+    he.he_set_last_error(1)                          # hipErrorInvalidValue
+    try:
+        got = d.download()
+    finally:
+        he.he_set_last_error(0)
+    d.close()
+    assert all(np.array_equal(a, b) for a, b in zip(got, want))
