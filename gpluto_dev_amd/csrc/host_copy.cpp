@@ -2,6 +2,9 @@
 #include "host_copy.hpp"
 #include "../../include/gpluto_amd.h"
 
+#include <sched.h>
+
+#include <algorithm>
 #include <atomic>
 #include <condition_variable>
 #include <cstring>
@@ -12,15 +15,24 @@ namespace gpl {
 
 namespace {
 
+// cores this thread may run on
+int cores()
+{
+  cpu_set_t set;
+  return sched_getaffinity(0, sizeof(set), &set) == 0 ? CPU_COUNT(&set) : 1;
+}
+
 // Moves chunks from pinned memory to the caller's arrays: the calling thread and
-// up to kHelpers more, each taking pieces of the chunk on offer.  Helpers that
-// cannot be started are simply missing.
+// up to kHelpers more, each taking pieces of the chunk on offer.  No more threads
+// than cores: one without a core of its own only takes turns with the others.
+// Helpers that cannot be started are simply missing.
 class Movers {
 public:
   explicit Movers(size_t total)
   {
     // a helper pays for itself from some megabytes on
-    const int want = total >= (size_t(32) << 20) ? kHelpers : (total >= (size_t(4) << 20) ? 2 : 0);
+    const int most = total >= (size_t(32) << 20) ? kHelpers : (total >= (size_t(4) << 20) ? 2 : 0);
+    const int want = most == 0 ? 0 : std::min(most, cores() - 1);
     try {
       helpers.reserve(want);
       for (int q = 0; q < want; q++) helpers.emplace_back([this] { serve(); });

@@ -119,7 +119,9 @@ int gpl_upload(gpl_ctx *ctx, const double *vc, const double *const *vs, int layo
  * ACTIVE: a state above 1 MiB goes through pinned host memory, a mixed-precision
  * or ghost-layered one through device memory too, up to 64 MiB of each, which
  * the first such call allocates and gpl_destroy frees; where they cannot be
- * had the call copies without them, more slowly. */
+ * had the call copies without them, more slowly.  Above 4 MiB up to seven
+ * helper threads, no more than the calling thread's spare cores, move the data
+ * to the caller's arrays; they end with the call. */
 int gpl_download(gpl_ctx *ctx, double *vc, double *const *vs, double *uc, int layout);
 
 /* The step state the main loop keeps in timeStep and g_stepNumber

@@ -88,3 +88,25 @@ def test_download_after_an_unrelated_error(he, precision, sides):
         he.he_set_last_error(0)
     d.close()
     assert all(np.array_equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("cores,helpers", [(1, 0), (2, 1), (4, 3)])
+def test_download_helpers_stay_within_the_cores(he, cores, helpers):
+    """A large download starts no more helper threads than the calling thread
+    has cores to spare."""
+    mine = os.sched_getaffinity(0)
+    if len(mine) < cores:
+        pytest.skip("too few cores")
+    d = _domain((80, 81, 82))                        # 100 MB
+    _fill(d)
+    want = d.download()
+    before = len(os.listdir("/proc/self/task"))
+    he.he_threads(1)
+    os.sched_setaffinity(0, sorted(mine)[:cores])
+    try:
+        got = d.download()
+    finally:
+        os.sched_setaffinity(0, mine)
+    d.close()
+    assert he.he_threads(1) - before == helpers
+    assert all(np.array_equal(a, b) for a, b in zip(got, want))
