@@ -25,13 +25,14 @@ public:
   // stage UA); 1D, one launch a step, ping-pongs both across steps
   double *VA = nullptr, *VB = nullptr, *UA = nullptr, *UB = nullptr;
   double *cur_v = nullptr, *cur_u = nullptr;
+  double *dU = nullptr, *Cdt = nullptr;   // stages by direction only
   double *cdt_part = nullptr;
   unsigned *arrived = nullptr;   // arrival counters of the launch that ends a step
   double *diag = nullptr;     // diagnostics partials (DIAG_BLOCKS rows) and result row
 
   ~HdEngine() override
   {
-    void *ptrs[] = {VA, VB, UA, UB, cdt_part, diag};
+    void *ptrs[] = {VA, VB, UA, UB, dU, Cdt, cdt_part, diag};
     for (void *p : ptrs) if (p) (void)hipFree(p);
   }
 
@@ -57,6 +58,10 @@ public:
     rc |= dev_alloc(bytes, (void **)&UA, 5*n*sizeof(double) + HD_ARRIVED*sizeof(unsigned));
     arrived = (unsigned *)(UA + 5*n);
     rc |= dev_alloc(bytes, (void **)&UB, 5*n*sizeof(double));
+    if (hd_by_direction(g)) {
+      rc |= dev_alloc(bytes, (void **)&dU, 5*n*sizeof(double));
+      rc |= dev_alloc(bytes, (void **)&Cdt, n*sizeof(double));
+    }
     rc |= dev_alloc(bytes, (void **)&cdt_part, (size_t)hd_blocks(g, nstages())*sizeof(double));
     rc |= dev_alloc(bytes, (void **)&diag, (size_t)(DIAG_BLOCKS + 1)*DIAG_MAXQ*sizeof(double));
     cur_v = VA;
@@ -130,7 +135,7 @@ public:
     HdStep ctl = {env.ctl, arrived, cfg.cfl, cfg.cfl_max_var, advance_dt, 1};
     if (g.dims == 1) {
       double *uo = cur_u == UA ? UB : UA;
-      const HdBufs b = {in, out, cur_u, cur_u, uo, cdt_part, env.err, {zone_rep(0), zone_rep(1), zone_rep(2)}};
+      const HdBufs b = {in, out, cur_u, cur_u, uo, dU, Cdt, cdt_part, env.err, {zone_rep(0), zone_rep(1), zone_rep(2)}};
       if (t) t->begin(K_HD_X);
       hd_launch_step1d(b, g, ctl, nst, cfg.limiter, cfg.solver, cfg.gamma, cfg.small_rho, cfg.small_prs,
                        env.stream);
@@ -143,13 +148,28 @@ public:
     for (int st = 1; st <= nst; st++) {
       const RKW w = st == 1 ? w1 : (st == 2 ? w2 : w3);
       const ZoneRep z = zone_rep(st - 1);
-      const HdBufs b = {in, out, st == 1 ? UA : UB, UA, st == nst ? UA : UB, cdt_part, env.err, {z, z, z}};
+      const HdBufs b = {in, out, st == 1 ? UA : UB, UA, st == nst ? UA : UB, dU, Cdt, cdt_part, env.err, {z, z, z}};
       ctl.ends_step = st == nst;
-      if (t) t->begin(kid);
-      hd_launch_stage(b, g, ctl, w, st == 1, st == 1, cfg.limiter, cfg.solver, cfg.gamma, cfg.small_rho,
-                      cfg.small_prs, env.stream);
-      if (t) t->end(kid);
+      if (dU) {
+        for (int d = 0; d < g.dims; d++) {
+          if (t) t->begin(K_HD_X + d);
+          hd_launch_sweep(d, b, g, env.ctl, w, st == 1, st == 1, cfg.limiter, cfg.solver, cfg.gamma,
+                          cfg.small_rho, cfg.small_prs, env.stream);
+          if (t) t->end(K_HD_X + d);
+        }
+      } else {
+        if (t) t->begin(kid);
+        hd_launch_stage(b, g, ctl, w, st == 1, st == 1, cfg.limiter, cfg.solver, cfg.gamma, cfg.small_rho,
+                        cfg.small_prs, env.stream);
+        if (t) t->end(kid);
+      }
       double *tmp = in; in = out; out = tmp;
+    }
+    if (dU) {
+      if (t) t->begin(K_DT);
+      launch_dt(cdt_part, hd_blocks(g, nst), (double)g.dims, env.ctl, cfg.cfl, cfg.cfl_max_var, advance_dt,
+                env.stream);
+      if (t) t->end(K_DT);
     }
     cur_v = in;
   }

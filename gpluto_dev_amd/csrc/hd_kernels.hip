@@ -14,11 +14,12 @@
 //    lane shuffle, through LDS or in registers, and dUc = rhs_x + rhs_y + rhs_z (update_stage.cpp:173-184,
 //    272-284, 369-380), the RK combination (rk_step.cpp:366-374,509-518) and
 //    ConsToPrim3D (mappers3D.cpp:104-194) follow in registers.
+//  * 2D and 3D boxes too narrow to fill those kernels' lanes (hd_by_direction): one
+//    launch per direction (k_hd_sweep), a thread per cell.
 //  * 1D (k_hd_step1d): a whole step is one launch; a block recomputes the cells
 //    that the later stages need beyond its own.
 #include "hd.hpp"
 #include "physics.hpp"
-#include <cmath>
 
 namespace gpl {
 
@@ -150,7 +151,7 @@ __device__ void step_control(const HdStep &st, double dt, int nparts, int dims, 
 // reduces the partials that the first stage's launch left.  No block waits
 // for another.
 // ---------------------------------------------------------------------------
-constexpr int TX = 64, NW = 8, TY = NW - 1;
+constexpr int TX = kHdCols, TY = kHdRows, NW = TY + 1;
 constexpr int SW = TX + 4, SH = NW + 3;        // staged columns i0-2 .. i0+65, rows j0-2 .. j0+8
 
 template <int LIM, int SOLVER, typename OFF>
@@ -521,6 +522,88 @@ void k_hd_stage2d(HdBox g, int L, HdBufs b, HdStep st, RKW w, int first_stage, i
 }
 
 // ---------------------------------------------------------------------------
+// One direction of a 2D or 3D stage, one thread per cell: it reconstructs cells
+// -1, 0, +1, solves both faces of its cell and forms rhs; dU and Cdt carry the sums
+// to the last direction, which applies the RK combination and ConsToPrim.  Every face
+// is solved twice and dU, Cdt go through memory, but no lane is idle however
+// narrow the box; hd_by_direction draws the line to the kernels above.
+// ---------------------------------------------------------------------------
+template <int D, bool LAST, int LIM, int SOLVER>
+__global__ __launch_bounds__(256)
+void k_hd_sweep(HdBox g, HdBufs b, const StepCtl *__restrict__ ctl, RKW w, int first_stage, int want_cdt,
+                double gamma, double small_rho, double small_prs)
+{
+  __shared__ double red[4];
+  const int c = blockIdx.x*blockDim.x + threadIdx.x;
+  double cdt_max = -1.0;
+  uint32_t e = 0;
+  if (c < g.ncell) {
+    const size_t n = (size_t)g.ncell;
+    const int nd = D == 0 ? g.nx : (D == 1 ? g.ny : g.nz);
+    const int sd = D == 0 ? 1 : (D == 1 ? g.nx : g.nx*g.ny);
+    const int p = D == 0 ? c % g.nx : (D == 1 ? (c/g.nx) % g.ny : c/(g.nx*g.ny));
+    double v[5][5];                 // [cell -2..+2][variable]
+#pragma unroll
+    for (int o = 0; o < 5; o++) {
+      bool flip;
+      const int i = c + (hd_source(p + o - 2, nd, g.lo[D], g.hi[D], flip) - p)*sd;
+#pragma unroll
+      for (int q = 0; q < 5; q++) v[o][q] = b.Vin[q*n + i];
+      if (flip) v[o][1 + D] = -v[o][1 + D];
+    }
+    double lo_l[5], lo_r[5], hi_l[5], hi_r[5];
+#pragma unroll
+    for (int q = 0; q < 5; q++) {
+      const double d0 = plm_slope<double, LIM>(v[1][q], v[2][q], v[3][q]);
+      lo_l[q] = v[1][q] + 0.5*plm_slope<double, LIM>(v[0][q], v[1][q], v[2][q]);
+      lo_r[q] = v[2][q] - 0.5*d0;
+      hi_l[q] = v[2][q] + 0.5*d0;
+      hi_r[q] = v[3][q] - 0.5*plm_slope<double, LIM>(v[2][q], v[3][q], v[4][q]);
+    }
+    FaceFlux<double> lo, hi;
+    hd_riemann<D, SOLVER>(lo_l, lo_r, gamma, lo);
+    hd_riemann<D, SOLVER>(hi_l, hi_r, gamma, hi);
+    e |= lo.err | hi.err;           // a face's bits come from both of its cells
+    const double ddx = D == 0 ? g.dx : (D == 1 ? g.dy : g.dz), dtdx = ctl->dt/ddx;
+    double du[5];
+#pragma unroll
+    for (int q = 0; q < 5; q++) {
+      double r = -dtdx*(hi.f[q] - lo.f[q]);
+      r += 0.0;
+      du[q] = D == 0 ? r : b.dU[q*n + c] + r;
+    }
+    double cd = 0.0;
+    if (want_cdt) {
+      cd = 0.5*(rmax(rabs(lo.Sl), rabs(lo.Sr)) + rmax(rabs(hi.Sl), rabs(hi.Sr)))/ddx;   // rhs.cpp:523,756,981
+      if (D > 0) cd = b.Cdt[c] + cd;
+    }
+    if (!LAST) {
+#pragma unroll
+      for (int q = 0; q < 5; q++) b.dU[q*n + c] = du[q];
+      if (want_cdt) b.Cdt[c] = cd;
+    } else {
+      double u[5], vn[5];
+#pragma unroll
+      for (int q = 0; q < 5; q++) {
+        const size_t o = q*n + c;
+        u[q] = first_stage ? b.Uin[o] + w.wR*du[q] : w.w0*b.U0[o] + w.w1*b.Uin[o] + w.wR*du[q];
+      }
+      const uint32_t ce = hd_cons_to_prim(u, gamma - 1.0, small_rho, small_prs, vn);
+      e |= ce;
+      zone_report(b.zr[0], c, ce);
+#pragma unroll
+      for (int q = 0; q < 5; q++) { b.Uout[q*n + c] = u[q]; b.Vout[q*n + c] = vn[q]; }
+      cdt_max = cd;
+    }
+  }
+  report_bits(b.err, e);
+  if (LAST && want_cdt) {
+    const double m = block_max(cdt_max, red);
+    if (threadIdx.x == 0) b.cdt_part[blockIdx.x] = m;
+  }
+}
+
+// ---------------------------------------------------------------------------
 // A whole step of a 1D box: NST stages with everything between them in
 // registers and LDS.  A block's B threads hold its own cells and 2 NST more on
 // either side; after stage s the outer 2 s cells of either side are no longer
@@ -637,40 +720,11 @@ void k_hd_step1d(HdBox g, HdBufs b, HdStep st, double gamma, double small_rho, d
     });
 }
 
-// threads of a 1D block
-int block1d(const HdBox &g) { return g.nx <= (1 << 14) ? 64 : 256; }
-
-// Planes per block of a 3D march, rows per wave of a 2D one; the longest of
-// lengths within 5%.
-//  3D: the shortest rounds of one block per CU, a segment costing its planes and
-//    about half of one more for its first face (128x96x112, us a stage: 149 at one
-//    plane, 123 at 8, 103 at the 13 of one round).
-//  2D: a wave solves 2 L + 1 faces in turn behind about five faces' worth of
-//    launch and first loads; more waves than SIMDs cost about the root of their
-//    number (511x333, us a stage at L = 1, 2, 3, 4, 8: 22, 21, 19, 23, 33;
-//    512^2: 28, 26, 24, 28, 31; 2000x1800: 255, 205, 195, 195, 194).
-int march_cells(const HdBox &g)
-{
-  if (g.dims == 1) return 1;
-  const bool d3 = g.dims == 3;
-  const long long across = d3 ? (long long)((g.nx + TX - 1)/TX)*((g.ny + TY - 1)/TY) : (g.nx + 62)/63;
-  const int n = d3 ? g.nz : g.ny;
-  int best = 32;
-  double tbest = 0.0;
-  for (int l = 32; l >= 1; l--) {
-    const long long items = across*((n + l - 1)/l);
-    const double per = (double)items/1024;
-    const double t = d3 ? (double)((items + 255)/256)*(l + 0.5) : (2*l + 6)*(per > 1.0 ? std::sqrt(per) : 1.0);
-    if (l == 32 || t < 0.95*tbest) { best = l; tbest = t; }
-  }
-  return best;
-}
-
 template <int LIM, int SOLVER>
 void stage_t(const HdBufs &b, const HdBox &g, const HdStep &st, RKW w, int first_stage, int want_dt,
              double gamma, double small_rho, double small_prs, hipStream_t s)
 {
-  const int nb = hd_blocks(g, 0), L = march_cells(g);
+  const int nb = hd_blocks(g, 0), L = hd_march_cells(g);
   auto go = [&](auto kernel, int threads) {
     hipLaunchKernelGGL(kernel, dim3(nb), dim3(threads), 0, s, g, L, b, st, w, first_stage, want_dt, nb,
                        gamma, small_rho, small_prs);
@@ -682,12 +736,26 @@ void stage_t(const HdBufs &b, const HdBox &g, const HdStep &st, RKW w, int first
     wide ? go(k_hd_stage3d<LIM, SOLVER, size_t>, 64*NW) : go(k_hd_stage3d<LIM, SOLVER, unsigned>, 64*NW);
 }
 
+template <int LIM, int SOLVER>
+void sweep_t(int dir, const HdBufs &b, const HdBox &g, const StepCtl *ctl, RKW w, int first_stage, int want_dt,
+             double gamma, double small_rho, double small_prs, hipStream_t s)
+{
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(hd_blocks(g, 0)), dim3(hd_sweep_block(g)), 0, s, g, b, ctl, w, first_stage,
+                       want_dt, gamma, small_rho, small_prs);
+  };
+  if (dir == 0)         go(k_hd_sweep<0, false, LIM, SOLVER>);
+  else if (dir == 2)    go(k_hd_sweep<2, true, LIM, SOLVER>);
+  else if (g.dims == 2) go(k_hd_sweep<1, true, LIM, SOLVER>);
+  else                  go(k_hd_sweep<1, false, LIM, SOLVER>);
+}
+
 template <int LIM, int SOLVER, int NST>
 void step1d_t(const HdBufs &b, const HdBox &g, const HdStep &st, double gamma, double small_rho,
               double small_prs, hipStream_t s)
 {
   const int nb = hd_blocks(g, NST);
-  if (block1d(g) == 64)
+  if (hd_block1d(g) == 64)
     hipLaunchKernelGGL((k_hd_step1d<LIM, SOLVER, NST, 64>), dim3(nb), dim3(64), 0, s, g, b, st, gamma,
                        small_rho, small_prs);
   else
@@ -696,17 +764,6 @@ void step1d_t(const HdBufs &b, const HdBox &g, const HdStep &st, double gamma, d
 }
 
 }  // namespace
-
-int hd_blocks(const HdBox &g, int nst)
-{
-  if (g.dims == 1) {
-    const int own = block1d(g) - 4*nst;
-    return (g.nx + own - 1)/own;
-  }
-  const int l = march_cells(g);
-  if (g.dims == 2) return (((g.nx + 62)/63)*((g.ny + l - 1)/l) + 3)/4;
-  return ((g.nx + TX - 1)/TX)*((g.ny + TY - 1)/TY)*((g.nz + l - 1)/l);
-}
 
 void hd_launch_stage(const HdBufs &b, const HdBox &g, const HdStep &st, RKW w, int first_stage,
                      int want_dt, int limiter, int solver, double gamma, double small_rho,
@@ -718,6 +775,19 @@ void hd_launch_stage(const HdBufs &b, const HdBox &g, const HdStep &st, RKW w, i
   } else {
     if (solver == 2) stage_t<VANLEER_LIM, 2>(b, g, st, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
     else             stage_t<VANLEER_LIM, 1>(b, g, st, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
+  }
+}
+
+void hd_launch_sweep(int dir, const HdBufs &b, const HdBox &g, const StepCtl *ctl, RKW w, int first_stage,
+                     int want_dt, int limiter, int solver, double gamma, double small_rho,
+                     double small_prs, hipStream_t s)
+{
+  if (limiter == MC_LIM) {
+    if (solver == 2) sweep_t<MC_LIM, 2>(dir, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
+    else             sweep_t<MC_LIM, 1>(dir, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
+  } else {
+    if (solver == 2) sweep_t<VANLEER_LIM, 2>(dir, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
+    else             sweep_t<VANLEER_LIM, 1>(dir, b, g, ctl, w, first_stage, want_dt, gamma, small_rho, small_prs, s);
   }
 }
 

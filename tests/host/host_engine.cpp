@@ -162,7 +162,7 @@ template void batch2d_dump_gather<float>(const BoxDesc &, const int *, const flo
                                          double *, hipStream_t);
 void batch2d_launch_dt(const double *, const int *, int, StepCtl *, double, double, int, hipStream_t) {}
 
-int hd_blocks(const HdBox &g, int) { return (g.ncell + 63)/64; }
+// HD launches: 200 a stage, 201 a 1D step, 210 + direction a sweep
 static void hd_seen(const HdBufs &b, const HdStep &st)
 {
   hd_arrived = st.arrived;
@@ -180,6 +180,12 @@ void hd_launch_step1d(const HdBufs &b, const HdBox &, const HdStep &st, int, int
 {
   hd_seen(b, st);
   launches.push_back({201, {}});
+}
+
+void hd_launch_sweep(int dir, const HdBufs &, const HdBox &, const StepCtl *, RKW, int, int, int, int, double, double,
+                     double, hipStream_t)
+{
+  launches.push_back({210 + dir, {}});
 }
 
 template <typename R>

@@ -44,6 +44,16 @@ def _fill(d, seed=3):
     d.upload(1.0 + 0.1*rng.random((d.nvar,) + sh), vs)
 
 
+K_DT, HD_STAGE, HD_SWEEP = 9, 200, 210                # host_engine.cpp's and common.hpp's kernel ids
+
+
+def _launches(he, most=64):
+    """The kernel launches recorded so far: (id, values)."""
+    out = (C.c_int * (9*most))()
+    k = he.he_launches(out, most)
+    return [(out[9*q], list(out[9*q + 1:9*q + 9])) for q in range(k)]
+
+
 @pytest.mark.parametrize("n,physics,precision,sides", [
     ((41, 43, 47), "MHD", "fp64", ()),               # whole FP64 fields
     ((9, 8, 7), "MHD", "mixed", ()),                 # FP32: unpacked on the host
@@ -110,3 +120,22 @@ def test_download_helpers_stay_within_the_cores(he, cores, helpers):
     d.close()
     assert he.he_threads(1) - before == helpers
     assert all(np.array_equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("n,by_direction", [
+    ((8, 16, 1500), True), ((3, 100, 200), True), ((20, 100, 100), True), ((65, 8, 1500), True),
+    ((16, 4096, 1), True), ((3, 32768, 1), True),
+    ((40, 33, 200), False), ((16, 16, 16), False), ((64, 8, 24), False), ((128, 96, 112), False),
+    ((4096, 8, 8), False), ((32, 4096, 1), False), ((62, 512, 1), False), ((64, 4096, 1), False),
+    ((511, 333, 1), False)])
+def test_hd_boxes_that_leave_lanes_idle_go_by_direction(he, n, by_direction):
+    """A narrow HD box takes a launch per direction, where the one-launch stage's
+    tiles would be mostly empty; other boxes take the latter."""
+    d = _domain(n, "HD")
+    _fill(d)
+    _launches(he)
+    d.advance_step(1e-4)
+    got = [k for k, _ in _launches(he)]
+    d.close()
+    dims = 2 if n[2] == 1 else 3
+    assert got == (2*[HD_SWEEP + q for q in range(dims)] + [K_DT] if by_direction else 2*[HD_STAGE])
