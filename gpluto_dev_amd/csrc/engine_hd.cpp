@@ -36,6 +36,10 @@ public:
     for (void *p : ptrs) if (p) (void)hipFree(p);
   }
 
+  // doubles of U^n up to the next 128-byte line, and with the counters behind it
+  size_t counters_at() const { return (5*n + 15)/16*16; }
+  size_t ua_doubles() const { return counters_at() + HD_ARRIVED*sizeof(unsigned)/sizeof(double); }
+
   int init(const gpl_config &c, const EngineEnv &e)
   {
     cfg = c; env = e;
@@ -54,9 +58,10 @@ public:
     int rc = 0;
     rc |= dev_alloc(bytes, (void **)&VA, 5*n*sizeof(double));
     rc |= dev_alloc(bytes, (void **)&VB, 5*n*sizeof(double));
-    // the arrival counters follow U^n, so that the upload clears them
-    rc |= dev_alloc(bytes, (void **)&UA, 5*n*sizeof(double) + HD_ARRIVED*sizeof(unsigned));
-    arrived = (unsigned *)(UA + 5*n);
+    // the arrival counters follow U^n, so that the upload clears them, on cache
+    // lines of their own: other blocks store U in the launch that counts
+    rc |= dev_alloc(bytes, (void **)&UA, ua_doubles()*sizeof(double));
+    arrived = (unsigned *)(UA + counters_at());
     rc |= dev_alloc(bytes, (void **)&UB, 5*n*sizeof(double));
     if (hd_by_direction(g)) {
       rc |= dev_alloc(bytes, (void **)&dU, 5*n*sizeof(double));
@@ -72,7 +77,7 @@ public:
   int upload(const double *vc, const double *const *, int layout) override
   {
     const Layout L = make_layout(cfg, layout);
-    std::vector<double> hv(5*n), hu(5*n + HD_ARRIVED*sizeof(unsigned)/sizeof(double));
+    std::vector<double> hv(5*n), hu(ua_doubles());
     for (int k = 0; k < L.nz; k++)
       for (int j = 0; j < L.ny; j++)
         for (int i = 0; i < L.nx; i++) {

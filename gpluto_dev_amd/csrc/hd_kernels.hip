@@ -630,6 +630,8 @@ void k_hd_step1d(HdBox g, HdBufs b, HdStep st, double gamma, double small_rho, d
   const int t = threadIdx.x, nx = g.nx;
   const size_t n = (size_t)nx;
   const int q0 = blockIdx.x*T - H, i = q0 + t;        // this thread's cell, ghosts included
+  // every wave uses dt in the first stage, before the barriers of the second, so
+  // before the block counts itself in
   const double dt = st.ctl->dt, dtdx = dt/g.dx;
   const bool periodic = g.lo[0] == GPL_PERIODIC;
   // the cell to start from; a periodic ghost is an image and evolves like it,

@@ -139,3 +139,20 @@ def test_hd_boxes_that_leave_lanes_idle_go_by_direction(he, n, by_direction):
     d.close()
     dims = 2 if n[2] == 1 else 3
     assert got == (2*[HD_SWEEP + q for q in range(dims)] + [K_DT] if by_direction else 2*[HD_STAGE])
+
+
+@pytest.mark.parametrize("n", [(3, 1, 1), (16, 1, 1), (4097, 1, 1), (5, 7, 1), (33, 21, 1), (3, 5, 7)])
+def test_hd_arrival_counters_have_their_own_lines(he, n):
+    """No array that the blocks of an HD launch store to shares a 128-byte line
+    with the counters that they arrive at."""
+    d = _domain(n, "HD")
+    _fill(d)
+    he.he_hd_arrived.restype = he.he_hd_u.restype = C.c_size_t
+    for _ in range(2):                               # 1D: both sets of buffers
+        d.advance_step(1e-4)
+        at = he.he_hd_arrived()
+        assert at % 128 == 0
+        for q in range(2):
+            u = he.he_hd_u(q)
+            assert u + 5*8*n[0]*n[1]*n[2] <= at or u >= at + 17*128
+    d.close()
