@@ -171,9 +171,11 @@ public:
     march[0] = march_length(fp64, (long long)g.nx*g.nz, g.ny);
     march[1] = march_length(fp64, (long long)g.nx*g.ny, g.nz);
     // GPL_MARCH = 1, 2, 4 .. 64 fixes both
+    bool march_fixed = false;
     if (const char *m = getenv("GPL_MARCH")) {
       const int l = atoi(m);
-      if (l >= 1 && l <= 64 && (l & (l - 1)) == 0) march[0] = march[1] = l;
+      march_fixed = l >= 1 && l <= 64 && (l & (l - 1)) == 0;
+      if (march_fixed) march[0] = march[1] = l;
     }
     // the slab pipeline: GPL_PIPE_SLABS slabs (0 or 1: off); every slab but
     // the last starts and ends at a multiple of the y/z march and of the EMF
@@ -183,22 +185,22 @@ public:
       if (const char *m = getenv("GPL_PIPE_SLABS")) want = atoi(m);
       // a slab's EMF launch covers only its planes: tiles marching 8 planes
       // keep four times as many workgroups in flight as the default 32
-      if (want >= 3 && !getenv("GPL_EMF_MARCH")) emf_march = -8;
+      const int emf = getenv("GPL_EMF_MARCH") ? emf_march : -8, lt = emf < 0 ? -emf : 0;
       // a slab starts at a multiple of every march length
-      if (want >= 3 && !getenv("GPL_MARCH")) march[0] = march[1] = 16;
-      const int lt = emf_march < 0 ? -emf_march : 0;
+      const int lm = march_fixed ? march[1] : 16;
       if (want >= 3 && fp64 && fused && !fused_xy && lt > 0 &&
           c.ct_emf_average == GPL_UCT_HLL && want <= kMaxSlab) {
-        const int unit = march[1] > lt ? march[1] : lt;
+        const int unit = lm > lt ? lm : lt;
         int p = (g.nz + want - 1)/want;
         p = (p + unit - 1)/unit*unit;
         if (p > 0 && (g.nz + p - 1)/p >= 3) {
           pipelined = true;
           slab_planes = p;
           nslab = (g.nz + p - 1)/p;
+          march[0] = march[1] = lm;
+          emf_march = emf;
         }
       }
-      if (!pipelined && want >= 3 && !getenv("GPL_EMF_MARCH")) emf_march = emf_auto;
     }
     rows = sweep_rows(g.nx, (long long)g.ny*g.nz);
     if (fp64 && fused && !fused_xy && !pipelined && !getenv("GPL_MARCH")) {

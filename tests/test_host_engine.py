@@ -156,3 +156,35 @@ def test_hd_arrival_counters_have_their_own_lines(he, n):
             u = he.he_hd_u(q)
             assert u + 5*8*n[0]*n[1]*n[2] <= at or u >= at + 17*128
     d.close()
+
+
+K_MHD_SWEEP_X, K_MHD_XY = 4, 13                      # common.hpp's kernel ids
+
+
+def _mhd_shape(he, n, precision="fp64", **kw):
+    """(march y, march z, rows, columns y, columns z, EMF march) of a box's launches."""
+    d = _domain(n, precision=precision, **kw)
+    _fill(d)
+    _launches(he)
+    d.advance_step(1e-4)
+    got = {tuple(v[:6]) for k, v in _launches(he) if k <= K_MHD_XY and k != K_DT}
+    d.close()
+    assert len(got) == 1
+    return got.pop()
+
+
+@pytest.mark.parametrize("n,precision,kw", [
+    ((64, 64, 64), "mixed", {}),                             # FP32
+    ((64, 64, 64), "fp64", {"ct_emf_average": "UCT_HLLD"}),
+    ((64, 64, 30), "fp64", {})])                             # two slabs of 16 planes
+def test_a_box_that_cannot_be_pipelined_keeps_its_launch_shape(he, n, precision, kw, monkeypatch):
+    want = _mhd_shape(he, n, precision, **kw)
+    monkeypatch.setenv("GPL_PIPE_SLABS", "4")
+    assert _mhd_shape(he, n, precision, **kw) == want
+
+
+def test_a_pipelined_box_marches_16(he, monkeypatch):
+    monkeypatch.setenv("GPL_PIPE_SLABS", "4")
+    assert _mhd_shape(he, (64, 64, 64))[:2] + _mhd_shape(he, (64, 64, 64))[3:] == (16, 16, 0, 0, -8)
+    monkeypatch.setenv("GPL_MARCH", "8")
+    assert _mhd_shape(he, (64, 64, 64))[:2] == (8, 8)
