@@ -69,14 +69,22 @@ void launch_zone_reset(unsigned long long *counts, hipStream_t s);
 // 128^3 100 + 106 against 108 + 113 at 8 and 117 + 127 at 4.
 //
 // FP32: four wavefronts per SIMD hide the load latency, so L is the largest of
-// 8, 4, 2, 1 that leaves 8192 wavefronts (512 for the last halving).  z march
-// and x+y kernel, us at 16 -> rule: 64^3 48 + 64 -> 16 + 20 (L = 2), 128^3
-// 81 + 110 -> 82 + 90 (L = 4), 192^3 280 + 270 -> 250 + 263 (L = 8).
+// 8, 4, 2, 1 that leaves 8192 wavefronts (512 for the last halving), and 16 where
+// that leaves `waves16`, which differs by kernel: the z march loses at 16 even on
+// large boxes (never: 0), the other two win once the chip is full (kWavesXY,
+// kWaves2D).  z march and x+y kernel, us at 16 -> rule: 64^3 48 + 64 -> 16 + 20
+// (L = 2), 128^3 81 + 110 -> 82 + 90 (L = 4), 192^3 280 + 270 -> 250 + 263 (L = 8).
+// x+y kernel at 8 / 16: 208^3 379 / 378, 224^3 430 / 439, 400x300x100 685 / 698, 256^3
+// 572 / 566, 320^3 2202 / 2130; z march 256^3 564 / 590, 320^3 1131 / 1168.
 //
-// The 2D y march: 512^2 FP64 67 -> 26 us (L = 4), 306x195 FP32 54 -> 9.5 (L = 2).
-inline int march_length(bool fp64, long long across, int n)
+// The 2D y march: 512^2 FP64 67 -> 26 us (L = 4), 306x195 FP32 54 -> 9.5 (L = 1).
+// FP32 step at the other lengths' best of 4 and 8 / at 16: 1024^2 219 / 246, 1500x1400
+// 501 / 508, 2000x1500 658 / 649, 300x8000 579 / 570, 3000^2 2061 / 2000.
+constexpr long long kWavesXY = 16384, kWaves2D = 2304;
+inline int march_length(bool fp64, long long across, int n, long long waves16)
 {
   if (!fp64) {
+    if (waves16 && across*((n + 15)/16)/64 >= waves16) return 16;
     int l = 8;
     while (l > 1 && across*((n + l - 1)/l)/64 < (l > 2 ? 8192 : 512)) l /= 2;
     return l;

@@ -203,7 +203,7 @@ static int batch_init(gpl_batch *b, const gpl_config *cfg, int nbox, const int *
   std::vector<int> yb[4];
   if (env) {
     b->march_idx = kAuto;
-    b->march[kAuto] = march_length(b->fp64, 64LL*((b->hbox[0].nx + 63)/64), b->hbox[0].ny);
+    b->march[kAuto] = march_length(b->fp64, 64LL*((b->hbox[0].nx + 63)/64), b->hbox[0].ny, kWaves2D);
   }
   for (int m = env ? kAuto : 0; m < (env ? kAuto + 1 : 3); m++) {
     const int L = b->march[m];

@@ -168,8 +168,8 @@ public:
     fused_xy = !fp64;
     if (const char *m = getenv("GPL_FUSED_XY")) fused_xy = atoi(m) != 0;
     fused_xy = fused_xy && fused && !rmhd && 20*(size_t)g.nx*rs <= 65536;
-    march[0] = march_length(fp64, (long long)g.nx*g.nz, g.ny);
-    march[1] = march_length(fp64, (long long)g.nx*g.ny, g.nz);
+    march[0] = march_length(fp64, (long long)g.nx*g.nz, g.ny, fused_xy ? kWavesXY : 0);
+    march[1] = march_length(fp64, (long long)g.nx*g.ny, g.nz, 0);
     // GPL_MARCH = 1, 2, 4 .. 64 fixes both
     bool march_fixed = false;
     if (const char *m = getenv("GPL_MARCH")) {

@@ -13,6 +13,7 @@
 #include <dirent.h>
 #include <stdlib.h>
 #include <string.h>
+#include <sys/mman.h>
 
 #include <algorithm>
 #include <map>
@@ -39,16 +40,19 @@ hipError_t fail(hipError_t e) { last = e; return e; }
 hipError_t take(std::map<void *, size_t> &live, size_t limit, void **p, size_t n)
 {
   if (held(live) + n > limit) { *p = nullptr; return fail(hipErrorOutOfMemory); }
-  if (posix_memalign(p, 256, n ? n : 1)) return fail(hipErrorOutOfMemory);
-  memset(*p, 0, n);
+  // zero pages, none of them there before it is touched
+  *p = mmap(nullptr, n ? n : 1, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0);
+  if (*p == MAP_FAILED) { *p = nullptr; return fail(hipErrorOutOfMemory); }
   live[*p] = n;
   return hipSuccess;
 }
 hipError_t give(std::map<void *, size_t> &live, void *p)
 {
   if (!p) return hipSuccess;
-  if (!live.erase(p)) return fail(hipErrorInvalidValue);
-  free(p);
+  const auto at = live.find(p);
+  if (at == live.end()) return fail(hipErrorInvalidValue);
+  munmap(p, at->second ? at->second : 1);
+  live.erase(at);
   return hipSuccess;
 }
 int threads_now()

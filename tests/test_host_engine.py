@@ -188,3 +188,27 @@ def test_a_pipelined_box_marches_16(he, monkeypatch):
     assert _mhd_shape(he, (64, 64, 64))[:2] + _mhd_shape(he, (64, 64, 64))[3:] == (16, 16, 0, 0, -8)
     monkeypatch.setenv("GPL_MARCH", "8")
     assert _mhd_shape(he, (64, 64, 64))[:2] == (8, 8)
+
+
+@pytest.mark.parametrize("n,xy,z", [((256, 256, 256), 16, 8), ((224, 224, 224), 8, 8), ((128, 128, 128), 4, 4)])
+def test_mixed_marches_have_a_length_each(he, n, xy, z):
+    """The mixed form's x+y kernel takes rows of 16 where that fills the chip; the
+    z march, which loses at 16, does not."""
+    d = _domain(n, precision="mixed")                # no state: the launches only
+    _launches(he)
+    d.advance_step(1e-4)
+    got = {tuple(v[:2]) for k, v in _launches(he) if k <= K_MHD_XY and k != K_DT}
+    d.close()
+    assert got == {(xy, z)}
+
+
+@pytest.mark.parametrize("n,precision,march", [
+    ((2000, 1500, 1), "mixed", 16), ((300, 8000, 1), "mixed", 16), ((1500, 1400, 1), "mixed", 4),
+    ((306, 195, 1), "mixed", 1), ((512, 512, 1), "fp64", 4)])
+def test_2d_march_length(he, n, precision, march):
+    d = _domain(n, precision=precision)
+    _launches(he)
+    d.advance_step(1e-4)
+    got = {v[0] for k, v in _launches(he) if k == 101}        # the y sweep
+    d.close()
+    assert got == {march}
