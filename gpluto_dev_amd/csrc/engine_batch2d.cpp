@@ -29,6 +29,12 @@ namespace {
 constexpr int kMarch[3] = {8, 16, 32};     // the autotuner's y-march lengths
 constexpr int kAuto = 3;                   // index of the length chosen by size (one box)
 constexpr int kBpc[4] = {2, 4, 8, 0};      // workgroups per CU; 0 = one per work group
+// Workgroups per CU of one box's finish: fewer than are resident (seven at its 70
+// registers), so that no second round of a few blocks trails the first.  Step, us,
+// at 8 / 7 / 6 / 5 / 4: 3000^2 FP32 1988 / 1901 / 1894 / 1900 / 1929, FP64 3033 / 2977 /
+// 2955 / 2940 / 2955; 2000x1500 FP32 646 / 623 / 624 / 628 / 635, FP64 1041 / 1028 / 1024 /
+// 1023 / 1032.
+constexpr int kFinishPerCU = 6;
 
 template <typename T>
 int upload_vec(T **dst, const std::vector<T> &v, size_t &bytes)
@@ -560,6 +566,7 @@ static void enqueue_stage(gpl_batch *b, const double *uin, double *uout, double 
     q.tiles = b->tiles + b->tbeg[gi]; q.ntiles = b->tbeg[gi + 1] - b->tbeg[gi];
     const int gx = grid_for(b, (q.nx_items + 3)/4), gy = grid_for(b, (q.ny_items + 3)/4);
     const int gt = grid_for(b, q.ntiles);
+    const int gf = b->owns_env || gt < kFinishPerCU*b->ncu ? gt : kFinishPerCU*b->ncu;   // (a batch tunes its own)
     // Boundary (Src/rk_step.cpp: at the start of every stage) on padded boxes
     if (b->padded)
       batch2d_boundary<R>(b->box + box0, nbg, b->maxp, b->side, (R *)b->V, vin, (size_t)b->ncell, st);
@@ -568,7 +575,7 @@ static void enqueue_stage(gpl_batch *b, const double *uin, double *uout, double 
     batch2d_launch<R>(B2_SWEEP_Y, q, w, first_stage, first_stage, c.limiter, b->ksolver, march, gy,
                       c.gamma, c.small_rho, c.small_prs, st);
     for (int ph : {b->tile_lanes ? B2_CT : B2_EMF, B2_FINISH}) {
-      batch2d_launch<R>(ph, q, w, first_stage, first_stage, c.limiter, b->ksolver, march, gt,
+      batch2d_launch<R>(ph, q, w, first_stage, first_stage, c.limiter, b->ksolver, march, ph == B2_FINISH ? gf : gt,
                         c.gamma, c.small_rho, c.small_prs, st);
       if (ph == B2_CT) break;
     }

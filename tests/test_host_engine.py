@@ -212,3 +212,14 @@ def test_2d_march_length(he, n, precision, march):
     got = {v[0] for k, v in _launches(he) if k == 101}        # the y sweep
     d.close()
     assert got == {march}
+
+
+@pytest.mark.parametrize("n,blocks", [((2000, 1500, 1), 6*256), ((600, 600, 1), 1407)])
+def test_2d_finish_leaves_no_trailing_round(he, n, blocks):
+    """One box's finish launches no more blocks than are resident at once."""
+    d = _domain(n, precision="mixed")
+    _launches(he)
+    d.advance_step(1e-4)
+    got = {v[1] for k, v in _launches(he) if k == 103}
+    d.close()
+    assert got == {blocks}
