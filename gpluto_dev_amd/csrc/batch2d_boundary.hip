@@ -60,8 +60,7 @@ void k2_bnd_dir(const BoxDesc *__restrict__ box, int dir, int type_lo, int type_
   // would hold the loads after it back by a trip to memory each
 #pragma unroll
   for (int l = 0; l < 2; l++) {
-    // one cell across: the upper side's second layer repeats its first
-    const size_t cq = at + (type == GPL_PERIODIC && upper && n == 1 ? hi : source(g0 + l))*sd;
+    const size_t cq = at + source(g0 + l)*sd;
     e[l][0] = Bt[cq];
     if (cell) {
       e[l][1] = Bt[cq + st];

@@ -161,10 +161,9 @@ def test_hd_arrival_counters_have_their_own_lines(he, n):
 K_MHD_SWEEP_X, K_MHD_XY = 4, 13                      # common.hpp's kernel ids
 
 
-def _mhd_shape(he, n, precision="fp64", **kw):
+def _mhd_shape(he, n, precision="fp64", sides=(), **kw):
     """(march y, march z, rows, columns y, columns z, EMF march) of a box's launches."""
-    d = _domain(n, precision=precision, **kw)
-    _fill(d)
+    d = _domain(n, precision=precision, sides=sides, **kw)
     _launches(he)
     d.advance_step(1e-4)
     got = {tuple(v[:6]) for k, v in _launches(he) if k <= K_MHD_XY and k != K_DT}
@@ -223,3 +222,14 @@ def test_2d_finish_leaves_no_trailing_round(he, n, blocks):
     got = {v[1] for k, v in _launches(he) if k == 103}
     d.close()
     assert got == {blocks}
+
+
+@pytest.mark.parametrize("physics,n", [
+    ("MHD", (2, 8, 1)), ("MHD", (8, 2, 1)), ("MHD", (2, 8, 8)), ("MHD", (8, 8, 2)), ("HD", (2, 1, 1)),
+    ("HD", (8, 2, 1)), ("HD", (8, 8, 2))])
+@pytest.mark.parametrize("sides", [(), WALLS])
+def test_boxes_below_three_zones_are_refused(he, physics, n, sides):
+    """The ghost fills count on it: the source layers of one side are active
+    zones that the other side does not write."""
+    with pytest.raises(RuntimeError, match="invalid argument"):
+        _domain(n, physics, sides=sides)
