@@ -233,3 +233,20 @@ def test_boxes_below_three_zones_are_refused(he, physics, n, sides):
     zones that the other side does not write."""
     with pytest.raises(RuntimeError, match="invalid argument"):
         _domain(n, physics, sides=sides)
+
+
+@pytest.mark.parametrize("n,sides,rows,y,z", [
+    # the boxes of tests/test_gpu_columns.py: every width above 5, with remainders
+    # in x and in the last wavefront
+    ((34, 29, 42), (), 5, 6, 5), ((48, 20, 36), (), 1, 7, 4), ((69, 20, 28), (), 3, 8, 6),
+    ((20, 65, 24), (), 3, 0, 7), ((62, 29, 20), (), 1, 6, 8),
+    # and of tests/test_gpu_launch_shapes.py: 4 and 5 per block, y marches in one
+    ((5, 3, 4), (), 1, 4, 4), ((9, 64, 5), (), 2, 4, 4), ((33, 17, 64), (), 5, 5, 4),
+    ((13, 65, 32), (), 9, 0, 5), ((18, 14, 21), ("outflow", "reflective", "outflow", "outflow",
+                                                 "reflective", "reflective"), 2, 4, 4),
+    ((21, 30, 11), (), 2, 4, 4), ((14, 19, 38), (), 3, 4, 4),
+    ((5, 21, 37), (), 4, 4, 4), ((20, 23, 29), (), 3, 4, 4), ((72, 17, 19), (), 2, 6, 5)])
+def test_columns_and_rows_of_the_size_rules(he, n, sides, rows, y, z):
+    """The whole columns and x rows per block that the GPU tests of these boxes
+    mean to run (0: marches)."""
+    assert _mhd_shape(he, n, sides=sides)[2:5] == (rows, y, z)
