@@ -1,4 +1,4 @@
-// The active zones of one variable for a download (launch_field_gather), and
+// The active zones of a download's variables (launch_fields_gather), and
 // the dbl dump image of a 3D MHD/RMHD box, gathered on the device in the
 // file's own order (Src/write_data.cpp:136-159 with FillOutputBuffer
 // :564-607): the eight primitives over the active zones, i fastest, then
@@ -66,27 +66,33 @@ template void mhd3d_dump_gather<float>(const Box3 &, const int *, const int *, c
 
 namespace {
 
-template <typename R>
+struct FieldSet { const void *src[kFields]; bool f32[kFields]; };
+
+// elements t0 .. t0 + count - 1 of the fields laid one after the other, n each
 __global__ __launch_bounds__(256)
-void k_field_gather(FieldGeom g, const R *__restrict__ src, size_t e0, size_t count, double *__restrict__ dst)
+void k_fields_gather(FieldGeom g, FieldSet f, size_t n, size_t t0, size_t count, double *__restrict__ dst)
 {
-  const size_t t = (size_t)blockIdx.x*blockDim.x + threadIdx.x;
+  const size_t t = (size_t)blockIdx.x*256 + threadIdx.x;
   if (t >= count) return;
-  const size_t e = e0 + t, r = e / g.n[0];
-  const int i = (int)(e - r*g.n[0]), k = (int)(r / g.n[1]), j = (int)(r - (size_t)k*g.n[1]);
-  dst[t] = (double)src[g.off + (size_t)(i + g.lo[0]) +
-                       (size_t)g.sx*((size_t)(j + g.lo[1]) + (size_t)g.sy*(k + g.lo[2]))];
+  const unsigned q = (unsigned)((t0 + t)/n), e = (unsigned)(t0 + t - q*n);
+  const unsigned r = e / (unsigned)g.n[0], i = e - r*(unsigned)g.n[0];
+  const unsigned k = r / (unsigned)g.n[1], j = r - k*(unsigned)g.n[1];
+  const size_t o = g.off + (size_t)(i + g.lo[0]) +
+                   (size_t)g.sx*((size_t)(j + g.lo[1]) + (size_t)g.sy*(k + g.lo[2]));
+  dst[t] = f.f32[q] ? (double)((const float *)f.src[q])[o] : ((const double *)f.src[q])[o];
 }
 
 }  // namespace
 
-hipError_t launch_field_gather(const FieldGeom &g, const void *src, bool f32, size_t e0, size_t count,
-                               double *dst, hipStream_t s)
+hipError_t launch_fields_gather(const FieldGeom &g, const std::vector<FieldOut> &out, size_t t0, size_t count,
+                                double *dst, hipStream_t s)
 {
+  FieldSet set = {};
+  for (size_t q = 0; q < out.size(); q++) { set.src[q] = out[q].src; set.f32[q] = out[q].f32; }
+  size_t n = (size_t)g.n[0]*g.n[1]*g.n[2];
   // the launch's own result: the thread's last error may be an older call's
-  void *args[] = {const_cast<FieldGeom *>(&g), &src, &e0, &count, &dst};
-  const void *kernel = f32 ? (const void *)k_field_gather<float> : (const void *)k_field_gather<double>;
-  return hipLaunchKernel(kernel, dim3((unsigned)((count + 255)/256)), dim3(256), args, 0, s);
+  void *args[] = {const_cast<FieldGeom *>(&g), &set, &n, &t0, &count, &dst};
+  return hipLaunchKernel((const void *)k_fields_gather, dim3((unsigned)((count + 255)/256)), dim3(256), args, 0, s);
 }
 
 }  // namespace gpl

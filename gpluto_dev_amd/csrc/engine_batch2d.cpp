@@ -283,6 +283,9 @@ static int batch_init(gpl_batch *b, const gpl_config *cfg, int nbox, const int *
     rc |= dev_alloc(b->bytes, (void **)&b->ctl, (size_t)nbox*sizeof(StepCtl));
   }
   if (rc) return rc == GPL_EHIP ? GPL_EHIP : GPL_ENOMEM;
+  size_t largest = 0;
+  for (int q = 0; q < nbox; q++) largest = std::max(largest, (size_t)nx[q]*ny[q]);
+  b->copy.prepare(18*largest);
   std::vector<StepCtl> z(nbox, StepCtl{0.0, 0.0, 0.0, 0});
   if (hipMemcpy(b->ctl, z.data(), nbox*sizeof(StepCtl), hipMemcpyHostToDevice) != hipSuccess ||
       hipMemset(b->err, 0, sizeof(uint32_t)) != hipSuccess)

@@ -69,6 +69,7 @@ public:
     }
     rc |= dev_alloc(bytes, (void **)&cdt_part, (size_t)hd_blocks(g, nstages())*sizeof(double));
     rc |= dev_alloc(bytes, (void **)&diag, (size_t)(DIAG_BLOCKS + 1)*DIAG_MAXQ*sizeof(double));
+    copy.prepare(10*n);
     cur_v = VA;
     cur_u = UA;
     return rc ? GPL_ENOMEM : 0;

@@ -246,6 +246,7 @@ public:
     rc |= dev_alloc(bytes, &E, 3*n*rs);
     rc |= dev_alloc(bytes, (void **)&cdt_part, (size_t)nparts*sizeof(double));
     rc |= dev_alloc(bytes, (void **)&diag, (size_t)(DIAG_BLOCKS + 1)*DIAG_MAXQ*sizeof(double));
+    copy.prepare(19*(size_t)na[0]*na[1]*na[2]);
     cur = 0;
     return rc ? GPL_ENOMEM : 0;
   }

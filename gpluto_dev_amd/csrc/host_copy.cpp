@@ -101,13 +101,12 @@ private:
   bool quit = false;
 };
 
-// part of a run of fields that are adjacent on both sides
+// part of a run of fields that are adjacent at the caller's and, unless the gather
+// kernel collects them, on the device
 struct Piece {
-  const void *src;
-  bool f32;
-  size_t e0, count;  // elements of the field
+  const double *src;
   double *dst;
-  size_t at;         // offset in its slot, doubles
+  size_t count, at;  // doubles; offset in its slot
 };
 
 }  // namespace
@@ -119,29 +118,59 @@ HostCopy::~HostCopy()
   for (hipEvent_t e : done) if (e) (void)hipEventDestroy(e);
 }
 
-bool HostCopy::reserve(size_t slot, bool gather)
+bool HostCopy::pinned(size_t bytes)
 {
-  const size_t want = kSlots*slot*sizeof(double);
-  for (int q = 0; q < kSlots; q++)
+  if (pin_cap >= bytes) return true;
+  if (pin) (void)hipHostFree(pin);
+  pin = nullptr;
+  pin_cap = 0;
+  if (hipHostMalloc((void **)&pin, bytes, hipHostMallocDefault) != hipSuccess) {
+    pin = nullptr;
+    (void)hipGetLastError();                   // dealt with by the caller: not for a later check to find
+    return false;
+  }
+  pin_cap = bytes;
+  return true;
+}
+
+bool HostCopy::reserve(size_t slot, int slots, bool gather)
+{
+  const size_t want = slots*slot*sizeof(double);
+  bool ok = pinned(want);
+  for (int q = 0; q < slots && ok; q++)
     if (!done[q] && hipEventCreateWithFlags(&done[q], hipEventDisableTiming) != hipSuccess) {
       done[q] = nullptr;
-      return false;
+      ok = false;
     }
-  if (pin_cap < want) {
-    if (pin) (void)hipHostFree(pin);
-    pin = nullptr;
-    pin_cap = 0;
-    if (hipHostMalloc((void **)&pin, want, hipHostMallocDefault) != hipSuccess) { pin = nullptr; return false; }
-    pin_cap = want;
-  }
-  if (gather && dev_cap < want) {
+  if (ok && gather && dev_cap < want) {
     if (dev) (void)hipFree(dev);
     dev = nullptr;
     dev_cap = 0;
-    if (hipMalloc((void **)&dev, want) != hipSuccess) { dev = nullptr; return false; }
-    dev_cap = want;
+    if (hipMalloc((void **)&dev, want) == hipSuccess) dev_cap = want;
+    else { dev = nullptr; ok = false; }
   }
-  return true;
+  if (!ok) (void)hipGetLastError();
+  return ok;
+}
+
+void HostCopy::prepare(size_t total)
+{
+  // touched here: a page's first access costs more than its copy
+  if (total <= kSmall && pinned(total*sizeof(double))) memset(pin, 0, total*sizeof(double));
+}
+
+int HostCopy::fetch_small(const FieldGeom &g, const std::vector<FieldOut> &out, hipStream_t s)
+{
+  const size_t n = (size_t)g.n[0]*g.n[1]*g.n[2], nf = out.size();
+  if (launch_fields_gather(g, out, 0, nf*n, pin, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
+    return GPL_EHIP;
+  for (size_t q = 0; q < nf;) {
+    size_t run = 1;                            // arrays that follow one another at the caller's
+    while (q + run < nf && out[q + run].dst == out[q].dst + run*n) run++;
+    memcpy(out[q].dst, pin + q*n, run*n*sizeof(double));
+    q += run;
+  }
+  return 0;
 }
 
 int HostCopy::fetch_whole(const FieldGeom &g, const std::vector<FieldOut> &out, hipStream_t s)
@@ -192,49 +221,44 @@ int HostCopy::fetch(const FieldGeom &g, const std::vector<FieldOut> &out, hipStr
   if (!total) return 0;
   bool gather = !g.whole;
   for (const FieldOut &f : out) gather = gather || f.f32;
-  // a small state goes through all slots at once, with one wait, a larger one in
-  // slots of an eighth of it, 16 MiB at most
-  const bool once = total <= (size_t(1) << 17);
-  // up to a megabyte the runtime's own staging is as fast and needs no buffer
-  if (once && !gather) return fetch_whole(g, out, s);
-  size_t slot = once ? (total + kSlots - 1)/kSlots : (total + 7)/8;
-  if (slot > kChunk) slot = kChunk;
-  if (!reserve(slot, gather)) {
-    (void)hipGetLastError();                   // dealt with here: not for a later check to find
+  const bool fits = out.size() <= kFields;     // the gather kernel's set
+  if (total <= kSmall && fits && pinned(total*sizeof(double))) return fetch_small(g, out, s);
+  // a larger state in slots of an eighth of it, 1 MiB at least, 16 MiB at most
+  const size_t slot = std::min(std::max((total + 7)/8, kSmall), kChunk);
+  const int slots = (int)std::min((total + slot - 1)/slot, (size_t)kSlots);
+  if (total <= kSmall || (gather && !fits) || !reserve(slot, slots, gather))
     return gather ? fetch_rows(g, out, s) : fetch_whole(g, out, s);
-  }
-  const size_t hold = once ? slot*kSlots : slot;   // doubles of a group
-  // groups of pieces, one group per slot; without a gather, fields that follow
-  // one another on both sides make one piece
+  // groups of pieces, one group per slot
   std::vector<std::vector<Piece>> groups;
-  size_t used = hold;
-  for (const FieldOut &f : out)
+  size_t used = slot;
+  for (const FieldOut &f : out) {
+    const double *src = gather ? nullptr : (const double *)f.src + g.off;
     for (size_t e = 0; e < n;) {
-      if (used == hold) { groups.emplace_back(); used = 0; }
-      const size_t c = n - e < hold - used ? n - e : hold - used;
+      if (used == slot) { groups.emplace_back(); used = 0; }
+      const size_t c = std::min(n - e, slot - used);
       Piece *last = groups.back().empty() ? nullptr : &groups.back().back();
-      if (last && last->dst + last->count == f.dst + e &&
-          (gather ? false : (const double *)last->src + last->e0 + last->count == (const double *)f.src + e))
+      if (last && last->dst + last->count == f.dst + e && (gather || last->src + last->count == src + e))
         last->count += c;
       else
-        groups.back().push_back({f.src, f.f32, e, c, f.dst + e, used});
+        groups.back().push_back({gather ? nullptr : src + e, f.dst + e, c, used});
       e += c;
       used += c;
     }
+  }
   const int ng = (int)groups.size();
   Movers movers(total*sizeof(double));
   auto send = [&](int k) -> bool {
     double *hp = pin + (size_t)(k % kSlots)*slot, *dp = dev + (size_t)(k % kSlots)*slot;
-    size_t sum = 0;
-    for (const Piece &p : groups[k]) {
-      const hipError_t e = gather
-          ? launch_field_gather(g, p.src, p.f32, p.e0, p.count, dp + p.at, s)
-          : hipMemcpyAsync(hp + p.at, (const double *)p.src + g.off + p.e0, p.count*sizeof(double),
-                           hipMemcpyDeviceToHost, s);
-      if (e != hipSuccess) return false;
-      sum += p.count;
+    if (gather) {
+      const size_t t0 = (size_t)k*slot, c = std::min(slot, total - t0);
+      if (launch_fields_gather(g, out, t0, c, dp, s) != hipSuccess ||
+          hipMemcpyAsync(hp, dp, c*sizeof(double), hipMemcpyDeviceToHost, s) != hipSuccess)
+        return false;
+    } else {
+      for (const Piece &p : groups[k])
+        if (hipMemcpyAsync(hp + p.at, p.src, p.count*sizeof(double), hipMemcpyDeviceToHost, s) != hipSuccess)
+          return false;
     }
-    if (gather && hipMemcpyAsync(hp, dp, sum*sizeof(double), hipMemcpyDeviceToHost, s) != hipSuccess) return false;
     return hipEventRecord(done[k % kSlots], s) == hipSuccess;
   };
   bool ok = true;

@@ -25,7 +25,7 @@ struct Launch { int kernel, value[8]; };       // what a launcher was asked for
 std::vector<Launch> launches;
 std::map<void *, size_t> live_dev, live_pin;
 size_t dev_limit = ~size_t(0), pin_limit = ~size_t(0);
-int threads_seen = 0;
+int threads_seen = 0, copies = 0;
 const void *hd_arrived = nullptr, *hd_u[2] = {};
 
 size_t held(const std::map<void *, size_t> &m)
@@ -78,10 +78,16 @@ hipError_t hipMalloc(void **p, size_t n) { return take(live_dev, dev_limit, p, n
 hipError_t hipFree(void *p) { return give(live_dev, p); }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return take(live_pin, pin_limit, p, n); }
 hipError_t hipHostFree(void *p) { return give(live_pin, p); }
-hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { memcpy(d, s, n); return hipSuccess; }
+hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind)
+{
+  memcpy(d, s, n);
+  copies++;
+  return hipSuccess;
+}
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t)
 {
   memcpy(d, s, n);
+  copies++;
   return hipSuccess;
 }
 hipError_t hipMemset(void *d, int v, size_t n) { memset(d, v, n); return hipSuccess; }
@@ -198,15 +204,16 @@ template void launch_diagnostics<double>(const DiagBox &, const double *, const 
 template void launch_diagnostics<float>(const DiagBox &, const float *, const double *, double *, double *, hipStream_t);
 int net_pack_upload(const float *, float *, NetPack *, hipStream_t) { return GPL_EUNSUPPORTED; }
 
-hipError_t launch_field_gather(const FieldGeom &g, const void *src, bool f32, size_t e0, size_t count, double *dst,
-                               hipStream_t)
+hipError_t launch_fields_gather(const FieldGeom &g, const std::vector<FieldOut> &out, size_t t0, size_t count,
+                                double *dst, hipStream_t)
 {
-  for (size_t t = 0; t < count; t++) {
-    const size_t e = e0 + t, r = e / g.n[0];
-    const int i = (int)(e % g.n[0]), j = (int)(r % g.n[1]), k = (int)(r / g.n[1]);
+  const size_t n = (size_t)g.n[0]*g.n[1]*g.n[2];
+  for (size_t t = t0; t < t0 + count; t++) {
+    const size_t q = t/n, e = t % n, r = e/g.n[0];
+    const int i = (int)(e % g.n[0]), j = (int)(r % g.n[1]), k = (int)(r/g.n[1]);
     const size_t o = g.off + (size_t)(i + g.lo[0]) +
                      (size_t)g.sx*((size_t)(j + g.lo[1]) + (size_t)g.sy*(k + g.lo[2]));
-    dst[t] = f32 ? (double)((const float *)src)[o] : ((const double *)src)[o];
+    dst[t - t0] = out[q].f32 ? (double)((const float *)out[q].src)[o] : ((const double *)out[q].src)[o];
   }
   return hipSuccess;
 }
@@ -222,6 +229,7 @@ void he_limits(size_t dev, size_t pin) { dev_limit = dev; pin_limit = pin; }
 size_t he_held(int pinned) { return held(pinned ? live_pin : live_dev); }
 void he_set_last_error(int e) { last = (hipError_t)e; }
 int he_last_error() { return (int)last; }
+int he_copies() { const int n = copies; copies = 0; return n; }
 int he_threads(int reset) { const int n = threads_seen; if (reset) threads_seen = 0; return n; }
 int he_launches(int *out, int most)            // rows of 9, the newest `most`; clears the record
 {

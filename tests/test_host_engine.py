@@ -250,3 +250,19 @@ def test_columns_and_rows_of_the_size_rules(he, n, sides, rows, y, z):
     """The whole columns and x rows per block that the GPU tests of these boxes
     mean to run (0: marches)."""
     assert _mhd_shape(he, n, sides=sides)[2:5] == (rows, y, z)
+
+
+@pytest.mark.parametrize("n,physics,precision,sides", [
+    ((13107, 1, 1), "HD", "fp64", ()),               # 10 fields: 2 doubles below a MiB
+    ((16, 16, 16), "MHD", "fp64", ()), ((16, 16, 16), "MHD", "mixed", ()), ((12, 13, 14), "MHD", "fp64", WALLS),
+    ((60, 60, 1), "MHD", "mixed", WALLS)])
+def test_small_downloads_copy_nothing_field_by_field(he, n, physics, precision, sides):
+    """A state of at most 1 MiB comes through one gather into memory that the
+    context holds since its creation."""
+    d = _domain(n, physics, precision, sides)
+    _fill(d)
+    pinned = he.he_held(1)
+    he.he_copies()
+    d.download()
+    assert he.he_copies() == 0 and he.he_held(1) == pinned
+    d.close()
