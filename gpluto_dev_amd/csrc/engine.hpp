@@ -57,13 +57,6 @@ public:
   virtual int dump_gather(double *dst, hipStream_t s) = 0;
   size_t bytes = 0;   // device memory held
   HostCopy copy;      // downloads in the active layout
-  int fetch(const FieldGeom &g, const std::vector<FieldOut> &out, hipStream_t s)
-  {
-    const size_t had = copy.device_bytes();
-    const int rc = copy.fetch(g, out, s);
-    bytes += copy.device_bytes() - had;
-    return rc;
-  }
 
   // Zone-by-zone error reports (off until set_zone_reports(1)): one uint32
   // array of zone_cells() entries per RK stage and the counters [stage 0..2,

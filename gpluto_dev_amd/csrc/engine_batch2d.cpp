@@ -480,10 +480,7 @@ static int gpl_batch_download_impl(gpl_batch *b, int box, double *vc, double *co
         if (map[q] >= 0) out.push_back({b->U + map[q]*nc, false, uc + q*na});
         else             out.push_back({prim(q), !b->fp64, uc + q*na});
       }
-    const size_t had = b->copy.device_bytes();
-    const int rc = b->copy.fetch(fg, out, b->stream);
-    b->bytes += b->copy.device_bytes() - had;
-    return rc;
+    return b->copy.fetch(fg, out, b->stream);
   }
   std::vector<double> hv(8*m), hu(6*m), hs(2*m);
   for (int s = 0; s < 8; s++) {
@@ -791,10 +788,7 @@ public:
   }
   int download(double *vc, double *const *vs, double *uc, int layout) override
   {
-    const size_t had = b->bytes;
-    const int rc = gpl_batch_download_impl(b, 0, vc, vs, uc, layout);
-    bytes += b->bytes - had;
-    return rc;
+    return gpl_batch_download_impl(b, 0, vc, vs, uc, layout);
   }
   void enqueue_step(int advance_dt, LaunchTimer *) override { ::enqueue_step(b, advance_dt); }
   int graph_period() const override { return ::graph_period(b); }

@@ -112,7 +112,7 @@ public:
       std::vector<FieldOut> out;
       if (vc) for (int q = 0; q < 5; q++) out.push_back({cur_v + q*n, false, vc + q*n});
       if (uc) for (int q = 0; q < 5; q++) out.push_back({cur_u + q*n, false, uc + q*n});
-      return fetch(fg, out, env.stream);
+      return copy.fetch(fg, out, env.stream);
     }
     for (int which = 0; which < 2; which++) {
       double *dst = which == 0 ? vc : uc;

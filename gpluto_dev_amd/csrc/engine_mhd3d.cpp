@@ -348,7 +348,7 @@ public:
           if (map[q] >= 0) out.push_back({U + map[q]*n, false, uc + q*na3});
           else             out.push_back({prim(q), !fp64, uc + q*na3});
         }
-      return fetch(fg, out, env.stream);
+      return copy.fetch(fg, out, env.stream);
     }
     std::vector<double> hv(8*n);
     if ((vc || uc) && from_device_v(V, fp64, hv)) return GPL_EHIP;

@@ -235,10 +235,7 @@ static int gpl_download_impl(gpl_ctx *c, double *vc, double *const *vs, double *
   if (layout != GPL_LAYOUT_ACTIVE && layout != GPL_LAYOUT_ARY4D) return GPL_EINVAL;
   hipSetDevice(c->dev);
   if (hipStreamSynchronize(c->stream) != hipSuccess) return GPL_EHIP;
-  const size_t had = c->engine->bytes;
-  const int rc = c->engine->download(vc, vs, uc, layout);
-  c->bytes += c->engine->bytes - had;
-  return rc;
+  return c->engine->download(vc, vs, uc, layout);
 }
 
 extern "C" int gpl_download(gpl_ctx *c, double *vc, double *const *vs, double *uc, int layout)

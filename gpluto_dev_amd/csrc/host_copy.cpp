@@ -114,7 +114,6 @@ struct Piece {
 HostCopy::~HostCopy()
 {
   if (pin) (void)hipHostFree(pin);
-  if (dev) (void)hipFree(dev);
   for (hipEvent_t e : done) if (e) (void)hipEventDestroy(e);
 }
 
@@ -133,24 +132,16 @@ bool HostCopy::pinned(size_t bytes)
   return true;
 }
 
-bool HostCopy::reserve(size_t slot, int slots, bool gather)
+bool HostCopy::reserve(size_t slot, int slots)
 {
-  const size_t want = slots*slot*sizeof(double);
-  bool ok = pinned(want);
-  for (int q = 0; q < slots && ok; q++)
+  if (!pinned(slots*slot*sizeof(double))) return false;
+  for (int q = 0; q < slots; q++)
     if (!done[q] && hipEventCreateWithFlags(&done[q], hipEventDisableTiming) != hipSuccess) {
       done[q] = nullptr;
-      ok = false;
+      (void)hipGetLastError();
+      return false;
     }
-  if (ok && gather && dev_cap < want) {
-    if (dev) (void)hipFree(dev);
-    dev = nullptr;
-    dev_cap = 0;
-    if (hipMalloc((void **)&dev, want) == hipSuccess) dev_cap = want;
-    else { dev = nullptr; ok = false; }
-  }
-  if (!ok) (void)hipGetLastError();
-  return ok;
+  return true;
 }
 
 void HostCopy::prepare(size_t total)
@@ -226,7 +217,7 @@ int HostCopy::fetch(const FieldGeom &g, const std::vector<FieldOut> &out, hipStr
   // a larger state in slots of an eighth of it, 1 MiB at least, 16 MiB at most
   const size_t slot = std::min(std::max((total + 7)/8, kSmall), kChunk);
   const int slots = (int)std::min((total + slot - 1)/slot, (size_t)kSlots);
-  if (total <= kSmall || (gather && !fits) || !reserve(slot, slots, gather))
+  if (total <= kSmall || (gather && !fits) || !reserve(slot, slots))
     return gather ? fetch_rows(g, out, s) : fetch_whole(g, out, s);
   // groups of pieces, one group per slot
   std::vector<std::vector<Piece>> groups;
@@ -248,12 +239,10 @@ int HostCopy::fetch(const FieldGeom &g, const std::vector<FieldOut> &out, hipStr
   const int ng = (int)groups.size();
   Movers movers(total*sizeof(double));
   auto send = [&](int k) -> bool {
-    double *hp = pin + (size_t)(k % kSlots)*slot, *dp = dev + (size_t)(k % kSlots)*slot;
+    double *hp = pin + (size_t)(k % kSlots)*slot;
     if (gather) {
-      const size_t t0 = (size_t)k*slot, c = std::min(slot, total - t0);
-      if (launch_fields_gather(g, out, t0, c, dp, s) != hipSuccess ||
-          hipMemcpyAsync(hp, dp, c*sizeof(double), hipMemcpyDeviceToHost, s) != hipSuccess)
-        return false;
+      const size_t t0 = (size_t)k*slot;
+      if (launch_fields_gather(g, out, t0, std::min(slot, total - t0), hp, s) != hipSuccess) return false;
     } else {
       for (const Piece &p : groups[k])
         if (hipMemcpyAsync(hp + p.at, p.src, p.count*sizeof(double), hipMemcpyDeviceToHost, s) != hipSuccess)

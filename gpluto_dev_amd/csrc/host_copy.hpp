@@ -7,20 +7,21 @@
 //    download, 1D 100 zones 40 -> 15, 4096 zones 150 -> 27, 10^3 MHD 65 -> 21, 16^3 300
 //    -> 41, 18x17x16 77 -> 46, 60^2 mixed with ghosts 97 -> 38.
 //  * Above, the fields are cut into chunks of an eighth of the state, 1 to 16 MiB; a
-//    chunk is copied into one of kSlots pinned buffers (through a device buffer that a
-//    gather kernel fills where the stored array is FP32 or holds ghost layers), and
-//    while later chunks are on their way, helper threads move it to the caller's
-//    arrays.  256^3, the eleven arrays of Vc and Vs (1.48 GB): 422 ms with pageable
-//    copies into host vectors and element loops, 27.6 this way (a pinned copy alone
-//    is 26); 128^3 55 -> 3.7, 192^3 mixed 222 -> 12.4.  Chunks below 1 MiB cost
-//    more in waits than they overlap: 24^3 196 -> 126 us, 24^3 mixed 262 -> 115.
+//    chunk is copied into one of kSlots pinned buffers (where the stored array is FP32
+//    or holds ghost layers, written there by the gather kernel), and while later chunks
+//    are on their way, helper threads move it to the caller's arrays.  256^3, the
+//    eleven arrays of Vc and Vs (1.48 GB): 422 ms with pageable copies into host
+//    vectors and element loops, 27.6 this way (a pinned copy alone is 26); 128^3 55 ->
+//    3.7.  Chunks below 1 MiB cost more in waits than they overlap (24^3 196 -> 126
+//    us).  A device buffer between gather and copy is no faster: Vc, Vs and Uc of
+//    192^3 mixed 21.4 ms with, 20.4 without, 128^3 mixed with ghosts 6.5 and 6.3, 24^3
+//    mixed 115 and 94 us.
 //
 // The buffers belong to one context (no sharing between contexts or threads): the
 // small one is allocated with it, the others at its first larger transfer, at most
-// kSlots chunks of 16 MiB pinned and, if a gather is needed, as much on the device,
-// and are freed with it.  Where they cannot be had (a full card, a limit on locked
-// memory) the transfer takes neither: pageable copies, unpacked on the host where a
-// gather would be needed.
+// kSlots chunks of 16 MiB, and are freed with it; no device memory.  Where they cannot
+// be had (a limit on locked memory) the transfer does without: pageable copies,
+// unpacked on the host where a gather would be needed.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -52,7 +53,6 @@ public:
   int fetch(const FieldGeom &g, const std::vector<FieldOut> &out, hipStream_t s);
   // Before the first transfer of at most `total` doubles: a small state's buffer
   void prepare(size_t total);
-  size_t device_bytes() const { return dev_cap; }
 
 private:
   static constexpr int kSlots = 4;
@@ -60,17 +60,17 @@ private:
   static constexpr size_t kSmall = size_t(1) << 17;   // doubles of a small state at most: 1 MiB
   static constexpr size_t kRows = size_t(1) << 18;    // doubles of fetch_rows' host buffer
   bool pinned(size_t bytes);
-  bool reserve(size_t chunk, int slots, bool gather);
+  bool reserve(size_t chunk, int slots);
   int fetch_small(const FieldGeom &g, const std::vector<FieldOut> &out, hipStream_t s);
   int fetch_whole(const FieldGeom &g, const std::vector<FieldOut> &out, hipStream_t s);   // no gather needed
   int fetch_rows(const FieldGeom &g, const std::vector<FieldOut> &out, hipStream_t s);
-  double *pin = nullptr, *dev = nullptr;
-  size_t pin_cap = 0, dev_cap = 0;                     // bytes
+  double *pin = nullptr;
+  size_t pin_cap = 0;                                  // bytes
   hipEvent_t done[kSlots] = {};
 };
 
 // dst[t] = element t0 + t of the fields laid one after the other, in FP64, for t <
-// count; at most kFields of them.  dst: device or pinned host memory.
+// count; at most kFields of them.  dst: pinned host memory.
 constexpr int kFields = 24;
 hipError_t launch_fields_gather(const FieldGeom &g, const std::vector<FieldOut> &out, size_t t0, size_t count,
                                 double *dst, hipStream_t s);

@@ -116,11 +116,10 @@ int gpl_upload(gpl_ctx *ctx, const double *vc, const double *const *vs, int layo
 /* Device -> host copy of Vc, Vs (MHD) and (if uc != NULL) the conserved Uc;
  * a NULL vc or vs is skipped.  ARY4D: Vs[d] carries the upper boundary face
  * (index n along d): the periodic image of face 0, else its own value.
- * ACTIVE: the state goes through pinned host memory, one above 1 MiB of mixed
- * precision or with ghost layers through device memory too: up to 1 MiB of it
- * from gpl_create on, up to 64 MiB of each above that from the first such call
- * on, freed by gpl_destroy; where they cannot be had the call copies without
- * them, more slowly.  Above 4 MiB up to seven
+ * ACTIVE: the state goes through pinned host memory, up to 1 MiB of it from
+ * gpl_create on, for a larger state up to 64 MiB from the first such call on,
+ * freed by gpl_destroy; where it cannot be had the call copies without it, more
+ * slowly.  No device memory is taken.  Above 4 MiB up to seven
  * helper threads, no more than the calling thread's spare cores, move the data
  * to the caller's arrays; they end with the call. */
 int gpl_download(gpl_ctx *ctx, double *vc, double *const *vs, double *uc, int layout);

@@ -266,3 +266,15 @@ def test_small_downloads_copy_nothing_field_by_field(he, n, physics, precision, 
     d.download()
     assert he.he_copies() == 0 and he.he_held(1) == pinned
     d.close()
+
+
+@pytest.mark.parametrize("precision,sides", [("mixed", ()), ("fp64", WALLS), ("fp64", ())])
+def test_downloads_take_no_device_memory(he, precision, sides):
+    """Not even where the state has to be gathered; the context's count of its
+    device bytes stays what it holds."""
+    d = _domain((41, 43, 47), precision=precision, sides=sides)
+    _fill(d)
+    held, counted = he.he_held(0), d.device_bytes()
+    d.download()
+    assert he.he_held(0) == held and d.device_bytes() == counted
+    d.close()
