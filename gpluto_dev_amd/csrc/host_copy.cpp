@@ -54,6 +54,9 @@ public:
     {
       std::lock_guard<std::mutex> l(m);
       to = (char *)dst; from = (const char *)src; size = bytes;
+      // enough pieces for every thread, of 256 KiB at least: a chunk of 1 MiB in one
+      // piece left the helpers idle (HD 511x333 278 -> 335 us a download, 270 in four)
+      piece = std::min(std::max(bytes/16, kPiece/4), kPiece);
       next.store(0);
       busy = (int)helpers.size();
       round++;
@@ -70,9 +73,9 @@ private:
   void work()
   {
     for (;;) {
-      const size_t o = next.fetch_add(kPiece);
+      const size_t o = next.fetch_add(piece);
       if (o >= size) return;
-      memcpy(to + o, from + o, size - o < kPiece ? size - o : kPiece);
+      memcpy(to + o, from + o, size - o < piece ? size - o : piece);
     }
   }
   void serve()
@@ -95,7 +98,7 @@ private:
   std::atomic<size_t> next{0};
   char *to = nullptr;
   const char *from = nullptr;
-  size_t size = 0;
+  size_t size = 0, piece = kPiece;
   unsigned long round = 0;
   int busy = 0;
   bool quit = false;
