@@ -110,15 +110,32 @@ inline int march_length(bool fp64, long long across, int n, long long waves16)
 // march -> columns: MHD HLLD 16^3 62 -> 55, 64^3 152 -> 138, 128x64^2 266 -> 242,
 // 128^2x64 (ratio 0.91, refused) 500 -> 516; RMHD HLL 64^3 245 -> 199, HLLD 64^3
 // 504 -> 376, HLLD van Leer RK3 50x44x38 455 -> 314.
-inline int sweep_columns(int nx, int na, int n, int march)
+//
+// That holds while the rows of 4 to 8 cells are still cached when the next column
+// block reads the rest of their lines: across z, whose rows lie a plane apart, less
+// far than across y, and for RMHD's dearer solves further.  Above `full` cells a
+// fifth is added, above `most` the columns are refused.  Sweep, us, columns / march:
+// MHD z 192^2x20 (0.74 M cells) 55 / 52, 160^2x32 (0.82 M) 60 / 66, 192^2x28 (1.03 M)
+// 84 / 74, 256^2x24 (1.6 M) 116 / 98, 400x300x20 (2.4 M) 206 / 139; MHD y 500x24x100 (1.2 M)
+// 66 / 73, 256x24x256 (1.6 M) 93 / 82, 384x16x384 (2.4 M) 159 / 123; RMHD HLL z 192^2x32
+// (1.2 M) 125 / 135, 256^2x24 167 / 158, y 384x16x384 199 / 214.
+struct ColumnLimit { long long full, most; };
+inline ColumnLimit column_limit(bool rmhd, bool z)
+{
+  if (rmhd) return z ? ColumnLimit{1300000, 1300000} : ColumnLimit{1LL << 40, 1LL << 40};
+  return z ? ColumnLimit{650000, 850000} : ColumnLimit{1000000, 1300000};
+}
+inline int sweep_columns(int nx, int na, int n, int march, const ColumnLimit &lim)
 {
   constexpr int kCUs = 256, kBlock = 256;
-  const long long mb = ((long long)nx*na*((n + march - 1)/march) + kBlock - 1)/kBlock;
+  const long long cells = (long long)nx*na*n, mb = ((long long)nx*na*((n + march - 1)/march) + kBlock - 1)/kBlock;
+  if (cells > lim.most) return 0;
+  const double far = cells > lim.full ? 1.2 : 1.0;
   double best = 0.9*(double)((mb + kCUs - 1)/kCUs)*(kBlock/64)*(march + 1.5);
   int x = 0;
   for (int c = 4; c <= 8 && c*n <= kBlock; c++) {
     const long long blocks = (long long)((nx + c - 1)/c)*na;
-    const double t = (double)((blocks + kCUs - 1)/kCUs)*((c*n + 63)/64);
+    const double t = far*(double)((blocks + kCUs - 1)/kCUs)*((c*n + 63)/64);
     if (t < best) { best = t; x = c; }
   }
   return x;

@@ -204,8 +204,8 @@ public:
     }
     rows = sweep_rows(g.nx, (long long)g.ny*g.nz);
     if (fp64 && fused && !fused_xy && !pipelined && !getenv("GPL_MARCH")) {
-      cols[0] = sweep_columns(g.nx, g.nz, g.ny, march[0]);
-      cols[1] = sweep_columns(g.nx, g.ny, g.nz, march[1]);
+      cols[0] = sweep_columns(g.nx, g.nz, g.ny, march[0], column_limit(rmhd, false));
+      cols[1] = sweep_columns(g.nx, g.ny, g.nz, march[1], column_limit(rmhd, true));
     }
     nparts = !fused ? mhd3d_blocks(g) : cols[1] ? (g.nx + cols[1] - 1)/cols[1]*g.ny
                                                 : mhd3d_march_blocks(g, march[1]);

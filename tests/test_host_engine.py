@@ -161,9 +161,9 @@ def test_hd_arrival_counters_have_their_own_lines(he, n):
 K_MHD_SWEEP_X, K_MHD_XY = 4, 13                      # common.hpp's kernel ids
 
 
-def _mhd_shape(he, n, precision="fp64", sides=(), **kw):
+def _mhd_shape(he, n, precision="fp64", sides=(), physics="MHD", **kw):
     """(march y, march z, rows, columns y, columns z, EMF march) of a box's launches."""
-    d = _domain(n, precision=precision, sides=sides, **kw)
+    d = _domain(n, physics, precision, sides, **kw)
     _launches(he)
     d.advance_step(1e-4)
     got = {tuple(v[:6]) for k, v in _launches(he) if k <= K_MHD_XY and k != K_DT}
@@ -278,3 +278,13 @@ def test_downloads_take_no_device_memory(he, precision, sides):
     d.download()
     assert he.he_held(0) == held and d.device_bytes() == counted
     d.close()
+
+
+@pytest.mark.parametrize("n,physics,y,z", [
+    ((256, 256, 24), "MHD", 0, 0), ((400, 300, 20), "MHD", 0, 0), ((192, 192, 28), "MHD", 0, 0),
+    ((256, 24, 256), "MHD", 0, 0), ((500, 24, 100), "MHD", 8, 0), ((160, 160, 32), "MHD", 0, 4),
+    ((256, 256, 24), "RMHD", 0, 0), ((192, 192, 32), "RMHD", 0, 4), ((500, 24, 150), "RMHD", 8, 0),
+    ((64, 64, 64), "MHD", 4, 4), ((64, 64, 64), "RMHD", 4, 4)])
+def test_large_flat_boxes_march(he, n, physics, y, z):
+    """Whole columns lose to the marches on flat boxes that the caches do not hold."""
+    assert _mhd_shape(he, n, physics=physics)[3:5] == (y, z)
