@@ -53,12 +53,16 @@ int from_device_v(void *src, bool fp64, std::vector<double> &dst)
 //   FP64 VL  96^3 52 / 57 / 69 / 116   128^3 123 / 101 / 98 / 134   192^3 370 / 316 / 306 / 323
 //   FP32 MC  96^3 25 / 29 / 33 / 80    128^3 63 / 55 / 53 / 102     192^3 196 / 158 / 158 / 167
 // so the edge kernel up to a million cells, tiles of 8 planes above, and tiles
-// of 32 (fewest bytes) once they alone are 2048, eight per CU.
+// of 32 (fewest bytes) once they alone are 2048, eight per CU, or where one march
+// through a flat box of at most 24 planes leaves 600 of them: three starts cost
+// more there than idle CUs (8 / 32: 640x300x20 156 / 136, FP32 108 / 90, 256x1024x12
+// 135 / 117, 320x512x20 142 / 135; but 400x300x20, 525 tiles, 110 / 114, and 512x320x32
+// 190 / 210).
 int emf_choice(const Box3 &g)
 {
   if (g.ncell <= 1000000) return 0;
   const long long across = (long long)((g.nx + 63)/64)*((g.ny + 3)/4);
-  return across*((g.nz + 31)/32) >= 2048 ? -32 : -8;
+  return across*((g.nz + 31)/32) >= 2048 || (g.nz <= 24 && across >= 600) ? -32 : -8;
 }
 
 class Mhd3dEngine : public Engine {

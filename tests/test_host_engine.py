@@ -288,3 +288,12 @@ def test_downloads_take_no_device_memory(he, precision, sides):
 def test_large_flat_boxes_march(he, n, physics, y, z):
     """Whole columns lose to the marches on flat boxes that the caches do not hold."""
     assert _mhd_shape(he, n, physics=physics)[3:5] == (y, z)
+
+
+@pytest.mark.parametrize("n,precision,emf", [
+    ((640, 300, 20), "fp64", -32), ((256, 1024, 12), "fp64", -32), ((640, 300, 20), "mixed", -32),
+    ((256, 256, 24), "fp64", -8), ((400, 300, 20), "fp64", -8), ((512, 320, 32), "fp64", -8),
+    ((1024, 64, 64), "fp64", -8), ((128, 128, 128), "fp64", -8), ((192, 192, 192), "fp64", -8), ((224, 224, 224), "fp64", -8), ((256, 256, 256), "fp64", -32),
+    ((320, 320, 320), "fp64", -32), ((100, 100, 100), "fp64", 0)])
+def test_emf_tiles_by_size(he, n, precision, emf):
+    assert _mhd_shape(he, n, precision)[5] == emf
