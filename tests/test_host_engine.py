@@ -309,3 +309,21 @@ def test_large_flat_boxes_march(he, n, physics, y, z):
     ((320, 320, 320), "fp64", -32), ((100, 100, 100), "fp64", 0)])
 def test_emf_tiles_by_size(he, n, precision, emf):
     assert _mhd_shape(he, n, precision)[5] == emf
+
+
+def test_a_context_without_pinned_memory(he):
+    """Neither its creation nor its downloads need any."""
+    d = _domain((16, 15, 14), precision="mixed", sides=WALLS)
+    _fill(d)
+    want = d.download()
+    d.close()
+    he.he_limits(UNLIMITED, 0)
+    try:
+        d = _domain((16, 15, 14), precision="mixed", sides=WALLS)
+        _fill(d)
+        got = d.download()
+    finally:
+        he.he_limits(UNLIMITED, UNLIMITED)
+    assert he.he_held(1) == 0 and he.he_last_error() == 0
+    d.close()
+    assert all(np.array_equal(a, b) for a, b in zip(got, want))
