@@ -156,13 +156,8 @@ void HostCopy::prepare(size_t total)
 int HostCopy::fetch_small(const FieldGeom &g, const std::vector<FieldOut> &out, hipStream_t s)
 {
   const size_t n = (size_t)g.n[0]*g.n[1]*g.n[2], nf = out.size();
-  bool one = g.whole;                          // stored as they leave: a copy, 4 us less than the kernel
-  for (size_t q = 0; q < nf; q++)
-    one = one && !out[q].f32 && (const double *)out[q].src == (const double *)out[0].src + q*n;
-  const hipError_t e = one ? hipMemcpyAsync(pin, (const double *)out[0].src + g.off, nf*n*sizeof(double),
-                                            hipMemcpyDeviceToHost, s)
-                           : launch_fields_gather(g, out, 0, nf*n, pin, s);
-  if (e != hipSuccess || hipStreamSynchronize(s) != hipSuccess) return GPL_EHIP;
+  if (launch_fields_gather(g, out, 0, nf*n, pin, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
+    return GPL_EHIP;
   for (size_t q = 0; q < nf;) {
     size_t run = 1;                            // arrays that follow one another at the caller's
     while (q + run < nf && out[q + run].dst == out[q].dst + run*n) run++;

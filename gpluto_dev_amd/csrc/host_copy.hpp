@@ -2,11 +2,12 @@
 //
 // A field is one variable over the active zones, i fastest.
 //  * Up to 1 MiB (kSmall) one kernel writes every field into a pinned buffer, made
-//    with the context (one copy does where the fields lie there as they leave: Vc of
-//    HD); one wait, then the caller's arrays.  Copies of the fields
+//    with the context; one wait, then the caller's arrays.  Copies of the fields
 //    by themselves cost 5 to 20 us each, and some runs of them 60 to 100: us a
 //    download, 1D 100 zones 40 -> 15, 4096 zones 150 -> 27, 10^3 MHD 65 -> 21, 16^3 300
-//    -> 41, 18x17x16 77 -> 46, 60^2 mixed with ghosts 97 -> 38.
+//    -> 41, 18x17x16 77 -> 46, 60^2 mixed with ghosts 97 -> 38.  Vc of HD, stored as it
+//    leaves, takes the launch too: one copy of 1052 zones is 11 us or, after another
+//    context's large transfers, 45; the launch 15 both times (4096 zones 16 and 20).
 //  * Above, the fields are cut into chunks of an eighth of the state, 1 to 16 MiB; a
 //    chunk is copied into one of kSlots pinned buffers (where the stored array is FP32
 //    or holds ghost layers, written there by the gather kernel), and while later chunks

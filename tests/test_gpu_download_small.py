@@ -23,7 +23,7 @@ def test_small_states(n, physics, precision, sides):
 
 @pytest.mark.parametrize("n", [(3, 1, 1), (61, 17, 1), (20, 20, 20)])
 def test_vc_of_a_small_hd_state(n):
-    """Vc by itself, one copy, against Vc beside Uc, gathered."""
+    """Vc by itself, one array on the device, against Vc beside Uc."""
     dims = 1 if n[1] == 1 else 2 if n[2] == 1 else 3
     g = StageUpdate(Definitions(physics="HD", dimensions=dims), RuntimeSetup(n=n, solver="hllc"))
     g.upload(ic.hd_blast(n, 3))

@@ -268,15 +268,16 @@ def test_small_downloads_copy_nothing_field_by_field(he, n, physics, precision, 
     d.close()
 
 
-def test_a_small_array_comes_in_one_copy(he):
-    """Vc of a small HD state lies on the device as it leaves."""
+def test_a_small_array_takes_no_copy(he):
+    """Vc of a small HD state lies on the device as it leaves; the copy engine's
+    latency depends on the transfers before, so the gather launch takes it too."""
     d = _domain((33, 20, 1), "HD")
     _fill(d)
     want = d.download()[0]
     vc = np.zeros((5, 1, 20, 33))
     he.he_copies()
     _lib.check(d._L.gpl_download(d._h, vc.ctypes.data, None, None, _lib.GPL_LAYOUT_ACTIVE), "gpl_download")
-    assert he.he_copies() == 1 and np.array_equal(vc, want)
+    assert he.he_copies() == 0 and np.array_equal(vc, want)
     d.close()
 
 
